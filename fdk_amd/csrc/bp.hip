@@ -37,6 +37,7 @@
 #include <cmath>
 #include <cstdlib>
 #include <cstring>
+#include <type_traits>
 #include <vector>
 
 #include "common.hpp"
@@ -739,40 +740,66 @@ __global__ __launch_bounds__(256) void bp_lds_pf_kernel(BpArgs a, BpMats M, BpSc
 }
 
 // ------------------------------------------------------------ wave-strip kernel
-// bp_wave_kernel: the same blocks, columns and lanes, for a mirror slab pair
-// whose matrices are mirror-symmetric (v(z) + v(nz-1-z) = W-1 for every
-// column, checked on the host), with no block-level synchronisation:
-//  * each wave stages, per view, ITS OWN u-interpolated detector strips in LDS:
+// bp_wave_kernel: the same blocks, columns and lanes, with no block-level
+// synchronisation in the view loop:
+//  * each wave stages, per view, ITS OWN u-interpolated detector strip in LDS:
 //    r(c) = w0 P[iu][c] + w1 P[iu+1][c] (w0, w1 the u weights times 1/w^2) over
-//    the v columns of its top z-run, and the same for the mirror run, which by
-//    symmetry reads columns W-1-c, stored reversed; top and mirror samples are
-//    interleaved, so one 16-byte LDS read brings r_top(iv), r_mir(iv),
-//    r_top(iv+1), r_mir(iv+1);
-//  * the mirror voxel has v' = W-1-v, so iv' = W-2-iv and t' = 1-t: its
-//    sample is r_mir(iv) + t (r_mir(iv+1) - r_mir(iv)) with the top voxel's iv
-//    and t, and the same validity (0 <= iv <= W-2);
+//    the v columns of its z-run, so a voxel's sample is one v interpolation;
+//  * SYM, a mirror slab pair whose matrices are mirror-symmetric (v(z) +
+//    v(nz-1-z) = W-1 for every column, checked on the host): the mirror run reads
+//    columns W-1-c, stored reversed and interleaved with the top run's, so one
+//    16-byte LDS read brings r_top(iv), r_mir(iv), r_top(iv+1), r_mir(iv+1).  The
+//    mirror voxel has v' = W-1-v, so iv' = W-2-iv and t' = 1-t: it shares the top
+//    voxel's floor, fraction and validity (0 <= iv <= W-2).  Otherwise each slab
+//    is one run of its own, with one strip;
 //  * the per-(column, view) values (u weights, v = Vb + z dV, strip bounds and
 //    flags) are computed once, lane s for view s, and broadcast with readlane;
 //  * the next view's strip loads are issued into registers before the current
-//    view is computed from LDS.
-// Per voxel pair: v, floor, fraction, 1-t, the LDS address (and the validity
-// test where the run crosses the detector edge) and four FMAs.
-constexpr int kWsQuads = 3;  // strip quads per lane and run (the host checks CT against it)
-// Quad slots a lane stages at a given ZPT: a 256-voxel run's strip fits 2 x 64
-// quads, and an always-empty third slot would still cost its (range-checked,
-// zero) loads and offsets every view.
+//    view is computed from LDS.  Each strip row has its own buffer resource, based
+//    at the strip's first column and exactly as long as the strip, so a lane's
+//    offsets never change (one subtraction for the mirror run), lanes past the
+//    strip read nothing, and no address is formed on the vector unit;
+//  * VS = 4 splits the views over the block's four waves, which then share one
+//    column and add their sums in LDS: for grids too small to fill the chip, where
+//    the loop over views is a chain of load latencies.
+// Per voxel pair (voxel): v, floor, fraction, 1-t, the LDS address (and the
+// validity test where the run crosses the detector edge) and four (two) FMAs.
+//
+// ZPT (a run is 64 ZPT voxels) is chosen on the host from the slab depth.
+//
+// What bounds it: vector issue (about 75 of 138 instructions a view are the taps at
+// ZPT 8) together with the L1 return path (64 bytes a clock: a strip is 4 rows of
+// 16-byte loads) and the strip's round trip through LDS.  Measured against the form
+// that formed 64-bit addresses per slot, kept three tap forms in one loop (16 to 32
+// register moves a view where they joined) and ran single slabs on the block-strip
+// kernels: 1024^3 pair, 64 FP16 views of 1024^2, with read-out 27.8 -> 22.3 ms;
+// 768 x 512 x 2048 pair, 32 FP32 views 12.5 -> 10.6 ms; 256^3 pair, 96 FP32 views
+// 1458 -> 784 us (the 128-deep slabs at ZPT 2 instead of half-empty ZPT 4 runs);
+// 256^3 box of a 1024^3 scan, 128 FP32 views 2096 -> 880 us; 101 x 92 x 83 volume,
+// detector 121 x 98, 2 x 40 views with the projector 632 -> 481 us (was the
+// direct-gather kernel: rows no multiple of 4).
+constexpr int kWsQuads = 3;  // strip quads per lane and run at ZPT 8
+// Quad slots a lane stages: a 64 ZPT-voxel run's strip of the usual 1.3 columns
+// a voxel fits 64 slots of 4 columns each up to ZPT 2, 128 at ZPT 4 and 192 at 8;
+// a slot that is always empty would still issue its loads every view.
 template <int ZPT>
-constexpr int ws_quads() { return ZPT == 4 ? 2 : kWsQuads; }
+constexpr int ws_quads() { return ZPT <= 2 ? 1 : ZPT == 4 ? 2 : kWsQuads; }
 
 // Per-view values of one column, kept in lane s for view s.
 struct WaveView {
-  float Vb, dV, w0, w1, Z2;
+  float Vb, dV, Z2;
+  float w0, w1;  // 16-bit views: times the view's scale
+  float zof;     // 16-bit views: (w0 + w1) * offset, before the scaling
   int iu;
   int c0;     // first strip column (multiple of 4)
   int quads;  // strip quads of 4 columns
-  int flags;  // 1: some voxel of the runs inside the view, 2: all inside, 4: the strip fits
+  int off;    // byte offset of (iu, c0) in the view (a view is under 2 GiB)
 };
 
+typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
+
+// w0 * a + w1 * b per column; 16-bit samples take w0, w1 times the view's scale
+// and zof = (w0 + w1) * offset.
 template <int DT>
 __device__ __forceinline__ float4 ws_combine(typename Quad<DT>::raw A, typename Quad<DT>::raw B,
                                              float w0, float w1, float zof) {
@@ -780,99 +807,138 @@ __device__ __forceinline__ float4 ws_combine(typename Quad<DT>::raw A, typename 
     return make_float4(fmaf(w1, B.x, w0 * A.x), fmaf(w1, B.y, w0 * A.y), fmaf(w1, B.z, w0 * A.z),
                        fmaf(w1, B.w, w0 * A.w));
   } else {
-    // w0, w1 already carry the view's scale; zof = (w0 + w1) * offset
-    const float4 qa = Quad<DT>::cvt(A, 1.0f, 0.0f), qb = Quad<DT>::cvt(B, 1.0f, 0.0f);
-    return make_float4(fmaf(w1, qb.x, fmaf(w0, qa.x, zof)), fmaf(w1, qb.y, fmaf(w0, qa.y, zof)),
-                       fmaf(w1, qb.z, fmaf(w0, qa.z, zof)), fmaf(w1, qb.w, fmaf(w0, qa.w, zof)));
+    float f[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const unsigned wa = A[e >> 1], wb = B[e >> 1];
+      float qa, qb;
+      if constexpr (DT == FDK_F16) {  // converted inside the mixed-precision FMA
+        qa = (float)__builtin_bit_cast(half2_t, wa)[e & 1];
+        qb = (float)__builtin_bit_cast(half2_t, wb)[e & 1];
+      } else {
+        qa = __uint_as_float((e & 1) ? wa & 0xffff0000u : wa << 16);
+        qb = __uint_as_float((e & 1) ? wb & 0xffff0000u : wb << 16);
+      }
+      f[e] = fmaf(qb, w1, fmaf(qa, w0, zof));
+    }
+    return make_float4(f[0], f[1], f[2], f[3]);
   }
 }
 
-template <int DT>
+template <int DT, bool SYM, int NQ>
 struct WsPre {
-  typename Quad<DT>::raw ta[kWsQuads], tb[kWsQuads], ma[kWsQuads], mb[kWsQuads];  // NQ <= kWsQuads used
+  typename Quad<DT>::raw ta[NQ], tb[NQ], ma[SYM ? NQ : 1], mb[SYM ? NQ : 1];
 };
 
 // Strip loads of one view: quad q of the top run reads columns c0+4q..c0+4q+3
-// of rows iu and iu+1; of the mirror run, columns W-4-c0-4q..W-1-c0-4q.
-// Columns outside the row read other samples of the view or (negative or past
-// the view) zero through the buffer range check; only columns of valid taps
-// are ever used.
-// FP32: branch-free, every offset computed before the first load and quads past
-// the strip given an offset past the view (zeros, never used), so the loads of
-// one view issue back to back and no register reuse has to wait on them.
-// 16-bit views (8-byte loads, half the registers in flight) keep a branch per
-// quad slot, which measured faster for them (2577 against 2463 GUPS in FP16).
-template <int DT, int NQ = kWsQuads>
-__device__ __forceinline__ void ws_issue(WsPre<DT>& pre, __amdgpu_buffer_rsrc_t rv, int W, int iu,
-                                         int c0, int quads, int lane) {
-  const int es = DT == FDK_F32 ? 4 : 2;
-  const int rowa = iu * W * es, rowb = rowa + W * es;
-  if constexpr (DT != FDK_F32) {
+// of rows iu and iu+1; of the mirror run, columns W-4-c0-4q..W-1-c0-4q.  A quad
+// that reaches past its row's end reads on into the next row (or, mirrored, back
+// into the one before); the kernel keeps such quads inside the view, and only
+// columns of valid taps are ever used.
+template <int DT, bool SYM, int NQ>
+__device__ __forceinline__ void ws_issue(WsPre<DT, SYM, NQ>& pre, const BpArgs& a, int s,
+                                         const WaveView& wv, int quads, int lane) {
+  constexpr int es = DT == FDK_F32 ? 4 : 2, qb = 4 * es;
+  const int off = __builtin_amdgcn_readlane(wv.off, s), len = quads * qb;
+  const char* view = static_cast<const char*>(a.proj) + (size_t)s * a.view_bytes;
+  const char* top = view + (unsigned)off;
+  // the mirror run's offsets, pinned before the first load: an offset formed
+  // between the loads lands in a register of a load in flight and waits for it
+  int om[SYM ? NQ : 1];
+  if constexpr (SYM) {
 #pragma unroll
     for (int k = 0; k < NQ; ++k) {
-      const int q = lane + kWave * k;
-      if (q < quads) {
-        const int ct = (c0 + 4 * q) * es, cm = (W - 4 - c0 - 4 * q) * es;
-        pre.ta[k] = Quad<DT>::load(rv, rowa + ct);
-        pre.tb[k] = Quad<DT>::load(rv, rowb + ct);
-        pre.ma[k] = Quad<DT>::load(rv, rowa + cm);
-        pre.mb[k] = Quad<DT>::load(rv, rowb + cm);
+      om[k] = len - qb - (lane + kWave * k) * qb;  // negative past the strip: out of range
+      asm volatile("" : "+v"(om[k]));
+    }
+  }
+  const __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc((void*)top, 0, len, fdk::kRawRsrcWord3);
+  const __amdgpu_buffer_rsrc_t rb =
+      __builtin_amdgcn_make_buffer_rsrc((void*)(top + a.row_bytes), 0, len, fdk::kRawRsrcWord3);
+#pragma unroll
+  for (int k = 0; k < NQ; ++k) {
+    if (k == 0 || lane + kWave * k < quads) {
+      pre.ta[k] = Quad<DT>::load(ra, (lane + kWave * k) * qb);
+      pre.tb[k] = Quad<DT>::load(rb, (lane + kWave * k) * qb);
+    }
+  }
+  if constexpr (SYM) {
+    const int c0 = __builtin_amdgcn_readlane(wv.c0, s);
+    const char* mir = view + (unsigned)(off + (a.W - 2 * c0) * es - len);
+    const __amdgpu_buffer_rsrc_t rma = __builtin_amdgcn_make_buffer_rsrc((void*)mir, 0, len, fdk::kRawRsrcWord3);
+    const __amdgpu_buffer_rsrc_t rmb =
+        __builtin_amdgcn_make_buffer_rsrc((void*)(mir + a.row_bytes), 0, len, fdk::kRawRsrcWord3);
+#pragma unroll
+    for (int k = 0; k < NQ; ++k) {
+      if (k == 0 || lane + kWave * k < quads) {
+        pre.ma[k] = Quad<DT>::load(rma, om[k]);
+        pre.mb[k] = Quad<DT>::load(rmb, om[k]);
       }
     }
-    return;
-  }
-  constexpr int kOut = (int)0xFFFFFFF0u;  // past any view's buffer range
-  int ta[NQ], tb[NQ], ma[NQ], mb[NQ];
-#pragma unroll
-  for (int k = 0; k < NQ; ++k) {
-    const int q = lane + kWave * k;
-    const bool ok = q < quads;
-    const int ct = (c0 + 4 * q) * es, cm = (W - 4 - c0 - 4 * q) * es;
-    ta[k] = ok ? rowa + ct : kOut;
-    tb[k] = ok ? rowb + ct : kOut;
-    ma[k] = ok ? rowa + cm : kOut;
-    mb[k] = ok ? rowb + cm : kOut;
-  }
-#pragma unroll
-  for (int k = 0; k < NQ; ++k) {
-    pre.ta[k] = Quad<DT>::load(rv, ta[k]);
-    pre.tb[k] = Quad<DT>::load(rv, tb[k]);
-    pre.ma[k] = Quad<DT>::load(rv, ma[k]);
-    pre.mb[k] = Quad<DT>::load(rv, mb[k]);
   }
 }
 
-template <int DT, int NQ = kWsQuads>
-__device__ __forceinline__ void ws_commit(const WsPre<DT>& pre, float2* strip, float w0, float w1,
-                                          float zof, int quads, int lane) {
+// Interpolates the loaded rows in u and stores the strip (float2 per column
+// {top, mirror} with SYM, else float).
+template <int DT, bool SYM, int NQ>
+__device__ __forceinline__ void ws_commit(const WsPre<DT, SYM, NQ>& pre, float* strip, float w0,
+                                          float w1, float zof, int quads, int lane) {
 #pragma unroll
   for (int k = 0; k < NQ; ++k) {
     const int q = lane + kWave * k;
     if (q < quads) {
       const float4 t = ws_combine<DT>(pre.ta[k], pre.tb[k], w0, w1, zof);
-      const float4 m = ws_combine<DT>(pre.ma[k], pre.mb[k], w0, w1, zof);
-      float4* d = reinterpret_cast<float4*>(strip + 4 * q);
-      d[0] = make_float4(t.x, m.w, t.y, m.z);  // mirror quad reversed
-      d[1] = make_float4(t.z, m.y, t.w, m.x);
+      if constexpr (SYM) {
+        const float4 m = ws_combine<DT>(pre.ma[k], pre.mb[k], w0, w1, zof);
+        float4* d = reinterpret_cast<float4*>(strip + 8 * q);
+        d[0] = make_float4(t.x, m.w, t.y, m.z);  // mirror quad reversed
+        d[1] = make_float4(t.z, m.y, t.w, m.x);
+      } else {
+        *reinterpret_cast<float4*>(strip + 4 * q) = t;
+      }
     }
   }
 }
 
-template <bool CHECK, int ZPT>
+// The taps of one view from the strip, in groups of G voxels: a group's LDS reads
+// are issued before the previous group's are used, so their latency overlaps.
+// Groups of 4 would need more than the 128 registers of 4 waves per SIMD at ZPT 8.
+template <bool CHECK, bool SYM, int ZPT>
 __device__ __forceinline__ void ws_compute(float (&acc)[ZPT], float (&accm)[ZPT],
                                            const float (&zt)[ZPT], float Vb, float dV,
-                                           const float2* base, const float2* zslot, int W) {
+                                           const float* strip, int c0, int zslot, int W) {
+  typedef typename std::conditional<SYM, float2, float>::type T;
+  constexpr int G = 1;
+  const T* base = reinterpret_cast<const T*>(strip) - c0;
+  const T* zero = reinterpret_cast<const T*>(strip) + zslot;
+  float t[ZPT];
+  T a[ZPT], b[ZPT];
+  auto read = [&](int g) {
 #pragma unroll
-  for (int j = 0; j < ZPT; ++j) {
-    const float v = fmaf(zt[j], dV, Vb);
-    const int iv = floor_int(v);
-    const float t = __builtin_amdgcn_fractf(v);
-    const float2* p = base + iv;
-    if (CHECK) p = (unsigned)iv <= (unsigned)(W - 2) ? p : zslot;
-    const float2 a = p[0], b = p[1];
-    const float omt = 1.0f - t;
-    acc[j] = fmaf(t, b.x, fmaf(omt, a.x, acc[j]));
-    accm[j] = fmaf(t, b.y, fmaf(omt, a.y, accm[j]));
+    for (int j = g; j < g + G; ++j) {
+      const float v = fmaf(zt[j], dV, Vb);
+      const int iv = floor_int(v);
+      t[j] = __builtin_amdgcn_fractf(v);
+      const T* p = base + iv;
+      if (CHECK) p = (unsigned)iv <= (unsigned)(W - 2) ? p : zero;
+      a[j] = p[0];
+      b[j] = p[1];
+    }
+  };
+  read(0);
+#pragma unroll
+  for (int g = 0; g < ZPT; g += G) {
+    if (g + G < ZPT) read(g + G);
+#pragma unroll
+    for (int j = g; j < g + G; ++j) {
+      const float omt = 1.0f - t[j];
+      if constexpr (SYM) {
+        acc[j] = fmaf(t[j], b[j].x, fmaf(omt, a[j].x, acc[j]));
+        accm[j] = fmaf(t[j], b[j].y, fmaf(omt, a[j].y, accm[j]));
+      } else {
+        acc[j] = fmaf(t[j], b[j], fmaf(omt, a[j], acc[j]));
+      }
+    }
   }
 }
 
@@ -881,23 +947,75 @@ __device__ __forceinline__ float lane_f(float v, int s) {
 }
 __device__ __forceinline__ int lane_i(int v, int s) { return __builtin_amdgcn_readlane(v, s); }
 
-template <int DT, int ZPT>
-__global__ __launch_bounds__(256) void bp_wave_kernel(BpArgs a, BpMats M, BpScale S, int CT) {
-  extern __shared__ float2 wstrip[];  // per wave: CT float2, the last two the zero slot
-  const unsigned lb = xcd_remap(blockIdx.x, gridDim.x);
+// One view of the loop: commit its strip, issue the next view's loads (nxt < 0:
+// none), add its taps.
+template <bool CHECK, int DT, bool SYM, int ZPT, int NQ>
+__device__ __forceinline__ void ws_view(float (&acc)[ZPT], float (&accm)[ZPT],
+                                        const float (&zt)[ZPT], WsPre<DT, SYM, NQ>& pre, int& quads,
+                                        const BpArgs& a, const WaveView& wv, int s, int nxt,
+                                        float* strip, int zslot, int lane) {
+  ws_commit<DT, SYM, NQ>(pre, strip, lane_f(wv.w0, s), lane_f(wv.w1, s),
+                         DT != FDK_F32 ? lane_f(wv.zof, s) : 0.f, quads, lane);
+  if (nxt >= 0) {
+    quads = lane_i(wv.quads, nxt);
+    ws_issue<DT, SYM, NQ>(pre, a, nxt, wv, quads, lane);
+  }
+  ws_compute<CHECK, SYM, ZPT>(acc, accm, zt, lane_f(wv.Vb, s), lane_f(wv.dV, s), strip,
+                              lane_i(wv.c0, s), zslot, a.W);
+}
+
+// Waves per SIMD the register allocator aims at, where its own choice is one short.
+template <int DT, bool SYM, int ZPT>
+constexpr int ws_waves() { return SYM && ZPT == 8 ? (DT == FDK_F32 ? 4 : 5) : SYM && ZPT == 4 && DT == FDK_F32 ? 6 : 1; }
+
+// floor(2^32 / d) of the divisors of bp_wave_kernel's block numbering: a
+// division costs 20 vector instructions, the multiplication a few scalar ones.
+struct WsGrid {
+  unsigned band, tile, cols;
+};
+__host__ __device__ inline unsigned udiv_inv(unsigned d) {
+  return d > 1 ? (unsigned)((1ull << 32) / d) : 0xffffffffu;
+}
+// n / d with inv = udiv_inv(d): the estimate is the quotient or one less.
+__host__ __device__ inline unsigned udiv_magic(unsigned n, unsigned d, unsigned inv) {
+  const unsigned q = (unsigned)(((unsigned long long)n * inv) >> 32);
+  return n - q * d >= d ? q + 1 : q;
+}
+
+template <int DT, bool SYM, int ZPT, int VS>
+__global__ __launch_bounds__(256, (ws_waves<DT, SYM, ZPT>())) void bp_wave_kernel(
+    BpArgs a, BpMats M, BpScale S, WsGrid G, int CT) {
+  constexpr int NQ = ws_quads<ZPT>(), kSides = SYM ? 2 : 1;
+  // per wave: CT columns of kSides floats, the last two the zero slot; then, with
+  // VS > 1, every wave's sums
+  extern __shared__ float wstrip[];
+  // Patches of 2x2 columns in kTile x kTile tiles, those at the right and lower edges
+  // cut to the grid: runs of blocks stay in compact regions, and none is padding
+  // (in whole tiles a grid of 101 x 92 columns would be a quarter padding, unevenly
+  // over the XCDs).
+  const int npx = (a.nxs + 1) / 2, npy = (a.nys + 1) / 2;
+  const int lb0 = (int)xcd_remap(blockIdx.x, gridDim.x);
+  const int lb = lb0 / VS;
+  if (lb >= npx * npy) return;  // the grid is rounded up to a multiple of 8
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
   const int lane = threadIdx.x % kWave;
-  const int tile = lb / (kTile * kTile);
-  const int within = lb % (kTile * kTile);
-  const int px = (tile % a.tiles_x) * kTile + within % kTile;
-  const int py = (tile / a.tiles_x) * kTile + within / kTile;
-  const int xs = 2 * px + (wave & 1);
-  const int ys = 2 * py + (wave >> 1);
-  if (xs >= a.nxs || ys >= a.nys) return;  // no block barrier: the wave just leaves
-  float2* strip = wstrip + wave * CT;
-  const float2* zslot = strip + CT - 2;
-  if (lane < 2) strip[CT - 2 + lane] = make_float2(0.f, 0.f);
+  const int band = (int)udiv_magic(lb, kTile * npx, G.band);
+  const int rows = min(kTile, npy - kTile * band);  // the last band's tiles may be lower
+  int in = lb - band * kTile * npx;
+  const int tile = rows == kTile ? in / (kTile * kTile) : (int)udiv_magic(in, kTile * rows, G.tile);
+  const int cols = min(kTile, npx - kTile * tile);  // a band's last tile may be narrower
+  in -= tile * kTile * rows;
+  const int row = cols == kTile ? in / kTile : (int)udiv_magic(in, cols, G.cols);
+  const int px = kTile * tile + in - row * cols, py = kTile * band + row;
+  const int colw = VS == 1 ? wave : lb0 % VS;  // the wave's column of the patch
+  const int xs = 2 * px + (colw & 1);
+  const int ys = 2 * py + (colw >> 1);
+  if (xs >= a.nxs || ys >= a.nys) return;  // VS == 1: no barrier follows; else the whole block leaves
+  float* strip = wstrip + wave * CT * kSides;
+  const int zslot = CT - 2;
+  if (lane < 2 * kSides) strip[(CT - 2) * kSides + lane] = 0.f;
   const int zb0 = blockIdx.y * (kWave * ZPT);
+  const int zend = min(zb0 + kWave * ZPT, a.zext) - 1;  // the run's last voxel
   const int zbase = zb0 + lane;
   const float x = (float)(a.x0 + xs);
   const float y = (float)(a.y0 + ys);
@@ -906,89 +1024,122 @@ __global__ __launch_bounds__(256) void bp_wave_kernel(BpArgs a, BpMats M, BpScal
   for (int j = 0; j < ZPT; ++j) {
     acc[j] = 0.f;
     accm[j] = 0.f;
-    zt[j] = (float)(a.z0 + zbase + j * kWave);
+    // lanes past the slab repeat its last voxel (and store nothing)
+    zt[j] = (float)(a.z0 + min(zbase + j * kWave, zend));
   }
 
   // lane s: the values of view s for this column
   WaveView wv{};
+  bool any = false, all = false, fits = false;  // inside the view: some of the run, all of it
   if (lane < a.nproj) {
     const float* m = M.m[lane];
     const float wd = fmaf(m[8], x, fmaf(m[9], y, m[11]));
     const float Z = 1.0f / wd;
-    const float U = fmaf(m[0], x, fmaf(m[1], y, m[3])) * Z;
+    const float un = fmaf(m[0], x, fmaf(m[1], y, m[3]));
+    const float U = un * Z;
     wv.Vb = fmaf(m[4], x, fmaf(m[5], y, m[7])) * Z;
     wv.dV = m[6] * Z;
     wv.Z2 = Z * Z;
     const float fu0 = floorf(U);
     wv.iu = (int)fu0;
     const bool uok = (unsigned)wv.iu <= (unsigned)(a.H - 2);
-    const float fu = U - fu0;
+    const float fu = fmaf(un, Z, -fu0);  // the fraction of the unrounded u
     wv.w0 = uok ? (1.0f - fu) * wv.Z2 : 0.0f;
     wv.w1 = uok ? fu * wv.Z2 : 0.0f;
-    // v over the top run, as the compute evaluates it (monotone in z)
-    const float va = fmaf((float)(a.z0 + zb0), wv.dV, wv.Vb);
-    const float vb = fmaf((float)(a.z0 + zb0 + kWave * ZPT - 1), wv.dV, wv.Vb);
-    const int ilo = floor_int(fminf(va, vb)), ihi = floor_int(fmaxf(va, vb));
-    const bool any = uok && ihi >= 0 && ilo <= a.W - 2;
-    const bool all = uok && ilo >= 0 && ihi <= a.W - 2;
-    wv.c0 = max(ilo, 0) & ~3;
-    const int c1 = min(ihi + 1, a.W - 1);
-    wv.quads = any ? (c1 - wv.c0 + 4) >> 2 : 0;
-    const bool fits = 4 * wv.quads <= CT - 2 && wv.quads <= kWave * ws_quads<ZPT>();
-    wv.flags = (any ? 1 : 0) | (all ? 2 : 0) | (fits ? 4 : 0);
-  }
-
-  WsPre<DT> pre;
-  int f_n = lane_i(wv.flags, 0);
-  if ((f_n & 5) == 5)
-    ws_issue<DT, ws_quads<ZPT>()>(pre, view_rsrc(a, 0), a.W, lane_i(wv.iu, 0), lane_i(wv.c0, 0),
-                                  lane_i(wv.quads, 0), lane);
-  for (int s = 0; s < a.nproj; ++s) {
-    const int f = f_n;
-    const float Vb = lane_f(wv.Vb, s), dV = lane_f(wv.dV, s);
-    float w0 = lane_f(wv.w0, s), w1 = lane_f(wv.w1, s);
-    const int c0 = lane_i(wv.c0, s), quads = lane_i(wv.quads, s);
-    float zof = 0.f;
-    float2 so = make_float2(1.f, 0.f);
     if (DT != FDK_F32) {
-      so = view_so(a, S, s);
-      zof = (w0 + w1) * so.y;
+      const float2 so = view_so(a, S, lane);
+      wv.zof = (wv.w0 + wv.w1) * so.y;
+      wv.w0 *= so.x;
+      wv.w1 *= so.x;
     }
-    if ((f & 5) == 5)
-      ws_commit<DT, ws_quads<ZPT>()>(pre, strip, DT == FDK_F32 ? w0 : w0 * so.x,
-                                     DT == FDK_F32 ? w1 : w1 * so.x, zof, quads, lane);
-    if (s + 1 < a.nproj) {
-      f_n = lane_i(wv.flags, s + 1);
-      if ((f_n & 5) == 5)
-        ws_issue<DT, ws_quads<ZPT>()>(pre, view_rsrc(a, s + 1), a.W, lane_i(wv.iu, s + 1),
-                                      lane_i(wv.c0, s + 1), lane_i(wv.quads, s + 1), lane);
-    }
-    if (!(f & 1)) continue;
-    if (f & 4) {
-      const float2* base = strip - c0;
-      if (f & 2)
-        ws_compute<false, ZPT>(acc, accm, zt, Vb, dV, base, zslot, a.W);
-      else
-        ws_compute<true, ZPT>(acc, accm, zt, Vb, dV, base, zslot, a.W);
-    } else {
-      // strip too wide for the LDS slot: the taps straight from memory
-      ColView c;
-      c.Vb = Vb;
-      c.dV = dV;
-      c.w0 = w0;
-      c.w1 = w1;
-      c.Z2 = lane_f(wv.Z2, s);
-      c.iu = lane_i(wv.iu, s);
-      c.uok = true;
-      float zm[ZPT];
+    // v over the run, as the compute evaluates it (monotone in z)
+    const float va = fmaf((float)(a.z0 + zb0), wv.dV, wv.Vb);
+    const float vb = fmaf((float)(a.z0 + zend), wv.dV, wv.Vb);
+    const int ilo = floor_int(fminf(va, vb)), ihi = floor_int(fmaxf(va, vb));
+    any = uok && ihi >= 0 && ilo <= a.W - 2;
+    all = uok && ilo >= 0 && ihi <= a.W - 2;
+    wv.c0 = max(ilo, 0) & ~3;
+    wv.off = any ? wv.iu * a.row_bytes + wv.c0 * (DT == FDK_F32 ? 4 : 2) : 0;
+    wv.quads = any ? (min(ihi + 1, a.W - 1) - wv.c0 + 4) >> 2 : 0;
+    // With rows of a multiple of 4 samples the quads end with the row.  Else the
+    // last one may reach up to 3 samples past it, which must not leave the view.
+    const int over = wv.c0 + 4 * wv.quads - a.W;
+    const bool inside = over <= 0 || (wv.iu + 3 <= a.H && (!SYM || wv.iu > 0));
+    fits = 4 * wv.quads <= CT - 2 && wv.quads <= kWave * NQ && inside;
+  }
+  // The wave's views: those whose whole run lies inside the view, then those that
+  // need the validity test (a loop each, so that each holds one form of the taps
+  // and the sums stay in place), then strips too wide for the LDS slot or at a
+  // corner of the view, whose taps come straight from memory.
+  unsigned mine = ~0u;
+  if constexpr (VS > 1) {
+    const int per = (a.nproj + VS - 1) / VS, s0 = wave * per;
+    mine = s0 < kMaxProj ? (unsigned)(((1ull << per) - 1) << s0) : 0u;
+  }
+  unsigned full = (unsigned)__ballot(any && fits && all) & mine;
+  unsigned edge = (unsigned)__ballot(any && fits && !all) & mine;
+  unsigned rest = (unsigned)__ballot(any && !fits) & mine;
+  WsPre<DT, SYM, NQ> pre;
+  int quads = 0;
+  // arguments the loop uses are here before it: a scalar load still pending at its
+  // entry would make every view wait for its LDS writes (one counter for both)
+  asm volatile("" ::"s"(a.proj), "s"(a.view_bytes), "s"(a.row_bytes), "s"(a.W));
+  if (full | edge) {
+    const int s = __ffs((int)(full ? full : edge)) - 1;
+    quads = lane_i(wv.quads, s);
+    ws_issue<DT, SYM, NQ>(pre, a, s, wv, quads, lane);
+  }
+  while (full) {
+    const int s = __ffs((int)full) - 1;
+    full &= full - 1;
+    ws_view<false, DT, SYM, ZPT, NQ>(acc, accm, zt, pre, quads, a, wv, s,
+                                     __ffs((int)(full ? full : edge)) - 1, strip, zslot, lane);
+  }
+  while (edge) {
+    const int s = __ffs((int)edge) - 1;
+    edge &= edge - 1;
+    ws_view<true, DT, SYM, ZPT, NQ>(acc, accm, zt, pre, quads, a, wv, s, __ffs((int)edge) - 1,
+                                    strip, zslot, lane);
+  }
+  for (; rest; rest &= rest - 1) {
+    const int s = __ffs((int)rest) - 1;
+    ColView c;
+    c.Vb = lane_f(wv.Vb, s);
+    c.dV = lane_f(wv.dV, s);
+    c.w0 = lane_f(wv.w0, s);
+    c.w1 = lane_f(wv.w1, s);
+    c.Z2 = lane_f(wv.Z2, s);
+    c.iu = lane_i(wv.iu, s);
+    c.uok = true;
+    const float of = DT != FDK_F32 ? view_so(a, S, s).y : 0.f;
+    float zm[ZPT];
 #pragma unroll
-      for (int j = 0; j < ZPT; ++j) zm[j] = (float)(a.nz - 1) - zt[j];
-      compute_direct<DT, true, ZPT>(acc, accm, zt, zm, c, a,
-                                    static_cast<const char*>(a.proj) + (size_t)s * a.view_bytes,
-                                    so.x, so.y);
+    for (int j = 0; j < ZPT; ++j) zm[j] = (float)(a.nz - 1) - zt[j];
+    compute_direct<DT, SYM, ZPT>(acc, accm, zt, zm, c, a,
+                                 static_cast<const char*>(a.proj) + (size_t)s * a.view_bytes,
+                                 1.f, of);
+  }
+  if constexpr (VS == 1) {
+    column_write<SYM, ZPT>(a, xs, ys, zbase, acc, accm);
+  } else {
+    // sums of the four view quarters: row r of 64 values is acc[r] or accm[r - ZPT]
+    constexpr int kRows = ZPT * kSides;
+    float* red = wstrip + 4 * CT * kSides;
+#pragma unroll
+    for (int j = 0; j < ZPT; ++j) {
+      red[(wave * kRows + j) * kWave + lane] = acc[j];
+      if (SYM) red[(wave * kRows + ZPT + j) * kWave + lane] = accm[j];
+    }
+    __syncthreads();
+    float* col = a.vol + ((long long)xs * a.nys + ys) * (long long)a.nzz;
+    for (int r = wave; r < kRows; r += 4) {
+      float v = 0.f;
+#pragma unroll
+      for (int w = 0; w < 4; ++w) v += red[(w * kRows + r) * kWave + lane];
+      const int zl = zbase + (r % ZPT) * kWave;
+      if (zl < a.zext) col[r < ZPT ? zl : a.nzz - 1 - zl] += v;
     }
   }
-  column_write<true, ZPT>(a, xs, ys, zbase, acc, accm);
 }
 
 // General matrices (a z term in rows 0 or 2): every voxel does the full
@@ -1138,9 +1289,10 @@ int fill_args(fdk_bp* h, int W, int H, long long view_stride, int esize, int npr
   return FDK_OK;
 }
 
-// Voxels per lane along z: 8, or 4 when that pads the column's z extent to
-// fewer wave runs (a 256-deep slab fills a ZPT 4 wave exactly and half of a
-// ZPT 8 one).  FDK_BP_ZPT = 4, 8 or 16 forces a value.
+// Voxels per lane along z of the older kernels: 8, or 4 when that pads the column's
+// z extent to fewer wave runs (a 256-deep slab fills a ZPT 4 wave exactly and half
+// of a ZPT 8 one).  FDK_BP_ZPT = 4, 8 or 16 forces a value (bp_wave_kernel: 1, 2, 4
+// or 8, 16 meaning 8).
 int zpt_choice(int zext) {
   static const int forced = [] {
     const char* e = std::getenv("FDK_BP_ZPT");
@@ -1187,8 +1339,8 @@ bool stage_dims(const BpArgs& a, const BpMats& M, int zpt, int* R, int* CT) {
 
 // Kernel choice: FDK_BP_KERNEL=v2 selects the direct-gather bp_column_kernel,
 // v3 the LDS-staged bp_lds_kernel, v4 bp_lds_pf_kernel where its register
-// prefetch covers the strip; by default bp_wave_kernel runs for mirror-symmetric
-// slab pairs whose strips fit, then the v4 / v3 / v2 chain.
+// prefetch covers the strip; by default bp_wave_kernel runs wherever its strips fit
+// (16-bit views also need 4-byte aligned rows and views), else the v4 / v3 / v2 chain.
 int kernel_choice() {
   static const int k = [] {
     const char* e = std::getenv("FDK_BP_KERNEL");
@@ -1220,26 +1372,34 @@ bool mirror_symmetric(const BpArgs& a, const BpMats& M) {
   return true;
 }
 
-// Strip slot CT (float2 per column, plus the two-entry zero slot) of
-// bp_wave_kernel: the v extent of one wave's z-run (64 * ZPT voxels) over the
-// views and the sub-volume's corners, with room for floor rounding and the
-// 4-column alignment of its start.  0 when a corner is behind the source.
-int wave_strip_ct(const BpArgs& a, const BpMats& M, int zpt) {
+// Strip slot CT (columns, plus the two-column zero slot) of bp_wave_kernel: the
+// v extent of one wave's z-run (64 * zpt voxels) over the views and the
+// sub-volume's corners, with room for floor rounding and the 4-column alignment
+// of its start.  0 when a corner is behind the source.
+int wave_strip_ct(double dvz, int zpt) {
+  const double span = dvz * (kWave * zpt - 1);
+  const double quads = (std::ceil(span) + 9) / 4 + 1;
+  return quads < 1e6 ? 4 * (int)quads + 2 : 0;
+}
+
+// The largest |dv/dz| over the views and the sub-volume's corners; 0 when a
+// corner is behind the source.
+double max_dvz(const BpArgs& a, const BpMats& M) {
   const double xs[2] = {(double)a.x0, (double)(a.x0 + a.nxs - 1)};
   const double ys[2] = {(double)a.y0, (double)(a.y0 + a.nys - 1)};
-  double dvz = 0.0;
+  double dvz = 1e-9;
   for (int s = 0; s < a.nproj; ++s) {
     const float* m = M.m[s];
     for (double x : xs)
       for (double y : ys) {
         const double w = (double)m[8] * x + (double)m[9] * y + (double)m[11];
-        if (!(w > 0.0)) return 0;
-        dvz = std::max(dvz, std::fabs((double)m[6] / w));
+        if (!(w > 0.0)) return 0.0;
+        const double d = std::fabs((double)m[6] / w);
+        if (!(d < 1e9)) return 0.0;
+        dvz = std::max(dvz, d);
       }
   }
-  const double span = dvz * (kWave * zpt - 1);
-  const int quads = ((int)std::ceil(span) + 9) / 4 + 1;
-  return 4 * quads + 2;
+  return dvz;
 }
 
 template <int DT, int ZPT>
@@ -1269,24 +1429,95 @@ bool launch_lds(fdk_bp* h, const BpArgs& a, const BpMats& M, const BpScale& S, u
   return true;
 }
 
-template <int DT, int ZPT>
-bool launch_wave(fdk_bp* h, const BpArgs& a, const BpMats& M, const BpScale& S, unsigned nblk) {
-  if (kernel_choice() < 5 || !h->sym || a.W % 4 != 0) return false;
-  if (DT != FDK_F32 && ((reinterpret_cast<uintptr_t>(a.proj) % 8) != 0 || a.view_stride % 4 != 0))
-    return false;
-  if (!mirror_symmetric(a, M)) return false;
-  const int CT = wave_strip_ct(a, M, ZPT);
-  if (CT <= 0 || (CT - 2) / 4 > kWave * ws_quads<ZPT>()) return false;
-  const size_t lds = (size_t)4 * CT * sizeof(float2);
-  if (lds > 64 * 1024) return false;
-  dim3 grid(nblk, (a.zext + kWave * ZPT - 1) / (kWave * ZPT));
-  hipLaunchKernelGGL((bp_wave_kernel<DT, ZPT>), grid, dim3(256), lds, h->stream, a, M, S, CT);
+// Waves below which the views are split over a block's four waves: 4096 is half a
+// wave in every slot of the chip (256 CUs x 4 SIMDs x 8).  Two passes with read-out,
+// split against whole: 32^3 pair 35.7 / 45.4 us, 48^3 equal, 112^3 159 / 150.
+constexpr long long kSplitWaves = 4096;
+
+template <int DT, bool SYM, int ZPT>
+bool launch_wave_zpt(fdk_bp* h, const BpArgs& a, const BpMats& M, const BpScale& S, int CT) {
+  constexpr int kSides = SYM ? 2 : 1;
+  size_t lds = (size_t)4 * CT * kSides * sizeof(float);
+  const unsigned npx = (unsigned)(a.nxs + 1) / 2, npy = (unsigned)(a.nys + 1) / 2;
+  const unsigned patches = npx * npy;
+  const WsGrid G{udiv_inv(kTile * npx), udiv_inv(kTile * std::max(1u, npy % kTile)),
+                 udiv_inv(std::max(1u, npx % kTile))};
+  dim3 grid((patches + 7u) & ~7u, (a.zext + kWave * ZPT - 1) / (kWave * ZPT));
+  if constexpr (ZPT <= 2) {
+    if ((long long)a.nxs * a.nys * grid.y < kSplitWaves && a.nproj >= 8) {
+      grid.x *= 4;
+      lds += (size_t)4 * ZPT * kSides * kWave * sizeof(float);
+      hipLaunchKernelGGL((bp_wave_kernel<DT, SYM, ZPT, 4>), grid, dim3(256), lds, h->stream, a, M, S, G, CT);
+      return true;
+    }
+  }
+  hipLaunchKernelGGL((bp_wave_kernel<DT, SYM, ZPT, 1>), grid, dim3(256), lds, h->stream, a, M, S, G, CT);
+  return true;
+}
+
+// Voxels per lane of bp_wave_kernel: of the values whose strips fit, the one with
+// the least vector instructions per view for a column of zext voxels.  A run of
+// 64 ZPT voxels costs about fixed + NQ staged quad slots + ZPT taps.  Forced values
+// (ZPT 1 / 2 / 4 / 8) agree: 512-deep slabs 34.5 / 19.7 / 15.1 / 14.4 ms, 256-deep
+// 8.1 / 4.5 / 3.2 / 4.1 ms, 128-deep 1.48 / 0.79 / 0.88 / 1.37 ms, a 256-deep single
+// slab 2.21 / 1.22 / 0.86 / 1.17 ms.
+template <bool SYM>
+int wave_zpt(double dvz, int zext, int* CT) {
+  constexpr int kZpt[4] = {8, 4, 2, 1}, kSlots[4] = {kWsQuads, 2, 1, 1};
+  constexpr int kFixed = 25, kSlot = SYM ? 20 : 10, kTap = SYM ? 9 : 7;
+  static const int forced = [] {
+    const char* e = std::getenv("FDK_BP_ZPT");
+    const int v = e ? std::atoi(e) : 0;
+    return v >= 8 ? 8 : (v == 4 || v == 2 || v == 1) ? v : 0;
+  }();
+  int best = 0;
+  long long cost = 0;
+  for (int k = 0; k < 4; ++k) {
+    const int z = kZpt[k], ct = wave_strip_ct(dvz, z);
+    if (ct <= 0 || (ct - 2) / 4 > kWave * kSlots[k]) continue;
+    if ((size_t)4 * ct * (SYM ? 2 : 1) * sizeof(float) > 60 * 1024) continue;
+    const long long runs = (zext + kWave * z - 1) / (kWave * z);
+    const long long c = runs * (kFixed + kSlots[k] * kSlot + z * kTap);
+    if (forced ? z == forced : (!best || c < cost)) {
+      best = z;
+      cost = c;
+      *CT = ct;
+    }
+  }
+  return best;
+}
+
+template <int DT, bool SYM>
+bool launch_wave_run(fdk_bp* h, const BpArgs& a, const BpMats& M, const BpScale& S,
+                     double dvz) {
+  int CT = 0;
+  switch (wave_zpt<SYM>(dvz, a.zext, &CT)) {
+    case 8: return launch_wave_zpt<DT, SYM, 8>(h, a, M, S, CT);
+    case 4: return launch_wave_zpt<DT, SYM, 4>(h, a, M, S, CT);
+    case 2: return launch_wave_zpt<DT, SYM, 2>(h, a, M, S, CT);
+    case 1: return launch_wave_zpt<DT, SYM, 1>(h, a, M, S, CT);
+  }
+  return false;
+}
+
+template <int DT>
+bool launch_wave(fdk_bp* h, const BpArgs& a, const BpMats& M, const BpScale& S) {
+  if (kernel_choice() < 5 || (DT != FDK_F32 && !a.buf16)) return false;
+  const double dvz = max_dvz(a, M);
+  if (!(dvz > 0.0)) return false;
+  if (h->sym && mirror_symmetric(a, M)) return launch_wave_run<DT, true>(h, a, M, S, dvz);
+  if (!launch_wave_run<DT, false>(h, a, M, S, dvz)) return false;
+  if (h->sym) {  // the bottom slab as a run of its own
+    BpArgs b = a;
+    b.z0 = (int)h->bot.z;
+    b.vol = a.vol + a.zext;
+    return launch_wave_run<DT, false>(h, b, M, S, dvz);
+  }
   return true;
 }
 
 template <int DT, int ZPT>
 void launch_column(fdk_bp* h, const BpArgs& a, const BpMats& M, const BpScale& S, unsigned nblk) {
-  if (launch_wave<DT, ZPT>(h, a, M, S, nblk)) return;
   if (launch_lds<DT, ZPT>(h, a, M, S, nblk)) return;
   dim3 grid(nblk, (a.zext + kWave * ZPT - 1) / (kWave * ZPT));
   if (h->sym) hipLaunchKernelGGL((bp_column_kernel<DT, true, ZPT>), grid, dim3(256), 0, h->stream, a, M, S);
@@ -1301,7 +1532,7 @@ int launch_bp_dt(fdk_bp* h, const BpArgs& a, const BpMats& M, const BpScale& S, 
     dim3 grid(nblk, (a.zext + kWave - 1) / kWave);
     if (h->sym) hipLaunchKernelGGL((bp_general_kernel<DT, true>), grid, dim3(256), 0, h->stream, a, M, S);
     else hipLaunchKernelGGL((bp_general_kernel<DT, false>), grid, dim3(256), 0, h->stream, a, M, S);
-  } else {
+  } else if (!launch_wave<DT>(h, a, M, S)) {
     switch (zpt_choice(a.zext)) {
       case 4: launch_column<DT, 4>(h, a, M, S, nblk); break;
       case 16: launch_column<DT, 16>(h, a, M, S, nblk); break;
