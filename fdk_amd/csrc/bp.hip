@@ -746,7 +746,8 @@ __global__ __launch_bounds__(256) void bp_lds_pf_kernel(BpArgs a, BpMats M, BpSc
 //    r(c) = w0 P[iu][c] + w1 P[iu+1][c] (w0, w1 the u weights times 1/w^2) over
 //    the v columns of its z-run, so a voxel's sample is one v interpolation;
 //  * SYM, a mirror slab pair whose matrices are mirror-symmetric (v(z) +
-//    v(nz-1-z) = W-1 for every column, checked on the host): the mirror run reads
+//    v(nz-1-z) = W-1 for every column, checked on the host) and whose rows are a
+//    multiple of 4 samples: the mirror run reads
 //    columns W-1-c, stored reversed and interleaved with the top run's, so one
 //    16-byte LDS read brings r_top(iv), r_mir(iv), r_top(iv+1), r_mir(iv+1).  The
 //    mirror voxel has v' = W-1-v, so iv' = W-2-iv and t' = 1-t: it shares the top
@@ -831,10 +832,9 @@ struct WsPre {
 };
 
 // Strip loads of one view: quad q of the top run reads columns c0+4q..c0+4q+3
-// of rows iu and iu+1; of the mirror run, columns W-4-c0-4q..W-1-c0-4q.  A quad
-// that reaches past its row's end reads on into the next row (or, mirrored, back
-// into the one before); the kernel keeps such quads inside the view, and only
-// columns of valid taps are ever used.
+// of rows iu and iu+1; of the mirror run (W % 4 == 0), columns W-4-c0-4q..W-1-c0-4q.
+// A quad that reaches past its row's end reads on into the next row; the kernel keeps
+// such quads inside the view, and only columns of valid taps are ever used.
 template <int DT, bool SYM, int NQ>
 __device__ __forceinline__ void ws_issue(WsPre<DT, SYM, NQ>& pre, const BpArgs& a, int s,
                                          const WaveView& wv, int quads, int lane) {
@@ -1064,7 +1064,7 @@ __global__ __launch_bounds__(256, (ws_waves<DT, SYM, ZPT>())) void bp_wave_kerne
     // With rows of a multiple of 4 samples the quads end with the row.  Else the
     // last one may reach up to 3 samples past it, which must not leave the view.
     const int over = wv.c0 + 4 * wv.quads - a.W;
-    const bool inside = over <= 0 || (wv.iu + 3 <= a.H && (!SYM || wv.iu > 0));
+    const bool inside = over <= 0 || wv.iu + 3 <= a.H;
     fits = 4 * wv.quads <= CT - 2 && wv.quads <= kWave * NQ && inside;
   }
   // The wave's views: those whose whole run lies inside the view, then those that
@@ -1505,7 +1505,13 @@ bool launch_wave(fdk_bp* h, const BpArgs& a, const BpMats& M, const BpScale& S) 
   if (kernel_choice() < 5 || (DT != FDK_F32 && !a.buf16)) return false;
   const double dvz = max_dvz(a, M);
   if (!(dvz > 0.0)) return false;
-  if (h->sym && mirror_symmetric(a, M)) return launch_wave_run<DT, true>(h, a, M, S, dvz);
+  // The mirrored run takes v' = W-1-v where the matrices give v' by themselves: equal
+  // to rounding, but a voxel on the detector's edge can fall on the other side of it.
+  // Rows of a multiple of 4 samples have always been read that way; others keep the
+  // matrices' positions, one run a slab.
+  const bool quads = a.W % 4 == 0 && (DT == FDK_F32 || (reinterpret_cast<uintptr_t>(a.proj) % 8 == 0 &&
+                                                        a.view_stride % 4 == 0));
+  if (h->sym && quads && mirror_symmetric(a, M)) return launch_wave_run<DT, true>(h, a, M, S, dvz);
   if (!launch_wave_run<DT, false>(h, a, M, S, dvz)) return false;
   if (h->sym) {  // the bottom slab as a run of its own
     BpArgs b = a;
