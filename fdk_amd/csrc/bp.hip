@@ -1622,6 +1622,11 @@ extern "C" int fdk_bp_create(int proj_width, int proj_height, int proj_count, in
   (void)hipGetDevice(&h->device);
   const size_t nvox = (size_t)h->top.w * h->top.h * h->nzz;
   hipError_t e = hipMalloc(&h->vol, nvox * sizeof(float));
+  if (e == hipErrorOutOfMemory) {  // once more with the library's scratch given back
+    (void)hipGetLastError();
+    fdk::scratch_trim();
+    e = hipMalloc(&h->vol, nvox * sizeof(float));
+  }
   if (e == hipSuccess) e = hipMemset(h->vol, 0, nvox * sizeof(float));
   h->staging_elems = (size_t)proj_width * proj_height * proj_count;
   if (e == hipSuccess) e = hipMalloc(&h->staging, h->staging_elems * sizeof(float));

@@ -5,6 +5,7 @@
 #include <map>
 #include <mutex>
 #include <string>
+#include <vector>
 
 #include "common.hpp"
 
@@ -53,6 +54,109 @@ int stage_alloc(void** p, size_t bytes, hipStream_t st) {
   }
   FDK_HIP(hipMallocFromPoolAsync(p, bytes, pool, st));
   return FDK_OK;
+}
+
+namespace {
+
+// Allocating and freeing would be refused while another thread captures a stream
+// in the default mode; these allocations are no part of any graph.
+struct Relaxed {
+  hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+  Relaxed() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+  ~Relaxed() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+};
+
+std::mutex g_scratch_mutex;
+std::map<int, std::vector<Scratch>> g_scratch;  // kept blocks, by device
+
+void scratch_free(Scratch& s) {
+  Relaxed relaxed;
+  (void)hipEventSynchronize(s.done);
+  (void)hipFree(s.p);
+  (void)hipEventDestroy(s.done);
+  (void)hipGetLastError();
+  s = Scratch{};
+}
+
+// The current device's kept blocks, taken off the list.
+std::vector<Scratch> scratch_take_all() {
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess) return {};
+  std::lock_guard<std::mutex> lock(g_scratch_mutex);
+  std::vector<Scratch> v;
+  v.swap(g_scratch[dev]);
+  return v;
+}
+
+}  // namespace
+
+void scratch_trim() {
+  for (Scratch& s : scratch_take_all()) scratch_free(s);
+}
+
+int scratch_get(Scratch* s, size_t bytes, hipStream_t st) {
+  *s = Scratch{};
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess) return FDK_ERR_HIP;
+  if (bytes > kScratchKeep) {
+    s->bytes = bytes;
+    if (hipMallocAsync(&s->p, bytes, st) == hipSuccess) return FDK_OK;
+    (void)hipGetLastError();
+    *s = Scratch{};
+    return FDK_ERR_OOM;
+  }
+  {
+    std::lock_guard<std::mutex> lock(g_scratch_mutex);
+    std::vector<Scratch>& v = g_scratch[dev];
+    size_t best = v.size();
+    for (size_t k = 0; k < v.size(); ++k)
+      if (v[k].bytes >= bytes && (best == v.size() || v[k].bytes < v[best].bytes)) best = k;
+    if (best < v.size()) {
+      *s = v[best];
+      v.erase(v.begin() + (long)best);
+    }
+  }
+  if (s->p) {
+    if (hipStreamWaitEvent(st, s->done, 0) == hipSuccess) return FDK_OK;
+    scratch_free(*s);  // waits for the block's last work instead
+  }
+  scratch_trim();  // a larger block replaces the kept ones
+  Relaxed relaxed;
+  s->bytes = (bytes + (2u << 20) - 1) >> 21 << 21;
+  if (hipEventCreateWithFlags(&s->done, hipEventDisableTiming) == hipSuccess) {
+    if (hipMalloc(&s->p, s->bytes) == hipSuccess) return FDK_OK;
+    (void)hipEventDestroy(s->done);
+  }
+  (void)hipGetLastError();
+  *s = Scratch{};
+  return FDK_ERR_OOM;
+}
+
+void scratch_put(Scratch* s, hipStream_t st) {
+  if (!s->p) return;
+  if (!s->done) {
+    (void)hipFreeAsync(s->p, st);
+    *s = Scratch{};
+    return;
+  }
+  int dev = 0;
+  if (hipEventRecord(s->done, st) != hipSuccess || hipGetDevice(&dev) != hipSuccess) {
+    (void)hipStreamSynchronize(st);
+    scratch_free(*s);
+    return;
+  }
+  {
+    std::lock_guard<std::mutex> lock(g_scratch_mutex);
+    std::vector<Scratch>& v = g_scratch[dev];
+    size_t kept = s->bytes;
+    for (const Scratch& q : v) kept += q.bytes;
+    if (kept <= kScratchKeep) {
+      v.push_back(*s);
+      *s = Scratch{};
+      return;
+    }
+  }
+  scratch_free(*s);
 }
 
 }  // namespace fdk

@@ -149,15 +149,13 @@ __device__ inline float tap_blend(const TapBuf& b) {
   return v0 * (1.f - b.fz) + v1 * b.fz;
 }
 
-template <int MODE, bool BUF>
-__global__ __launch_bounds__(256) void fp_kernel(RayGeom g, const float* __restrict__ vol,
-                                                 float step, float* __restrict__ out) {
-  const int i = blockIdx.x * 64 + threadIdx.x;
-  const int j = blockIdx.y * 4 + threadIdx.y;
-  const int sv = blockIdx.z;
-  if (i >= g.nu || j >= g.nv) return;
+// The ray of a pixel in voxel coordinates, o + t s with t in mm, and the part of it
+// between the planes of the outermost voxel centres; false: it misses them.
+__device__ __forceinline__ bool ray_span(const RayGeom& g, int view, int i, int j, float& ox,
+                                         float& oy, float& oz, float& sx, float& sy, float& sz,
+                                         float& tnear, float& tfar) {
   double o[3], d[3];
-  pixel_ray(g, g.first + sv, i, j, o, d);
+  pixel_ray(g, view, i, j, o, d);
   // slab test against the voxel-centre box
   const double bmax[3] = {g.cx * g.vx, g.cy * g.vy, g.cz * g.vz};
   double tn = -1e300, tf = 1e300;
@@ -167,19 +165,30 @@ __global__ __launch_bounds__(256) void fp_kernel(RayGeom g, const float* __restr
     tn = fmax(tn, fmin(t0, t1));
     tf = fmin(tf, fmax(t0, t1));
   }
+  ox = (float)(o[0] / g.vx + g.cx), oy = (float)(g.cy - o[1] / g.vy), oz = (float)(g.cz - o[2] / g.vz);
+  sx = (float)(d[0] / g.vx), sy = (float)(-d[1] / g.vy), sz = (float)(-d[2] / g.vz);
+  tnear = (float)tn;
+  tfar = (float)tf;
+  return tf > tn;
+}
+
+template <int MODE, bool BUF>
+__global__ __launch_bounds__(256) void fp_kernel(RayGeom g, const float* __restrict__ vol,
+                                                 float step, float* __restrict__ out) {
+  const int i = blockIdx.x * 64 + threadIdx.x;
+  const int j = blockIdx.y * 4 + threadIdx.y;
+  const int sv = blockIdx.z;
+  if (i >= g.nu || j >= g.nv) return;
+  float ox, oy, oz, sx, sy, sz, tnear, tfar;
   float sum = 0.f;
-  if (tf > tn) {
-    const float ox = (float)(o[0] / g.vx + g.cx), oy = (float)(g.cy - o[1] / g.vy),
-                oz = (float)(g.cz - o[2] / g.vz);
-    const float sx = (float)(d[0] / g.vx), sy = (float)(-d[1] / g.vy), sz = (float)(-d[2] / g.vz);
-    const float tfar = (float)tf;
+  if (ray_span(g, g.first + sv, i, j, ox, oy, oz, sx, sy, sz, tnear, tfar)) {
     // Four samples per iteration: their gathers are issued together, so one
     // memory latency covers four steps.  t advances by the same float additions
     // and the samples are summed in the same order as a one-step loop, and a
     // sample past tfar adds nothing, so the result is the one-step loop's.
     const __amdgpu_buffer_rsrc_t rv = __builtin_amdgcn_make_buffer_rsrc(
         (void*)vol, 0, BUF ? g.nx * g.ny * g.nz * 4 : 0, fdk::kRawRsrcWord3);
-    float t = (float)tn;
+    float t = tnear;
     bool more = MODE == FDK_FP_CLAMP ? t < tfar : t <= tfar;
     while (more) {
       float tk[4], sk[4];
@@ -208,6 +217,146 @@ __global__ __launch_bounds__(256) void fp_kernel(RayGeom g, const float* __restr
         if (ok[k]) sum += sk[k];
       t = tk[3] + step;
       more = ok[3] && (MODE == FDK_FP_CLAMP ? t < tfar : t <= tfar);
+    }
+  }
+  out[((long long)sv * g.nv + j) * g.nu + i] = sum * step;
+}
+
+// ------------------------------------------------------ z-fastest form of the march
+// fp_zfast_kernel marches the same rays through a copy of the volume in
+// [x][y][z] order, padded by two voxels on every side.  A wave's 64 lanes are 64
+// detector rows v of one column u: their rays cross the same few (x, y) columns at
+// every step, whatever the view angle, and 64 neighbouring z of them, so a tap load
+// reads one run of about 70 voxels.  (Lanes along u, as in fp_kernel, step across the
+// volume's rows: one cache line a lane where the rays run along x.)  The pads hold
+// what the edge mode asks for -- the edge voxel, or zero -- so no tap is clamped,
+// selected or masked; indices past the pads are clamped into them.
+//
+// What bounds it: the texture-address unit, which takes 16 clocks for a wave's
+// gather whether a lane asks for 4, 8 or (nearly) 16 bytes (busy 91 % of the time
+// with four 8-byte gathers a sample, vector issue 60 %).  So the copy holds each
+// voxel beside its y neighbour and one 16-byte gather brings four of the eight taps:
+// two gathers a sample.
+// Measured, 24 views of 256^2 through 256^3 at half-voxel steps: 5.10 ms (fp_kernel)
+// -> 1.38 (8-byte gathers) -> 0.78 ms, 830 Gsamples/s, copy included.  Splitting the rays over
+// 4 or 16 waves for launches with few of them gained nothing (8 views: 313 against
+// 230 us).
+constexpr int kFpPad = 2;
+constexpr int kFpTurn = 3;  // samples in flight a ray: 3 and 4 alike (783 us), 2 slower (807 us)
+
+// dst[x][y][z] = {v(x, y, z), v(x, y + 1, z)} over the padded volume.
+template <int MODE>
+__global__ __launch_bounds__(256) void fp_pad_kernel(const float* __restrict__ vol,
+                                                     float2* __restrict__ dst, int nx, int ny, int nz) {
+  __shared__ float t[2][32][33];
+  const int mx = nx + 2 * kFpPad, my = ny + 2 * kFpPad, mz = nz + 2 * kFpPad;
+  const int x0 = blockIdx.x * 32, z0 = blockIdx.y * 32;
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    const int y = (int)blockIdx.z - kFpPad + h;
+    const int cy = min(max(y, 0), ny - 1);
+    for (int k = threadIdx.y; k < 32; k += 8) {
+      const int x = x0 + (int)threadIdx.x - kFpPad, z = z0 + k - kFpPad;
+      const int cx = min(max(x, 0), nx - 1), cz = min(max(z, 0), nz - 1);
+      const float v = vol[((long long)cz * ny + cy) * nx + cx];
+      t[h][k][threadIdx.x] = MODE == FDK_FP_CLAMP || (cx == x && cy == y && cz == z) ? v : 0.f;
+    }
+  }
+  __syncthreads();
+  for (int k = threadIdx.y; k < 32; k += 8) {
+    const int x = x0 + k, z = z0 + (int)threadIdx.x;
+    if (x < mx && z < mz)
+      dst[((long long)x * my + blockIdx.z) * mz + z] = make_float2(t[0][threadIdx.x][k], t[1][threadIdx.x][k]);
+  }
+}
+
+typedef float f32x4_a8 __attribute__((ext_vector_type(4), aligned(8)));
+
+// The eight taps of a sample: q[x] = {(y0,z0), (y1,z0), (y0,z1), (y1,z1)}.
+struct TapZ {
+  float4 q[2];
+  float fx, fy, fz;
+};
+
+// BUF: 32-bit byte offsets through a buffer resource.
+template <bool BUF>
+__device__ __forceinline__ TapZ tap_fetch_z(__amdgpu_buffer_rsrc_t rv, const float2* __restrict__ vol,
+                                            int nx, int ny, int nz, float px, float py, float pz) {
+  TapZ b;
+  const float tx = truncf(px), ty = truncf(py), tz = truncf(pz);  // as the reference
+  b.fx = px - tx;
+  b.fy = py - ty;
+  b.fz = pz - tz;
+  const int my = ny + 2 * kFpPad, mz = nz + 2 * kFpPad;
+  const int ix = (int)__builtin_amdgcn_fmed3f(tx, -(float)kFpPad, (float)nx);
+  const int iy = (int)__builtin_amdgcn_fmed3f(ty, -(float)kFpPad, (float)ny);
+  const int iz = (int)__builtin_amdgcn_fmed3f(tz, -(float)kFpPad, (float)nz);
+  if constexpr (BUF) {
+    // |ix my + iy| < 2^23 (checked on the host): full-rate 24-bit products
+    const int off = ((__mul24(__mul24(ix, my) + iy, mz) + iz) << 3) +
+                    ((kFpPad * my + kFpPad) * mz + kFpPad) * 8;
+    b.q[0] = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(rv, off, 0, 0));
+    b.q[1] = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(rv, off, my * mz * 8, 0));
+  } else {
+    const float2* p = vol + ((long long)(ix + kFpPad) * my + iy + kFpPad) * mz + iz + kFpPad;
+    const f32x4_a8 a = *reinterpret_cast<const f32x4_a8*>(p);
+    const f32x4_a8 c = *reinterpret_cast<const f32x4_a8*>(p + (long long)my * mz);
+    b.q[0] = make_float4(a.x, a.y, a.z, a.w);
+    b.q[1] = make_float4(c.x, c.y, c.z, c.w);
+  }
+  return b;
+}
+
+__device__ __forceinline__ float lerp(float a, float b, float t) { return fmaf(t, b - a, a); }
+
+__device__ __forceinline__ float tap_blend_z(const TapZ& b) {
+  const float4 a = b.q[0], c = b.q[1];
+  const float v0 = lerp(lerp(a.x, c.x, b.fx), lerp(a.y, c.y, b.fx), b.fy);
+  const float v1 = lerp(lerp(a.z, c.z, b.fx), lerp(a.w, c.w, b.fx), b.fy);
+  return lerp(v0, v1, b.fz);
+}
+
+// Grid: x = blocks in the order v, u, view, rounded up to a multiple of 8 and
+// remapped so that each XCD marches a contiguous run of them (4 % on 24 views of
+// 256^2 through 256^3).
+template <int MODE, bool BUF>
+__global__ __launch_bounds__(256) void fp_zfast_kernel(RayGeom g, const float2* __restrict__ vol,
+                                                       int vol_bytes, float step, int bv, int bu,
+                                                       long long blocks, float* __restrict__ out) {
+  const long long b = (long long)(blockIdx.x % 8u) * (gridDim.x / 8u) + blockIdx.x / 8u;
+  if (b >= blocks) return;
+  const int j = (int)(b % bv) * 64 + threadIdx.x;
+  const int i = (int)(b / bv % bu) * 4 + threadIdx.y;
+  const int sv = (int)(b / bv / bu);
+  if (i >= g.nu || j >= g.nv) return;
+  float ox, oy, oz, sx, sy, sz, tnear, tfar;
+  float sum = 0.f;
+  if (ray_span(g, g.first + sv, i, j, ox, oy, oz, sx, sy, sz, tnear, tfar)) {
+    const __amdgpu_buffer_rsrc_t rv = __builtin_amdgcn_make_buffer_rsrc(
+        (void*)vol, 0, BUF ? vol_bytes : 0, fdk::kRawRsrcWord3);
+    float t = tnear;
+    bool more = MODE == FDK_FP_CLAMP ? t < tfar : t <= tfar;
+    while (more) {  // kFpTurn samples a turn, summed in step order (see fp_kernel)
+      float tk[kFpTurn], sk[kFpTurn];
+      bool ok[kFpTurn];
+      TapZ tb[kFpTurn];
+      tk[0] = t;
+#pragma unroll
+      for (int k = 1; k < kFpTurn; ++k) tk[k] = tk[k - 1] + step;
+#pragma unroll
+      for (int k = 0; k < kFpTurn; ++k)
+        tb[k] = tap_fetch_z<BUF>(rv, vol, g.nx, g.ny, g.nz, fmaf(sx, tk[k], ox), fmaf(sy, tk[k], oy),
+                                 fmaf(sz, tk[k], oz));
+#pragma unroll
+      for (int k = 0; k < kFpTurn; ++k) {
+        sk[k] = tap_blend_z(tb[k]);
+        ok[k] = MODE == FDK_FP_CLAMP ? tk[k] < tfar : tk[k] <= tfar;
+      }
+#pragma unroll
+      for (int k = 0; k < kFpTurn; ++k)
+        if (ok[k]) sum += sk[k];
+      t = tk[kFpTurn - 1] + step;
+      more = ok[kFpTurn - 1] && (MODE == FDK_FP_CLAMP ? t < tfar : t <= tfar);
     }
   }
   out[((long long)sv * g.nv + j) * g.nu + i] = sum * step;
@@ -315,6 +464,70 @@ int upload_ell(const fdk_ellipsoid* host, int n, hipStream_t st, EllDev** out) {
   return FDK_OK;
 }
 
+// Seconds fp_kernel takes for a view's samples more than fp_zfast_kernel would.  Its
+// lanes step along u, so |sin a| of a voxel row apart: a gather costs it from one
+// line (rays along y) to a line a lane (rays along x).  Measured through 256^3: 2 ps a
+// sample at 0 degrees, 10 ps at 90, 7.4 ps averaged over a scan; fp_zfast_kernel
+// takes 1.2 ps at every angle.
+double zfast_saving(const RayGeom& r, int count, double step) {
+  const double diag = std::hypot(r.nx * r.vx, r.ny * r.vy);
+  const double samples = (double)r.nu * r.nv * 0.6 * diag / step;  // a view's, about
+  double ps = 0.0;
+  for (int k = 0; k < count; ++k) {
+    const double a = r.direction * ((r.first + k) * r.scan_deg / r.nproj) / 180.0 * kPi + r.vpa;
+    ps += 2.0 + 8.0 * std::fabs(std::sin(a)) - 1.2;
+  }
+  return samples * ps * 1e-12;
+}
+
+// Seconds for the padded copy: 12 us for the second launch and the block's event, and
+// 12 bytes a voxel at 2.8 TB/s (75 us at 256^3).  One view at 0 degrees stays with
+// fp_kernel (256^3: 52 against 106 us), four round the scan do not (327 against 140).
+double zfast_cost(double voxels) { return 12e-6 + voxels * 12.0 / 2.8e12; }
+
+// Runs fp_zfast_kernel (and the padded copy it reads) where it pays; *done says
+// whether it did.  It does not while the stream is captured, where nothing is
+// allocated, nor when the copy does not fit in device memory.
+int launch_zfast(const RayGeom& r, const float* vol, int count, float step, int mode, float* out,
+                 hipStream_t st, bool* done) {
+  *done = false;
+  const long long mx = r.nx + 2 * kFpPad, my = r.ny + 2 * kFpPad, mz = r.nz + 2 * kFpPad;
+  if (zfast_saving(r, count, step) < 1.2 * zfast_cost((double)mx * my * mz)) return FDK_OK;
+  if (my > 65535) return FDK_OK;  // grid z of the copy
+  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(st, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone) {
+    (void)hipGetLastError();
+    return FDK_OK;
+  }
+  const size_t bytes = (size_t)(mx * my * mz) * sizeof(float2);
+  const long long bv = (r.nv + 63) / 64, bu = (r.nu + 3) / 4, blocks = bv * bu * count;
+  if (blocks > (1LL << 22)) return FDK_OK;  // 2^30 threads
+  fdk::Scratch ws;
+  if (fdk::scratch_get(&ws, bytes, st) != FDK_OK) return FDK_OK;
+  float2* pad = static_cast<float2*>(ws.p);
+  const dim3 pg((unsigned)(mx + 31) / 32, (unsigned)(mz + 31) / 32, (unsigned)my);
+  if (mode == FDK_FP_CLAMP)
+    hipLaunchKernelGGL((fp_pad_kernel<FDK_FP_CLAMP>), pg, dim3(32, 8), 0, st, vol, pad, r.nx, r.ny, r.nz);
+  else
+    hipLaunchKernelGGL((fp_pad_kernel<FDK_FP_ZERO>), pg, dim3(32, 8), 0, st, vol, pad, r.nx, r.ny, r.nz);
+  const dim3 grid((unsigned)((blocks + 7) / 8 * 8));
+  const bool buf = bytes < (1ull << 31) && mx * my < (1LL << 23) && mz < (1LL << 23);
+  const int nb = buf ? (int)bytes : 0, nbv = (int)bv, nbu = (int)bu;
+  if (mode == FDK_FP_CLAMP && buf)
+    hipLaunchKernelGGL((fp_zfast_kernel<FDK_FP_CLAMP, true>), grid, dim3(64, 4), 0, st, r, pad, nb, step, nbv, nbu, blocks, out);
+  else if (mode == FDK_FP_CLAMP)
+    hipLaunchKernelGGL((fp_zfast_kernel<FDK_FP_CLAMP, false>), grid, dim3(64, 4), 0, st, r, pad, nb, step, nbv, nbu, blocks, out);
+  else if (buf)
+    hipLaunchKernelGGL((fp_zfast_kernel<FDK_FP_ZERO, true>), grid, dim3(64, 4), 0, st, r, pad, nb, step, nbv, nbu, blocks, out);
+  else
+    hipLaunchKernelGGL((fp_zfast_kernel<FDK_FP_ZERO, false>), grid, dim3(64, 4), 0, st, r, pad, nb, step, nbv, nbu, blocks, out);
+  const hipError_t e = hipGetLastError();
+  fdk::scratch_put(&ws, st);
+  if (e != hipSuccess) return fdk::fail(FDK_ERR_HIP, "forward projection: %s", hipGetErrorString(e));
+  *done = true;
+  return FDK_OK;
+}
+
 }  // namespace
 
 extern "C" int fdk_fp_project(const fdk_geometry* g, const float* dev_vol, int first, int count,
@@ -327,6 +540,9 @@ extern "C" int fdk_fp_project(const fdk_geometry* g, const float* dev_vol, int f
   if (step_mm <= 0) step_mm = std::min(g->dx, std::min(g->dy, g->dz));
   if (count == 0) return FDK_OK;
   hipStream_t st = static_cast<hipStream_t>(stream);
+  bool done = false;
+  if (int rc = launch_zfast(r, dev_vol, count, (float)step_mm, mode, dev_out, st, &done)) return rc;
+  if (done) return FDK_OK;
   dim3 grid((g->nu + 63) / 64, (g->nv + 3) / 4, count);
   // paired-tap buffer path when the volume's byte offsets fit 32 bits
   const bool buf = g->nx >= 2 && (long long)g->nx * g->ny * g->nz * 4 < (1LL << 31);
