@@ -15,17 +15,12 @@
 // MI355X design: one workgroup filters two rows at once as one complex
 // transform (row a in the real part, row b in the imaginary part).  Because H
 // is real and even, H * DFT(a + i b) inverts to filt(a) + i filt(b) exactly, so
-// no real-to-complex unpacking is needed.  For N = 2^9 .. 2^13 the transform is
-// a Stockham plan of radix-16 (and radix-2/4/8) passes with compile-time
-// strides, the inverse running the forward radices in reverse order: each
-// thread keeps the points it loaded for the first pass, multiplies by H in
-// registers between the last forward and first inverse pass, and stores the
-// points its last inverse pass produced, so only the inner passes go through
-// LDS (N complex floats, 64 KiB at N = 8192).  Other lengths run an in-place
-// radix-2^2 FFT entered in bit-reversed order, the filter multiply doubling as
-// the inverse's bit-reversal.  Loads apply the cos table, stores crop,
-// optionally transpose (v fastest, what the backprojector reads) and convert to
-// the stored dtype.  Twiddles are an FP64-built table.
+// no real-to-complex unpacking is needed.  filter_wide_kernel (N = 2^7 .. 2^14) holds 16
+// points a thread and runs radix-16 passes (the last ones of radix 2 to 16), the inverse
+// as the forward passes' adjoint; other lengths run an in-place radix-2^2 FFT entered in
+// bit-reversed order, the filter multiply doubling as the inverse's bit-reversal.  Loads
+// apply the cos table, stores crop, optionally transpose (v fastest, what the
+// backprojector reads) and convert to the stored dtype.  Twiddles are an FP64-built table.
 #include <hip/hip_runtime.h>
 #include <hip/hip_fp16.h>
 
@@ -111,14 +106,7 @@ __device__ void fft_lds(float2* buf, const float2* __restrict__ tw, int N, int l
   }
 }
 
-// ---------------------------------------------------------------- Stockham FFT
-// Self-sorting mixed-radix FFT in LDS (natural order in and out): each pass
-// reads R values per butterfly (stride N/R), twiddles them, runs a radix-R DFT
-// in registers and writes them back at stride Ns, the product of the radices
-// before it.  Radix-16/8 passes cut the LDS round trips per transform to 3-4
-// (against log4 N in-place passes with a bit-reversed entry), and the filter
-// multiply rides on the first inverse pass's reads.
-
+// ------------------------------------------------ register DFTs of filter_wide_kernel
 // v * (sign * i): sign -1 multiplies by -i, +1 by +i.
 __device__ __forceinline__ float2 mul_si(float2 v, float sign) {
   return sign < 0 ? make_float2(v.y, -v.x) : make_float2(-v.y, v.x);
@@ -213,204 +201,6 @@ __device__ __forceinline__ void dft<16>(float2 (&v)[16], float sign) {
   for (int k = 0; k < 16; ++k) v[k] = x[k];
 }
 
-// LDS slot of point i: with PAD, one spare slot after every 16 points, so the
-// stride-16 writes of the first pass (and the 2 KiB-apart runs of the second)
-// spread over the banks instead of landing on one.
-template <bool PAD>
-__device__ __forceinline__ int sk_slot(int i) {
-  return PAD ? i + (i >> 4) : i;
-}
-
-// Slot distance of a run of d points, d a multiple of 16: the pad term of
-// sk_slot(i + d) then carries no bit from i, so sk_slot(i + d) = sk_slot(i) + sk_span(d).
-template <bool PAD>
-constexpr int sk_span(int d) {
-  return PAD ? d + d / 16 : d;
-}
-
-// Stockham passes over N points in buf with BPT butterflies per thread: a pass
-// of radix R reads the R values of butterfly j at stride NB = N / R, twiddles
-// them by e^{-2 pi i (j mod NS) r / (NS R)} (NS = the product of the radices
-// before it), runs a radix-R DFT in registers and writes them at stride NS.
-// N, NS and the radix are compile-time, so every LDS access is one per-thread
-// base plus an immediate offset.  Butterfly q of a thread is j = tid + 256 q;
-// a pass with fewer than 256 butterflies leaves the upper threads idle.
-template <int N, int R, int BPT>
-__device__ __forceinline__ bool sk_active(int q) {
-  constexpr int NB = N / R;
-  return NB >= 256 * (q + 1) || (int)threadIdx.x + q * 256 < NB;
-}
-
-template <int R, int BPT, bool PAD, int N>
-__device__ __forceinline__ void sk_read(const float2* buf, float2 (&v)[BPT][R]) {
-  constexpr int NB = N / R;
-  static_assert(NB % 16 == 0, "a read stride keeps the pad term separable");
-  constexpr int kReadSpan = sk_span<PAD>(NB);
-#pragma unroll
-  for (int q = 0; q < BPT; ++q) {
-    if (sk_active<N, R, BPT>(q)) {
-      const float2* src = buf + sk_slot<PAD>(threadIdx.x + q * 256);
-#pragma unroll
-      for (int r = 0; r < R; ++r) v[q][r] = src[r * kReadSpan];
-    }
-  }
-}
-
-template <int R, int BPT, int N, int NS>
-__device__ __forceinline__ void sk_dft(float2 (&v)[BPT][R], float sign, const float2* __restrict__ tw) {
-#pragma unroll
-  for (int q = 0; q < BPT; ++q) {
-    if (sk_active<N, R, BPT>(q)) {
-      if constexpr (NS > 1) {
-        // twiddle r of this butterfly: tw[step r], e^{-2 pi i step r / N}
-        const int j = threadIdx.x + q * 256;
-        const unsigned step8 = (unsigned)((j & (NS - 1)) * (N / (NS * R))) * 8u;
-        const __amdgpu_buffer_rsrc_t twr =
-            __builtin_amdgcn_make_buffer_rsrc((void*)tw, 0, N * 8, fdk::kRawRsrcWord3);
-        unsigned off = 0;
-#pragma unroll
-        for (int r = 1; r < R; ++r) {
-          off += step8;
-          float2 w = __builtin_bit_cast(float2, __builtin_amdgcn_raw_buffer_load_b64(twr, off, 0, 0));
-          w.y *= -sign;
-          v[q][r] = cmul(v[q][r], w);
-        }
-      }
-      dft<R>(v[q], sign);
-    }
-  }
-}
-
-template <int R, int BPT, bool PAD, int N, int NS>
-__device__ __forceinline__ void sk_write(float2* buf, const float2 (&v)[BPT][R]) {
-#pragma unroll
-  for (int q = 0; q < BPT; ++q) {
-    if (sk_active<N, R, BPT>(q)) {
-      const int j = threadIdx.x + q * 256;
-      const int k = j & (NS - 1);
-      const int base = (j - k) * R + k;
-      if constexpr (NS == 1) {
-        // base = j R: its R outputs stay inside one 16-point run (R <= 16, base % 16 + R <= 16)
-        float2* dst = buf + sk_slot<PAD>(base);
-#pragma unroll
-        for (int r = 0; r < R; ++r) dst[r] = v[q][r];
-      } else if constexpr (NS % 16 == 0) {
-        float2* dst = buf + sk_slot<PAD>(base);
-#pragma unroll
-        for (int r = 0; r < R; ++r) dst[r * sk_span<PAD>(NS)] = v[q][r];
-      } else {
-#pragma unroll
-        for (int r = 0; r < R; ++r) buf[sk_slot<PAD>(base + r * NS)] = v[q][r];
-      }
-    }
-  }
-}
-
-// One pass LDS -> LDS.
-template <int R, int BPT, bool PAD, int N, int NS>
-__device__ __forceinline__ void sk_pass(float2* buf, float sign, const float2* __restrict__ tw) {
-  float2 v[BPT][R];
-  sk_read<R, BPT, PAD, N>(buf, v);
-  sk_dft<R, BPT, N, NS>(v, sign, tw);
-  __syncthreads();  // every thread has read its inputs
-  sk_write<R, BPT, PAD, N, NS>(buf, v);
-  __syncthreads();
-}
-
-template <int N, int R>
-constexpr int sk_bpt() {
-  return N / R >= 256 ? N / R / 256 : 1;
-}
-
-// The whole filter on a thread's N/256 points, x[i] = point tid + 256 i on the
-// way in and out: forward passes of radices R1, R2, R3 (, R4), the filter
-// multiply, and inverse passes in the reverse radix order.  With that order
-// the points a thread loads are its first pass's inputs, its last forward
-// pass's outputs are its first inverse pass's inputs (the multiply runs in
-// registers), and its last inverse pass's outputs are the points it stores, so
-// of the 2 x passes LDS round trips only 2 x (passes - 1) remain.  R4 = 1:
-// three passes per direction.
-template <int R1, int R2, int R3, int R4, bool PAD>
-__device__ __forceinline__ void sk_filter(float2* buf, const float2* __restrict__ tw,
-                                          const float* __restrict__ H,
-                                          float2 (&x)[R1 * R2 * R3 * R4 / 256]) {
-  constexpr int N = R1 * R2 * R3 * R4;
-  constexpr int RL = R4 > 1 ? R4 : R3;      // last forward radix = first inverse radix
-  constexpr int NSL = N / RL;               // its stride in both directions
-  constexpr int B1 = sk_bpt<N, R1>(), BL = sk_bpt<N, RL>();
-  static_assert(B1 * R1 * 256 == N, "the first pass's inputs are the loaded points");
-  {
-    float2 v[B1][R1];
-#pragma unroll
-    for (int q = 0; q < B1; ++q)
-#pragma unroll
-      for (int r = 0; r < R1; ++r) v[q][r] = x[q + B1 * r];
-    sk_dft<R1, B1, N, 1>(v, -1.f, tw);
-    sk_write<R1, B1, PAD, N, 1>(buf, v);
-    __syncthreads();
-  }
-  sk_pass<R2, sk_bpt<N, R2>(), PAD, N, R1>(buf, -1.f, tw);
-  if constexpr (R4 > 1) sk_pass<R3, sk_bpt<N, R3>(), PAD, N, R1 * R2>(buf, -1.f, tw);
-  {
-    float2 v[BL][RL];
-    sk_read<RL, BL, PAD, N>(buf, v);
-    sk_dft<RL, BL, N, NSL>(v, -1.f, tw);
-#pragma unroll
-    for (int q = 0; q < BL; ++q) {
-      if (sk_active<N, RL, BL>(q)) {
-        const int j = threadIdx.x + q * 256;
-#pragma unroll
-        for (int r = 0; r < RL; ++r) {
-          const float h = H[j + r * NSL];
-          v[q][r] = make_float2(v[q][r].x * h, v[q][r].y * h);
-        }
-      }
-    }
-    sk_dft<RL, BL, N, 1>(v, 1.f, tw);
-    __syncthreads();  // every thread has read the last forward pass's inputs
-    sk_write<RL, BL, PAD, N, 1>(buf, v);
-    __syncthreads();
-  }
-  if constexpr (R4 > 1) {
-    sk_pass<R3, sk_bpt<N, R3>(), PAD, N, R4>(buf, 1.f, tw);
-    sk_pass<R2, sk_bpt<N, R2>(), PAD, N, R4 * R3>(buf, 1.f, tw);
-  } else {
-    sk_pass<R2, sk_bpt<N, R2>(), PAD, N, R3>(buf, 1.f, tw);
-  }
-  {
-    float2 v[B1][R1];
-    sk_read<R1, B1, PAD, N>(buf, v);
-    sk_dft<R1, B1, N, N / R1>(v, 1.f, tw);
-#pragma unroll
-    for (int q = 0; q < B1; ++q)
-#pragma unroll
-      for (int r = 0; r < R1; ++r) x[q + B1 * r] = v[q][r];
-  }
-}
-
-// Radix plans for N = 2^M, 9 <= M <= 13 (256 threads): the first radix is
-// N / 256 (16 at M = 13, two butterflies per thread), so every thread starts
-// with the points it loaded.  The LDS is padded for M <= 12 (N + N/16 slots; at
-// M = 13 that would pass 64 KiB).
-template <int M>
-constexpr bool sk_pad() {
-  return M <= 12;
-}
-
-template <int M>
-__device__ __forceinline__ void filter_sk(float2* buf, const float2* tw, const float* H,
-                                          float2 (&x)[(1 << M) / 256]) {
-  constexpr bool P = sk_pad<M>();
-  if constexpr (M == 9) sk_filter<2, 16, 16, 1, P>(buf, tw, H, x);
-  else if constexpr (M == 10) sk_filter<4, 16, 16, 1, P>(buf, tw, H, x);
-  else if constexpr (M == 11) sk_filter<8, 16, 16, 1, P>(buf, tw, H, x);
-  else if constexpr (M == 12) sk_filter<16, 16, 16, 1, P>(buf, tw, H, x);
-  else {
-    static_assert(M == 13, "plans cover 2^9 .. 2^13");
-    sk_filter<16, 16, 16, 2, P>(buf, tw, H, x);
-  }
-}
-
 __device__ inline unsigned f2ord(float f) {
   const unsigned u = __float_as_uint(f);
   return (u & 0x80000000u) ? ~u : (u | 0x80000000u);
@@ -467,6 +257,16 @@ __device__ __forceinline__ StoreCtx store_ctx(const FilterArgs& a, int view) {
   return c;
 }
 
+// Widens a view's {min, max} words.  A look at the words first spares most of the
+// atomics, which all waves of a view would queue up for (16 views of 2048^2 into FP16:
+// 1.44 ms with an atomic a wave in the kernel this one replaced); a stale word only
+// costs an atomic that changes nothing.
+__device__ __forceinline__ void minmax_update(unsigned* mm, float lo, float hi) {
+  const unsigned l = f2ord(lo), h = f2ord(hi);
+  if (l < __hip_atomic_load(mm, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMin(mm, l);
+  if (h > __hip_atomic_load(mm + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMax(mm + 1, h);
+}
+
 // Per-view min/max: a wave-level reduction, then one atomic per wave.
 __device__ __forceinline__ void store_minmax(const FilterArgs& a, StoreCtx& c, int view) {
   if (!a.minmax) return;
@@ -475,10 +275,7 @@ __device__ __forceinline__ void store_minmax(const FilterArgs& a, StoreCtx& c, i
     lo = fminf(lo, __shfl_xor(lo, o));
     hi = fmaxf(hi, __shfl_xor(hi, o));
   }
-  if ((threadIdx.x & 63) == 0) {
-    atomicMin(&a.minmax[2 * view], f2ord(lo));
-    atomicMax(&a.minmax[2 * view + 1], f2ord(hi));
-  }
+  if ((threadIdx.x & 63) == 0) minmax_update(a.minmax + 2 * view, lo, hi);
 }
 
 // Stores output sample u of rows ra (fa) and ra+1 (fb) in store mode Q's form
@@ -522,25 +319,8 @@ __device__ __forceinline__ void store_pair(const FilterArgs& a, StoreCtx& c, int
     store_pair_q<kStoreF32, true>(a, c, view, u, ra, has_b, fa, fb);
 }
 
-// A thread's E output points x[i] (point tid + 256 i) cropped, scaled and
-// stored: one loop per store mode, so no per-point mode branches remain.
-template <int Q, bool MM, int E>
-__device__ __forceinline__ void store_points(const FilterArgs& a, int view, int ra, bool has_b,
-                                             int off, const float2 (&x)[E]) {
-  const float inv = 1.0f / (float)a.N;
-  StoreCtx sc = store_ctx(a, view);
-#pragma unroll
-  for (int i = 0; i < E; ++i) {
-    const int u = (int)threadIdx.x + 256 * i - off;
-    if (u >= 0 && u < a.nu) store_pair_q<Q, MM>(a, sc, view, u, ra, has_b, x[i].x * inv, x[i].y * inv);
-  }
-  if constexpr (MM) store_minmax(a, sc, view);
-}
-
-
-// M = log2 N selects the Stockham plan (9..13); M = 0 runs the in-place
-// bit-reversed radix-2^2 FFT for the other lengths.
-template <int M>
+// The other lengths (N < 128), views of 2 GiB and more, and FDK_FILTER_FFT=inplace: the
+// in-place bit-reversed radix-2^2 FFT, a block per row pair.
 __global__ __launch_bounds__(256) void filter_rows_kernel(FilterArgs a) {
   extern __shared__ float2 buf[];
   const int view = blockIdx.y;
@@ -583,75 +363,16 @@ __global__ __launch_bounds__(256) void filter_rows_kernel(FilterArgs a) {
       rrb = (float)(((double)xb[4] + xb[5] + xb[6]) / 3);
     }
   }
-  if constexpr (M != 0) {
-    // Every load of the thread's E points issued before any is used (clamped
-    // addresses, pads selected afterwards), so one memory latency covers them.
-    // Row and cos-table loads go through buffer resources (one 32-bit offset
-    // per point serves all four); a missing cos table is a zero-size resource
-    // whose loads return 0 and are replaced by 1.
-    constexpr int E = (1 << M) / 256;
-    const float* sbb = has_b ? sb : sa;
-    const float* cbb = has_b ? cb : ca;
-    const int row_bytes = nu * 4;
-    const __amdgpu_buffer_rsrc_t rxa = __builtin_amdgcn_make_buffer_rsrc((void*)sa, 0, row_bytes, fdk::kRawRsrcWord3);
-    const __amdgpu_buffer_rsrc_t rxb = __builtin_amdgcn_make_buffer_rsrc((void*)sbb, 0, row_bytes, fdk::kRawRsrcWord3);
-    const __amdgpu_buffer_rsrc_t rwa =
-        __builtin_amdgcn_make_buffer_rsrc((void*)ca, 0, ca ? row_bytes : 0, fdk::kRawRsrcWord3);
-    const __amdgpu_buffer_rsrc_t rwb =
-        __builtin_amdgcn_make_buffer_rsrc((void*)cbb, 0, cbb ? row_bytes : 0, fdk::kRawRsrcWord3);
-    float xa[E], xb[E], wa[E], wb[E];
-#pragma unroll
-    for (int i = 0; i < E; ++i) {
-      const unsigned po = (unsigned)min(max((int)threadIdx.x + 256 * i - off, 0), nu - 1) * 4u;
-      xa[i] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rxa, po, 0, 0));
-      xb[i] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rxb, po, 0, 0));
-      wa[i] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rwa, po, 0, 0));
-      wb[i] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rwb, po, 0, 0));
+  for (int n = threadIdx.x; n < a.N; n += blockDim.x) {
+    const int p = n - off;
+    float va, vb;
+    if (p < 0) { va = la; vb = lb; }
+    else if (p >= nu) { va = rra; vb = rrb; }
+    else {
+      va = sa[p] * (ca ? ca[p] : 1.f);
+      vb = has_b ? sb[p] * (cb ? cb[p] : 1.f) : 0.f;
     }
-    if (!ca) {
-#pragma unroll
-      for (int i = 0; i < E; ++i) wa[i] = wb[i] = 1.f;
-    }
-    float2 x[E];
-#pragma unroll
-    for (int i = 0; i < E; ++i) {
-      const int n = threadIdx.x + 256 * i;
-      const int p = n - off;
-      float va = xa[i] * wa[i], vb = has_b ? xb[i] * wb[i] : 0.f;
-      if (p < 0) {
-        va = la;
-        vb = lb;
-      } else if (p >= nu) {
-        va = rra;
-        vb = rrb;
-      }
-      x[i] = make_float2(va, vb);
-    }
-    filter_sk<M>(buf, a.tw, a.H, x);
-    // x[i] is now output point tid + 256 i: crop, scale and store it
-    if (a.qmode == kStoreNone)
-      store_points<kStoreNone, true>(a, view, ra, has_b, off, x);
-    else if (a.qmode == kStoreF16)
-      store_points<kStoreF16, false>(a, view, ra, has_b, off, x);
-    else if (a.qmode == kStoreBF16)
-      store_points<kStoreBF16, false>(a, view, ra, has_b, off, x);
-    else if (a.minmax)
-      store_points<kStoreF32, true>(a, view, ra, has_b, off, x);
-    else
-      store_points<kStoreF32, false>(a, view, ra, has_b, off, x);
-    return;
-  } else {
-    for (int n = threadIdx.x; n < a.N; n += blockDim.x) {
-      const int p = n - off;
-      float va, vb;
-      if (p < 0) { va = la; vb = lb; }
-      else if (p >= nu) { va = rra; vb = rrb; }
-      else {
-        va = sa[p] * (ca ? ca[p] : 1.f);
-        vb = has_b ? sb[p] * (cb ? cb[p] : 1.f) : 0.f;
-      }
-      buf[brev_n(n, a.logN)] = make_float2(va, vb);
-    }
+    buf[brev_n(n, a.logN)] = make_float2(va, vb);
   }
   __syncthreads();
   {
@@ -679,6 +400,534 @@ __global__ __launch_bounds__(256) void filter_rows_kernel(FilterArgs a) {
     store_pair(a, sc, view, u, ra, has_b, c.x * inv, c.y * inv);
   }
   store_minmax(a, sc, view);
+}
+
+// ------------------------------------------------------------ row filter, 16 points a thread
+// filter_wide_kernel: T = N / 16 threads hold a row pair, 16 points each: point
+// t + T i of thread t, i < 16.  Radices 16, 16, then N / 256 as one or two passes (16
+// and 8 at N = 128).  In every pass a thread's inputs are its points t + T i, so
+//  * forward, a pass reads them, twiddles, transforms and writes the self-sorted order;
+//  * the inverse is the forward passes' adjoint in reverse order: read what the pass
+//    wrote, conjugate transform, conjugate twiddles, write to t + T i.  It needs the
+//    same twiddles in the same threads, and the last pass's outputs, the filter
+//    multiply and the first adjoint's inputs are the same registers, as are the points
+//    loaded and the points stored.
+// A block keeps to its rows' place and walks over many pairs, so what depends on the
+// thread alone is loaded once: H / N and the third and fourth pass's twiddles in
+// registers, the second pass's 16 x 15 in LDS.  QUAD: two pairs in lockstep (half the
+// barriers, twice the independent work), their transposed outputs one 16-byte store a
+// point.  An XCD takes an eighth of the rows (32 at least) of one view, then of the next:
+// the cos-table rows stay in its L2, and the stores of neighbouring rows meet there as
+// lines.
+//
+// What bounds it: at 200 registers and 2 waves per SIMD vector issue is half the time
+// (330 us of 600 at the size below), the rest LDS exchanges, barriers and the transposed
+// stores (60 us; 220 us as 8-byte stores of a pair).  The form it replaces (256 threads a
+// pair whatever N, twiddles and H loaded for every pair) kept the texture-address unit
+// busy 90 % of the time: 60 strided twiddle loads, 64 row and cos loads of which half are
+// pads, 32 loads of edge samples and 8 scattered stores a thread.  Measured, 32 views of
+// 2048^2 transposed: 916 -> 598 us (row-major 765 -> 540); 32 of 1000^2 241 -> 90; 8 of
+// 4096^2 into FP16 1900 -> 1025; 4 of 300^2 11.0 -> 12.5 (the only loss seen:
+// too few rows to fill the chip at 16 points a thread); one of 9000^2 (was in place)
+// 2425 -> 782.
+typedef unsigned u32x2_t __attribute__((ext_vector_type(2)));
+typedef unsigned u32x4_t __attribute__((ext_vector_type(4)));
+typedef unsigned u32x2_t __attribute__((ext_vector_type(2)));
+typedef unsigned u32x4_t __attribute__((ext_vector_type(4)));
+
+template <int M>
+struct Wide {
+  static constexpr int N = 1 << M, T = N / 16;
+  static constexpr int THREADS = T > 256 ? T : 256, PB = THREADS / T;  // row pairs per block
+  static constexpr int R2 = M == 7 ? 8 : 16;
+  static constexpr int R3 = M <= 8 ? 1 : M >= 12 ? 16 : N / 256;
+  static constexpr int R4 = M >= 13 ? N / 4096 : 1;
+  static constexpr int SLOTS = N + N / 16;  // LDS points of a pair, one spare per 16
+  static constexpr int TW2 = (R2 - 1) * 16;
+  static constexpr size_t lds(bool quad) {
+    return sizeof(float2) * ((quad ? 2 : 1) * PB * SLOTS + TW2);
+  }
+};
+
+// Twiddles e^{-2 pi i k r / (NS R)} of a thread's 16 / R butterflies, r = 1 .. R-1.
+template <int M, int R, int NS>
+struct WideTw {
+  static constexpr int B = 16 / R;
+  float2 w[R > 1 ? B * (R - 1) : 1];
+  __device__ __forceinline__ void load(const float2* __restrict__ tw, int t) {
+    if constexpr (R > 1) {
+#pragma unroll
+      for (int q = 0; q < B; ++q) {
+        const int k = (t + q * Wide<M>::T) & (NS - 1);
+#pragma unroll
+        for (int r = 1; r < R; ++r) w[q * (R - 1) + r - 1] = tw[k * r * (Wide<M>::N / (NS * R))];
+      }
+    }
+  }
+};
+
+__device__ __forceinline__ float2 cmul_conj(float2 a, float2 w) {  // a * conj(w)
+  return make_float2(a.x * w.x + a.y * w.y, a.y * w.x - a.x * w.y);
+}
+
+// The radix-R DFTs of a thread's points x[q + B r].
+template <int R, bool INV>
+__device__ __forceinline__ void wide_dft(float2 (&x)[16]) {
+  constexpr int B = 16 / R;
+#pragma unroll
+  for (int q = 0; q < B; ++q) {
+    float2 v[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) v[r] = x[q + B * r];
+    dft<R>(v, INV ? 1.f : -1.f);
+#pragma unroll
+    for (int r = 0; r < R; ++r) x[q + B * r] = v[r];
+  }
+}
+
+// LDS slot of point t + T i, and of output r of butterfly j = t + T q of a pass.
+template <int M>
+__device__ __forceinline__ int wide_own(int t, int i) {
+  constexpr int T = Wide<M>::T;
+  return T % 16 == 0 ? t + (t >> 4) + i * (T + T / 16) : (t + T * i) + ((t + T * i) >> 4);
+}
+template <int M, int R, int NS>
+__device__ __forceinline__ int wide_out(int t, int q, int r) {
+  const int j = t + Wide<M>::T * q, k = j & (NS - 1), o = (j - k) * R + k;
+  if constexpr (NS == 1) return o + (o >> 4) + r;  // R = 16: one 16-point run
+  else if constexpr (NS % 16 == 0) return o + (o >> 4) + r * (NS + NS / 16);
+  else return (o + r * NS) + ((o + r * NS) >> 4);
+}
+
+template <int M, int R, int NS>
+__device__ __forceinline__ void wide_put(float2* buf, const float2 (&x)[16], int t) {
+  constexpr int B = 16 / R;
+#pragma unroll
+  for (int q = 0; q < B; ++q)
+#pragma unroll
+    for (int r = 0; r < R; ++r) buf[wide_out<M, R, NS>(t, q, r)] = x[q + B * r];
+}
+template <int M, int R, int NS>
+__device__ __forceinline__ void wide_get(const float2* buf, float2 (&x)[16], int t) {
+  constexpr int B = 16 / R;
+#pragma unroll
+  for (int q = 0; q < B; ++q)
+#pragma unroll
+    for (int r = 0; r < R; ++r) x[q + B * r] = buf[wide_out<M, R, NS>(t, q, r)];
+}
+template <int M>
+__device__ __forceinline__ void wide_put_own(float2* buf, const float2 (&x)[16], int t) {
+#pragma unroll
+  for (int i = 0; i < 16; ++i) buf[wide_own<M>(t, i)] = x[i];
+}
+template <int M>
+__device__ __forceinline__ void wide_get_own(const float2* buf, float2 (&x)[16], int t) {
+#pragma unroll
+  for (int i = 0; i < 16; ++i) x[i] = buf[wide_own<M>(t, i)];
+}
+
+template <int R, bool INV>
+__device__ __forceinline__ void wide_twiddle(float2 (&x)[16], const float2* w) {
+  constexpr int B = 16 / R;
+#pragma unroll
+  for (int q = 0; q < B; ++q)
+#pragma unroll
+    for (int r = 1; r < R; ++r) {
+      const float2 f = w[q * (R - 1) + r - 1];
+      x[q + B * r] = INV ? cmul_conj(x[q + B * r], f) : cmul(x[q + B * r], f);
+    }
+}
+
+// The second pass's twiddles from LDS: tw2[(r - 1) 16 + k].
+template <int M, bool INV>
+__device__ __forceinline__ void wide_twiddle2(float2 (&x)[16], const float2* tw2, int t) {
+  constexpr int R = Wide<M>::R2, B = 16 / R;
+#pragma unroll
+  for (int q = 0; q < B; ++q) {
+    const int k = (t + q * Wide<M>::T) & 15;
+#pragma unroll
+    for (int r = 1; r < R; ++r) {
+      const float2 f = tw2[(r - 1) * 16 + k];
+      x[q + B * r] = INV ? cmul_conj(x[q + B * r], f) : cmul(x[q + B * r], f);
+    }
+  }
+}
+
+// Lane k of the thread's group of min(T, 64) lanes.
+template <int T>
+__device__ __forceinline__ float wide_lane(float v, int k) {
+  if constexpr (T >= 64) return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), k));
+  else return __shfl(v, k, T);
+}
+
+// The 16 points of a pair's rows (t + T i: sample t + T i - off), cos-weighted, the
+// points left and right of the row set to the pads.  Loads past a resource's end read
+// 0, so no address is clamped; slices that hold no sample are not loaded.
+template <int M>
+__device__ __forceinline__ void wide_load(const FilterArgs& a, const float* sa, const float* sb,
+                                          const float* ca, bool live, bool has_b, int t, int off,
+                                          float2 (&x)[16]) {
+  constexpr int T = Wide<M>::T;
+  const int nu = a.nu, row_bytes = nu * 4;
+  float la = 0.f, lb = 0.f, ra = 0.f, rb = 0.f;
+  const int kpad = a.pad;
+  if constexpr (T >= 64) {
+    const int na = live ? row_bytes : 0, nb = has_b ? row_bytes : 0;
+    const __amdgpu_buffer_rsrc_t rxa = __builtin_amdgcn_make_buffer_rsrc((void*)sa, 0, na, fdk::kRawRsrcWord3);
+    const __amdgpu_buffer_rsrc_t rxb = __builtin_amdgcn_make_buffer_rsrc((void*)sb, 0, nb, fdk::kRawRsrcWord3);
+    const __amdgpu_buffer_rsrc_t rca = __builtin_amdgcn_make_buffer_rsrc((void*)ca, 0, ca ? na : 0, fdk::kRawRsrcWord3);
+    const __amdgpu_buffer_rsrc_t rcb =
+        __builtin_amdgcn_make_buffer_rsrc((void*)(ca + nu), 0, ca ? nb : 0, fdk::kRawRsrcWord3);
+    const auto ld = [](__amdgpu_buffer_rsrc_t r, int o) {
+      return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, o, 0, 0));
+    };
+    float ea = 0.f, eb = 0.f;  // lanes 0..3: samples 0..3, lanes 4..7: nu-1 .. nu-4
+    if (kpad) {
+      const int l = threadIdx.x & 7, e = (l < 4 ? l : nu + 3 - l) * 4;
+      ea = ld(rxa, e);
+      eb = ld(rxb, e);
+      if (ca) {
+        ea *= ld(rca, e);
+        eb *= ld(rcb, e);
+      }
+    }
+#pragma unroll
+    for (int c = 0; c < 16; c += 8) {  // 8 slices in flight
+      float xa[8], xb[8], wa[8], wb[8];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const int lo = T * (c + i) - off;
+        xa[i] = xb[i] = 0.f;
+        wa[i] = wb[i] = 1.f;
+        if (lo + T > 0 && lo < nu) {
+          xa[i] = ld(rxa, (t + lo) * 4);
+          xb[i] = ld(rxb, (t + lo) * 4);
+          if (ca) {
+            wa[i] = ld(rca, (t + lo) * 4);
+            wb[i] = ld(rcb, (t + lo) * 4);
+          }
+        }
+      }
+#pragma unroll
+      for (int i = 0; i < 8; ++i) x[c + i] = make_float2(xa[i] * wa[i], xb[i] * wb[i]);
+    }
+    if (kpad == 0) return;
+    const auto la_of = [&](float v, int k) { return wide_lane<64>(v, k); };
+    if (kpad == 4) {
+      la = (la_of(ea, 0) + la_of(ea, 1) + la_of(ea, 2) + la_of(ea, 3)) / 4;
+      ra = (la_of(ea, 4) + la_of(ea, 5) + la_of(ea, 6) + la_of(ea, 7)) / 4;
+      lb = (la_of(eb, 0) + la_of(eb, 1) + la_of(eb, 2) + la_of(eb, 3)) / 4;
+      rb = (la_of(eb, 4) + la_of(eb, 5) + la_of(eb, 6) + la_of(eb, 7)) / 4;
+    } else {
+      la = (float)(((double)la_of(ea, 0) + la_of(ea, 1) + la_of(ea, 2)) / 3);
+      ra = (float)(((double)la_of(ea, 4) + la_of(ea, 5) + la_of(ea, 6)) / 3);
+      lb = (float)(((double)la_of(eb, 0) + la_of(eb, 1) + la_of(eb, 2)) / 3);
+      rb = (float)(((double)la_of(eb, 4) + la_of(eb, 5) + la_of(eb, 6)) / 3);
+    }
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      const int lo = T * i - off;
+      if (lo < 0 || lo + T > nu) {
+        if (t + lo < 0) x[i] = make_float2(la, lb);
+        else if (t + lo >= nu) x[i] = make_float2(ra, rb);
+      }
+    }
+  } else {
+    // several pairs in a wave
+    const auto at = [&](const float* s, const float* c, bool ok, int p) {
+      return ok ? s[p] * (c ? c[p] : 1.f) : 0.f;
+    };
+    const float* cb = ca ? ca + nu : nullptr;
+    float ea[8], eb[8];
+    if (kpad) {
+#pragma unroll
+      for (int l = 0; l < 8; ++l) {
+        const int e = l < 4 ? l : nu + 3 - l;
+        ea[l] = at(sa, ca, live, e);
+        eb[l] = at(sb, cb, has_b, e);
+      }
+      if (kpad == 4) {
+        la = (ea[0] + ea[1] + ea[2] + ea[3]) / 4;
+        ra = (ea[4] + ea[5] + ea[6] + ea[7]) / 4;
+        lb = (eb[0] + eb[1] + eb[2] + eb[3]) / 4;
+        rb = (eb[4] + eb[5] + eb[6] + eb[7]) / 4;
+      } else {
+        la = (float)(((double)ea[0] + ea[1] + ea[2]) / 3);
+        ra = (float)(((double)ea[4] + ea[5] + ea[6]) / 3);
+        lb = (float)(((double)eb[0] + eb[1] + eb[2]) / 3);
+        rb = (float)(((double)eb[4] + eb[5] + eb[6]) / 3);
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      const int p = t + T * i - off;
+      x[i] = p < 0 ? make_float2(la, lb)
+             : p >= nu ? make_float2(ra, rb)
+                       : make_float2(at(sa, ca, live, p), at(sb, cb, has_b, p));
+    }
+  }
+}
+
+// Min/max of the lanes of one pair (all of a wave, or groups of T lanes).
+template <int T>
+__device__ __forceinline__ void wide_minmax(const FilterArgs& a, StoreCtx& c, int view, int t) {
+  constexpr int L = T < 64 ? T : 64;
+  float lo = c.lo, hi = c.hi;
+#pragma unroll
+  for (int o = L / 2; o > 0; o >>= 1) {
+    lo = fminf(lo, __shfl_xor(lo, o, L));
+    hi = fmaxf(hi, __shfl_xor(hi, o, L));
+  }
+  if ((t & (L - 1)) == 0) minmax_update(a.minmax + 2 * view, lo, hi);
+}
+
+// Stores the 16 points, cropped.  FP32 goes through a resource of the view (transposed)
+// or the row: points outside the row fall outside it and are dropped.
+template <int M, int Q, bool MM>
+__device__ __forceinline__ void wide_store(const FilterArgs& a, int view, int ra, bool live, bool has_b,
+                                           int t, int off, const float2 (&x)[16]) {
+  constexpr int T = Wide<M>::T;
+  StoreCtx c = store_ctx(a, view);
+  if constexpr (Q == kStoreF32 && T >= 64) {
+    float* d = a.dst + view * a.dst_view;
+    if (a.transpose) {
+      const __amdgpu_buffer_rsrc_t rd = __builtin_amdgcn_make_buffer_rsrc(
+          (void*)d, 0, live ? a.nu * a.nrows * 4 : 0, fdk::kRawRsrcWord3);
+      const int o0 = (int)(((unsigned)(t - off) * a.nrows + ra) * 4u);  // wraps outside the row
+      const bool both = has_b && (a.nrows & 1) == 0;
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        const int lo = T * i - off;
+        if (lo + T <= 0 || lo >= a.nu) continue;
+        const int o = (int)((unsigned)o0 + (unsigned)(i * T * 4) * a.nrows);
+        if (both) {
+          __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2_t, x[i]), rd, o, 0, 0);
+        } else {
+          __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(x[i].x), rd, o, 0, 0);
+          // (t + lo >= 0: the row above must not take a value for the one below)
+          if (has_b && t + lo >= 0 && t + lo < a.nu)
+            __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(x[i].y), rd, o + 4, 0, 0);
+        }
+      }
+    } else {
+      float* row = d + (long long)ra * a.dst_pitch;
+      const __amdgpu_buffer_rsrc_t rda =
+          __builtin_amdgcn_make_buffer_rsrc((void*)row, 0, live ? a.nu * 4 : 0, fdk::kRawRsrcWord3);
+      const __amdgpu_buffer_rsrc_t rdb = __builtin_amdgcn_make_buffer_rsrc(
+          (void*)(row + a.dst_pitch), 0, has_b ? a.nu * 4 : 0, fdk::kRawRsrcWord3);
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        const int lo = T * i - off;
+        if (lo + T <= 0 || lo >= a.nu) continue;
+        __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(x[i].x), rda, (t + lo) * 4, 0, 0);
+        __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(x[i].y), rdb, (t + lo) * 4, 0, 0);
+      }
+    }
+    if constexpr (MM) {
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        const int u = t + T * i - off;
+        if (live && u >= 0 && u < a.nu) {
+          c.lo = fminf(c.lo, has_b ? fminf(x[i].x, x[i].y) : x[i].x);
+          c.hi = fmaxf(c.hi, has_b ? fmaxf(x[i].x, x[i].y) : x[i].x);
+        }
+      }
+    }
+  } else {
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      const int u = t + T * i - off;
+      if (live && u >= 0 && u < a.nu) store_pair_q<Q, MM>(a, c, view, u, ra, has_b, x[i].x, x[i].y);
+    }
+  }
+  if constexpr (MM)
+    if (live) wide_minmax<T>(a, c, view, t);
+}
+
+// The outputs of rows ra, ra+1 (w) and ra+2, ra+3 (x), transposed: one 16-byte store a
+// point.
+template <int M, bool MM>
+__device__ __forceinline__ void wide_store4(const FilterArgs& a, int view, int ra, bool live, int t, int off,
+                                            const float2 (&w)[16], const float2 (&x)[16]) {
+  constexpr int T = Wide<M>::T;
+  const int left = live ? a.nrows - ra : 0;  // rows of the four that exist
+  if (left <= 0) return;
+  float* d = a.dst + view * a.dst_view + ra;
+  const int bytes = a.nu * a.nrows * 4 - ra * 4;
+  StoreCtx c = store_ctx(a, view);
+  const unsigned o0 = (unsigned)(t - off) * a.nrows * 4u;  // wraps outside the row
+#pragma unroll
+  for (int i = 0; i < 16; ++i) {
+    const int lo = T * i - off;
+    if (lo + T <= 0 || lo >= a.nu) continue;
+    const float2 y = w[i];
+    const int o = (int)(o0 + (unsigned)(i * T * 4) * a.nrows);
+    const bool in = t + lo >= 0 && t + lo < a.nu;
+    if constexpr (T >= 64) {
+      const __amdgpu_buffer_rsrc_t rd = __builtin_amdgcn_make_buffer_rsrc((void*)d, 0, bytes, fdk::kRawRsrcWord3);
+      if (left >= 4) {  // outside the row the offset is negative or past the view: dropped
+        const u32x4_t v = {__float_as_uint(y.x), __float_as_uint(y.y), __float_as_uint(x[i].x),
+                           __float_as_uint(x[i].y)};
+        __builtin_amdgcn_raw_buffer_store_b128(v, rd, o, 0, 0);
+      } else if (in) {
+        __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(y.x), rd, o, 0, 0);
+        if (left > 1) __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(y.y), rd, o + 4, 0, 0);
+        if (left > 2) __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(x[i].x), rd, o + 8, 0, 0);
+      }
+    } else if (in) {
+      float* q = d + (long long)(t + lo) * a.nrows;
+      if (left >= 4) {
+        typedef float f32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));
+        *reinterpret_cast<f32x4_a4*>(q) = f32x4_a4{y.x, y.y, x[i].x, x[i].y};
+      } else {
+        q[0] = y.x;
+        if (left > 1) q[1] = y.y;
+        if (left > 2) q[2] = x[i].x;
+      }
+    }
+    if (MM && in) {
+      c.lo = fminf(c.lo, y.x);
+      c.hi = fmaxf(c.hi, y.x);
+      if (left > 1) c.lo = fminf(c.lo, y.y), c.hi = fmaxf(c.hi, y.y);
+      if (left > 2) c.lo = fminf(c.lo, x[i].x), c.hi = fmaxf(c.hi, x[i].x);
+      if (left > 3) c.lo = fminf(c.lo, x[i].y), c.hi = fmaxf(c.hi, x[i].y);
+    }
+  }
+  if constexpr (MM) wide_minmax<T>(a, c, view, t);
+}
+
+struct WideGrid {
+  int items, chunk;  // row quads in all (the last group padded), quads of one XCD
+  int nviews, group;
+};
+
+template <int M, bool QUAD>
+__global__ __launch_bounds__(Wide<M>::THREADS, (M == 14 ? 4 : 2)) void filter_wide_kernel(FilterArgs a, WideGrid g) {
+  using W = Wide<M>;
+  constexpr int N = W::N, T = W::T, R2 = W::R2, R3 = W::R3, R4 = W::R4;
+  constexpr int P = QUAD ? 2 : 1, ROWS = 2 * P;  // row pairs and rows of an item
+  extern __shared__ float2 wide_lds[];
+  const int t = threadIdx.x & (T - 1);
+  const int sub = T >= 64 ? __builtin_amdgcn_readfirstlane(threadIdx.x / T) : (int)threadIdx.x / T;
+  float2* tw2 = wide_lds;
+  float2* buf[P];
+#pragma unroll
+  for (int p = 0; p < P; ++p) buf[p] = wide_lds + W::TW2 + (sub * P + p) * W::SLOTS;
+  for (int k = threadIdx.x; k < W::TW2; k += W::THREADS)
+    tw2[k] = a.tw[(k & 15) * (k / 16 + 1) * (N / (16 * R2))];
+  WideTw<M, R3, 256> tw3;
+  tw3.load(a.tw, t);
+  WideTw<M, R4, 4096> tw4;
+  tw4.load(a.tw, t);
+  float h[16];
+#pragma unroll
+  for (int i = 0; i < 16; ++i) h[i] = a.H[t + T * i] * (1.0f / N);  // exact: N is a power of two
+  const int off = (N - a.nu) >> 1;
+  const int nsets = (a.nrows + ROWS - 1) / ROWS, per_group = g.nviews * g.group;
+  // (the first barrier below also covers tw2)
+
+  // XCD x (block % 8) walks items [x chunk, (x + 1) chunk)
+  const int xcd = blockIdx.x % 8u, stride = (int)(gridDim.x / 8u) * W::PB;
+  const int end = min(g.items, (xcd + 1) * g.chunk);
+  for (int it0 = xcd * g.chunk + (int)(blockIdx.x / 8u) * W::PB; it0 < end; it0 += stride) {
+    const int it = it0 + sub;
+    const int grp = it / per_group, in = it - grp * per_group;
+    const int set = grp * g.group + in % g.group;
+    const bool live = it < end && set < nsets;  // others only take part in the barriers
+    const int view = live ? in / g.group : 0, ra = live ? ROWS * set : 0;
+    float2 x[P][16];
+#define WIDE_EACH _Pragma("unroll") for (int p = 0; p < P; ++p)
+    WIDE_EACH {
+      const int r = ra + 2 * p;
+      const bool has_a = live && r < a.nrows, has_b = live && r + 1 < a.nrows;
+      const float* sa = a.src + view * a.src_view + (long long)r * a.src_pitch;
+      wide_load<M>(a, sa, sa + a.src_pitch, a.cos_table ? a.cos_table + (long long)r * a.nu : nullptr,
+                   has_a, has_b, t, off, x[p]);
+    }
+    WIDE_EACH {
+      wide_dft<16, false>(x[p]);
+      wide_put<M, 16, 1>(buf[p], x[p], t);
+    }
+    __syncthreads();
+    WIDE_EACH {
+      wide_get_own<M>(buf[p], x[p], t);
+      wide_twiddle2<M, false>(x[p], tw2, t);
+      wide_dft<R2, false>(x[p]);
+    }
+    if constexpr (R3 > 1) {
+      __syncthreads();
+      WIDE_EACH wide_put<M, R2, 16>(buf[p], x[p], t);
+      __syncthreads();
+      WIDE_EACH {
+        wide_get_own<M>(buf[p], x[p], t);
+        wide_twiddle<R3, false>(x[p], tw3.w);
+        wide_dft<R3, false>(x[p]);
+        }
+    }
+    if constexpr (R4 > 1) {
+      __syncthreads();
+      WIDE_EACH wide_put<M, R3, 256>(buf[p], x[p], t);
+      __syncthreads();
+      WIDE_EACH {
+        wide_get_own<M>(buf[p], x[p], t);
+        wide_twiddle<R4, false>(x[p], tw4.w);
+        wide_dft<R4, false>(x[p]);
+      }
+    }
+    // The filter, then the adjoints; a thread writes only the points it alone has read
+    // last, so the first needs no barrier before its writes.
+    WIDE_EACH {
+#pragma unroll
+      for (int i = 0; i < 16; ++i) x[p][i] = make_float2(x[p][i].x * h[i], x[p][i].y * h[i]);
+    }
+    if constexpr (R4 > 1) {
+      WIDE_EACH {
+        wide_dft<R4, true>(x[p]);
+        wide_twiddle<R4, true>(x[p], tw4.w);
+        wide_put_own<M>(buf[p], x[p], t);
+      }
+      __syncthreads();
+      WIDE_EACH wide_get<M, R3, 256>(buf[p], x[p], t);
+      __syncthreads();
+    }
+    if constexpr (R3 > 1) {
+      WIDE_EACH {
+        wide_dft<R3, true>(x[p]);
+        wide_twiddle<R3, true>(x[p], tw3.w);
+        wide_put_own<M>(buf[p], x[p], t);
+        }
+      __syncthreads();
+      WIDE_EACH wide_get<M, R2, 16>(buf[p], x[p], t);
+      __syncthreads();
+    }
+    WIDE_EACH {
+      wide_dft<R2, true>(x[p]);
+      wide_twiddle2<M, true>(x[p], tw2, t);
+      wide_put_own<M>(buf[p], x[p], t);
+    }
+    __syncthreads();
+    WIDE_EACH {
+      wide_get<M, 16, 1>(buf[p], x[p], t);
+      wide_dft<16, true>(x[p]);
+    }
+#undef WIDE_EACH
+    const bool has_b = live && ra + 1 < a.nrows;
+    if constexpr (QUAD) {
+      if (a.minmax) wide_store4<M, true>(a, view, ra, live, t, off, x[0], x[1]);
+      else wide_store4<M, false>(a, view, ra, live, t, off, x[0], x[1]);
+    } else if (a.qmode == kStoreNone) {
+      wide_store<M, kStoreNone, true>(a, view, ra, live, has_b, t, off, x[0]);
+    } else if (a.qmode == kStoreF16) {
+      wide_store<M, kStoreF16, false>(a, view, ra, live, has_b, t, off, x[0]);
+    } else if (a.qmode == kStoreBF16) {
+      wide_store<M, kStoreBF16, false>(a, view, ra, live, has_b, t, off, x[0]);
+    } else if (a.minmax) {
+      wide_store<M, kStoreF32, true>(a, view, ra, live, has_b, t, off, x[0]);
+    } else {
+      wide_store<M, kStoreF32, false>(a, view, ra, live, has_b, t, off, x[0]);
+    }
+    __syncthreads();  // the last reads are done
+  }
 }
 
 // FP32 staging -> FP16/BF16 with q = (p - min) / (max - min) per view, four
@@ -727,8 +976,7 @@ __global__ void correct_kernel(const float* __restrict__ src, const float* __res
   dst[o] = src[o] * table[(long long)y * tpitch + x];
 }
 
-// Twiddles e^{-2 pi i k / N}, k < N (the Stockham passes index the whole
-// circle), evaluated in FP64 and rounded to float.
+// Twiddles e^{-2 pi i k / N}, k < N, evaluated in FP64 and rounded to float.
 __global__ void twiddle_kernel(float2* tw, int N) {
   const int k = blockIdx.x * blockDim.x + threadIdx.x;
   if (k < N) {
@@ -785,14 +1033,51 @@ int log2_exact(int N) {
   return (1 << m) == N ? m : -1;
 }
 
-// 1: Stockham FFT where a plan exists (default); FDK_FILTER_FFT=inplace keeps
-// the in-place radix-2^2 FFT for every length.
+// 1: filter_wide_kernel where it applies (default); FDK_FILTER_FFT=inplace keeps the
+// in-place radix-2^2 FFT for every length.
 int fft_choice() {
   static const int k = [] {
     const char* e = std::getenv("FDK_FILTER_FFT");
     return (e && std::strcmp(e, "inplace") == 0) ? 0 : 1;
   }();
   return k;
+}
+
+// Blocks per CU that the LDS and the registers (2 waves per SIMD; 4 at M = 14, whose
+// block has 16 waves) allow.
+template <int M>
+constexpr int wide_resident() { return M <= 12 ? 2 : 1; }
+
+template <int M, bool QUAD>
+int launch_wide_sets(const FilterArgs& a, int nviews, hipStream_t st) {
+  using W = Wide<M>;
+  constexpr int ROWS = QUAD ? 4 : 2;
+  const int nsets = (a.nrows + ROWS - 1) / ROWS;
+  const int group = std::max(32 / ROWS, (nsets + 7) / 8);  // 32 rows fill a 128-byte line
+  const long long items = (long long)((nsets + group - 1) / group) * group * nviews;
+  const long long chunk = ((items + 7) / 8 + W::PB - 1) / W::PB * W::PB;
+  const long long per_xcd = std::min<long long>(chunk / W::PB, 32 * wide_resident<M>());
+  const WideGrid g{(int)items, (int)chunk, nviews, group};
+  const void* fn = reinterpret_cast<const void*>(&filter_wide_kernel<M, QUAD>);
+  const size_t lds = W::lds(QUAD);
+  if (lds > 64 * 1024) FDK_HIP(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+  hipLaunchKernelGGL((filter_wide_kernel<M, QUAD>), dim3((unsigned)(8 * per_xcd)), dim3(W::THREADS), lds, st, a, g);
+  FDK_HIP(hipGetLastError());
+  return FDK_OK;
+}
+
+template <int M>
+int launch_wide(const FilterArgs& a, int nviews, hipStream_t st) {
+  const long long waves = (long long)((a.nrows + 1) / 2) * nviews * Wide<M>::T / 64;
+  if constexpr (M <= 13)
+    if (a.transpose && a.qmode == kStoreF32 && waves >= 4096) return launch_wide_sets<M, true>(a, nviews, st);
+  return launch_wide_sets<M, false>(a, nviews, st);
+}
+
+// 32-bit offsets in a row and a view, and pair counts that fit the kernel's ints.
+bool wide_ok(const FilterArgs& a, int nviews) {
+  return a.logN >= 7 && a.logN <= 14 && (long long)a.nu * a.nrows * 4 < (1LL << 31) &&
+         (long long)(a.nrows + 64) * nviews < (1LL << 29);
 }
 
 int launch_filter(FilterArgs& a, int nviews, hipStream_t st) {
@@ -805,17 +1090,20 @@ int launch_filter(FilterArgs& a, int nviews, hipStream_t st) {
   a.logN = log2_exact(a.N);
   if (!a.tw)
     if (int r = twiddles(a.N, &a.tw)) return r;
-  const int plan = (fft_choice() && a.logN >= 9 && a.logN <= 13) ? a.logN : 0;
-  const size_t lds = sizeof(float2) * (plan >= 9 && plan <= 12 ? a.N + a.N / 16 : a.N);
-  dim3 grid((a.nrows + 1) / 2, nviews);
-  switch (plan) {
-    case 9: hipLaunchKernelGGL(filter_rows_kernel<9>, grid, dim3(256), lds, st, a); break;
-    case 10: hipLaunchKernelGGL(filter_rows_kernel<10>, grid, dim3(256), lds, st, a); break;
-    case 11: hipLaunchKernelGGL(filter_rows_kernel<11>, grid, dim3(256), lds, st, a); break;
-    case 12: hipLaunchKernelGGL(filter_rows_kernel<12>, grid, dim3(256), lds, st, a); break;
-    case 13: hipLaunchKernelGGL(filter_rows_kernel<13>, grid, dim3(256), lds, st, a); break;
-    default: hipLaunchKernelGGL(filter_rows_kernel<0>, grid, dim3(256), lds, st, a); break;
+  if (fft_choice() && wide_ok(a, nviews)) {
+    switch (a.logN) {
+      case 7: return launch_wide<7>(a, nviews, st);
+      case 8: return launch_wide<8>(a, nviews, st);
+      case 9: return launch_wide<9>(a, nviews, st);
+      case 10: return launch_wide<10>(a, nviews, st);
+      case 11: return launch_wide<11>(a, nviews, st);
+      case 12: return launch_wide<12>(a, nviews, st);
+      case 13: return launch_wide<13>(a, nviews, st);
+      case 14: return launch_wide<14>(a, nviews, st);
+    }
   }
+  const dim3 grid((a.nrows + 1) / 2, nviews);
+  hipLaunchKernelGGL(filter_rows_kernel, grid, dim3(256), sizeof(float2) * a.N, st, a);
   FDK_HIP(hipGetLastError());
   return FDK_OK;
 }
