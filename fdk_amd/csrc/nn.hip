@@ -479,10 +479,12 @@ __device__ __forceinline__ void fwd5_fetch(HaloRegs<TP, TR>& pre, const Conv& a,
   for (int j = 0; j < kPer; ++j) {
     const int hz = row / kRows, hy = row - hz * kRows, hx = w >> 2;
     bool ok = j + 1 < kPer || t + 256 * j < kChunks;
-    if (!f.interior) {
-      const int zz = f.z0 - 1 + hz, yy = f.y0 - 1 + hy, xx = f.x0 - 1 + hx;
-      ok = ok && zz >= 0 && zz < a.d && yy >= 0 && yy < a.h && xx >= 0 && xx < a.w;
-    }
+    // every tile is checked, interior ones too: without branches the loads
+    // issue back to back (a 96-to-32 decoder convolution on 128 x 256 x 256
+    // voxels 1187 -> 1169 us; a second, unchecked loop for interior tiles 1178)
+    ok &= (unsigned)(f.z0 - 1 + hz) < (unsigned)a.d;
+    ok &= (unsigned)(f.y0 - 1 + hy) < (unsigned)a.h;
+    ok &= (unsigned)(f.x0 - 1 + hx) < (unsigned)a.w;
     // fwd4_fetch's ((h - 1) >> sh) + 1 == (h + sh) >> sh for h >= 0, sh in {0, 1}
     const unsigned off = ((unsigned)((hz + sh) >> sh) * (unsigned)plane +
                           (unsigned)(((hy + sh) >> sh) * rowe + ((hx + sh) >> sh) * cc + 8 * (w & 3))) *
@@ -664,7 +666,7 @@ __device__ __forceinline__ bf16x8 fwd5_read_a(const uint4* hb, int i) {
   return __builtin_bit_cast(bf16x8, hb[(dz * (Q + 2) + yi) * (4 * kHaloX) + 16 * mt + dx]);
 }
 
-template <int NT, int Q, int TP, bool PF>
+template <int NT, int Q, int TP>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void conv3d_fwd5_kernel(
     Conv a, int tiles_x, int tiles_y, int ntiles, int tpb) {
   using HS = HaloShape<TP, Q>;
@@ -672,7 +674,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void c
   const int wave = threadIdx.x / 64, lane = threadIdx.x % 64;
   const int m = lane % 16, kq = lane / 16;
   const int pz = wave % TP;                          // the wave's output plane in the tile
-  const int cw = a.co0 + (wave / TP) * (16 * NT);   // and its first output channel
+  const int cw = a.co0 + 64 * blockIdx.y + (wave / TP) * (16 * NT);  // and its first output channel
   const uint4* hb = halo5 + (pz * HS::rows * 4 + kq) * kHaloX + m;
   const __amdgpu_buffer_rsrc_t wr = __builtin_amdgcn_make_buffer_rsrc(
       (void*)a.wt, 0, (int)(27u * a.cout * a.cin * 2u), fdk::kRawRsrcWord3);
@@ -681,7 +683,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void c
   const int nchunks = a.cin / 32;
   const int first = blockIdx.x * tpb, last = min(first + tpb, ntiles);
   uint4 pre[HS::per];
-  if (PF && first < last) fwd5_fetch<TP, Q>(pre, a, fwd4_tile<TP, Q>(a, first, tiles_x, tiles_y), 0);
+  if (first < last) fwd5_fetch<TP, Q>(pre, a, fwd4_tile<TP, Q>(a, first, tiles_x, tiles_y), 0);
   for (int tile = first; tile < last; ++tile) {
     const Fwd4Tile f = fwd4_tile<TP, Q>(a, tile, tiles_x, tiles_y);
     f32x4 acc[Q][2][NT];
@@ -692,22 +694,19 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void c
 #pragma unroll
         for (int nt = 0; nt < NT; ++nt) acc[q][mt][nt] = f32x4{0.f, 0.f, 0.f, 0.f};
     for (int ch = 0; ch < nchunks; ++ch) {
-      if (!PF) fwd5_fetch<TP, Q>(pre, a, f, ch * 32);
       __syncthreads();  // every wave is done reading the previous halo
       fwd4_commit<TP, Q>(halo5, pre);
       __syncthreads();
       const unsigned cb = (unsigned)ch * 64u;  // 32 channels x 2 bytes
       bf16x8 b[2][3][NT];
       fwd5_load_slice<NT>(b[0], wr, lane_off, cb, nt_bytes, 3u * tap_bytes);
-      if (PF) {
-        int nt_ = tile, nc = ch + 1;
-        if (nc == nchunks) {
-          nc = 0;
-          ++nt_;
-        }
-        if (nt_ < last)
-          fwd5_fetch<TP, Q>(pre, a, nt_ == tile ? f : fwd4_tile<TP, Q>(a, nt_, tiles_x, tiles_y), nc * 32);
+      int nt_ = tile, nc = ch + 1;
+      if (nc == nchunks) {
+        nc = 0;
+        ++nt_;
       }
+      if (nt_ < last)
+        fwd5_fetch<TP, Q>(pre, a, nt_ == tile ? f : fwd4_tile<TP, Q>(a, nt_, tiles_x, tiles_y), nc * 32);
       // steps i = (slice, input row, half): A fragments kAhead steps ahead of
       // their MFMAs, the next slice's weights at the first step of a slice
       constexpr int K = 2 * (Q + 2), kSteps = 9 * K, kAhead = 2;
@@ -1986,14 +1985,20 @@ static bool lean_ok(const Conv& a) {
          27LL * a.cout * a.cin * 2 < (1LL << 31);
 }
 
-template <int TP, bool PF>
-static int launch_fwd5_pass(const Conv& a, hipStream_t st) {
-  const void* fn = reinterpret_cast<const void*>(&conv3d_fwd5_kernel<2, 4, TP, PF>);
+template <int TP>
+static int launch_fwd5_pass(const Conv& a, int passes, hipStream_t st) {
+  const void* fn = reinterpret_cast<const void*>(&conv3d_fwd5_kernel<2, 4, TP>);
   const int lds = HaloShape<TP, 4>::chunks * (int)sizeof(uint4);
   FDK_HIP(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, lds));
   const int tiles_x = a.w / 32, tiles_y = a.h / 4, ntiles = tiles_x * tiles_y * (a.n * a.d / TP);
-  const int tpb = 2;
-  hipLaunchKernelGGL((conv3d_fwd5_kernel<2, 4, TP, PF>), dim3((ntiles + tpb - 1) / tpb), dim3(256), lds,
+  // One tile a block: 512 blocks are resident, so two would leave the chip half
+  // empty below 1024 tiles and its last round longer above (64 -> 64 channels
+  // on 128^3 voxels 511 -> 480 us, on 4 x 8 x 112 x 96 107 -> 98, 32 -> 32 on
+  // 16 x 64 x 96 21.5 -> 12.1).  Two on the 4-plane tiles from 16 rounds on,
+  // where the second tile's loads run under the first (96 -> 32 on 128 x 256 x
+  // 256 1198 -> 1170 us; 3, 4 and 8 no faster).
+  const int tpb = TP == 4 && ntiles >= 8192 ? 2 : 1;
+  hipLaunchKernelGGL((conv3d_fwd5_kernel<2, 4, TP>), dim3((ntiles + tpb - 1) / tpb, passes), dim3(256), lds,
                      st, a, tiles_x, tiles_y, ntiles, tpb);
   FDK_HIP(hipGetLastError());
   return FDK_OK;
@@ -2010,11 +2015,13 @@ static bool fwd5_ok(const Conv& a) {
 }
 
 static int launch_fwd5(const Conv& a, hipStream_t st) {
+  const int passes = a.cout / 64;
+  if (passes > 0)
+    if (int r = launch_fwd5_pass<2>(a, passes, st)) return r;
+  if (a.cout % 64 == 0) return FDK_OK;
   Conv p = a;
-  for (p.co0 = 0; p.co0 + 64 <= a.cout; p.co0 += 64)
-    if (int r = launch_fwd5_pass<2, true>(p, st)) return r;
-  if (p.co0 < a.cout) return launch_fwd5_pass<4, true>(p, st);  // the last 32 channels
-  return FDK_OK;
+  p.co0 = 64 * passes;
+  return launch_fwd5_pass<4>(p, 1, st);  // the last 32 channels
 }
 
 static int launch_fwd4(const Conv& a, hipStream_t st) {

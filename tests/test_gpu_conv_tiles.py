@@ -1,0 +1,48 @@
+"""3x3x3 convolution layers: the work split of the forward kernel, against the
+FP64 restatement."""
+import numpy as np
+import pytest
+
+import fdk_amd.unet as U
+from oracle import nn_ref as R
+
+pytestmark = pytest.mark.gpu
+
+
+def bf(torch, a):
+    return torch.as_tensor(R.to_bf16_bits(a).view(np.int16)).cuda()
+
+
+def rel(a, b):
+    return float(np.linalg.norm(np.ravel(a - b)) / max(np.linalg.norm(np.ravel(b)), 1e-300))
+
+
+@pytest.mark.parametrize("cout", [64, 96, 128, 224])
+def test_forward_passes(torch_cuda, cout):
+    """1, 1, 2 and 3 passes of 64 output channels in one launch, and the 32 that
+    96 and 224 leave."""
+    torch = torch_cuda
+    rng = np.random.default_rng(cout)
+    shape = (1, 4, 8, 64)
+    x = R.bf16_round(rng.standard_normal(shape + (32,)))
+    w = R.bf16_round(rng.standard_normal((27, cout, 32)) / np.sqrt(27 * 32))
+    b = rng.standard_normal(cout).astype(np.float32)
+    y = torch.empty(shape + (cout,), dtype=torch.float32, device="cuda")
+    U.conv3d(bf(torch, x), bf(torch, w), torch.as_tensor(b).cuda(), y, shape, 32, cout, relu=False, out_f32=True)
+    assert rel(y.cpu().numpy(), R.conv3d(x, w, b)) < 1e-5
+
+
+@pytest.mark.parametrize("n", [8191, 8193])
+def test_forward_tiles_per_block(torch_cuda, n):
+    """One tile a block below 8192 tiles and two from there on (an odd count):
+    every sample equals, bit for bit, the same sample computed by itself."""
+    torch = torch_cuda
+    rng = np.random.default_rng(n)
+    s = bf(torch, R.bf16_round(rng.standard_normal((3, 4, 4, 32, 32))))
+    w = bf(torch, R.bf16_round(rng.standard_normal((27, 32, 32)) / np.sqrt(27 * 32)))
+    one = torch.empty((3, 4, 4, 32, 32), dtype=torch.int16, device="cuda")
+    U.conv3d(s, w, None, one, (3, 4, 4, 32), 32, 32, relu=True)
+    k = torch.arange(n, device="cuda") % 3
+    y = torch.empty((n, 4, 4, 32, 32), dtype=torch.int16, device="cuda")
+    U.conv3d(s[k].contiguous(), w, None, y, (n, 4, 4, 32), 32, 32, relu=True)
+    assert torch.equal(y, one[k])
