@@ -2126,8 +2126,16 @@ static bool wgrad_tr_ok(const Wgrad& a) {
 static int launch_wgrad_tr(const Wgrad& a, hipStream_t st) {
   const int tiles_x = a.w / 32, tiles_y = a.h / 4, vt = tiles_x * tiles_y * (a.n * a.d / 2);
   const int chunks = (a.cout / 32) * (a.cin / 32);
-  // about 1024 blocks: every CU busy several times over, few partial sums to add
-  const int gx = std::max(1, std::min(vt, 1024 / chunks));
+  // Every block adds its 27 x 32 x 32 partial sums to dW with atomics, so
+  // fewer, longer blocks cost less of them.  At most the 512 that the CUs hold
+  // (68 KiB of LDS each): 32 -> 32 at 4 x 64 x 64 x 128 takes 132 us, 110
+  // without the atomics, 172 with 1024 blocks, 143 with 256; two rounds where
+  // one would leave a fifth of the chip idle.  On few tiles the atomics (about
+  // 0.05 us a block) grow against the tiles (about 2 us each a CU): their sum
+  // is least at sqrt(40 tiles / chunk pairs) blocks a pair (layer backward, 64
+  // -> 64 at 2 x 16 x 32 x 64: 102 -> 85 us; factors 80, 20, 10: 89, 87, 94).
+  const int one = 512 / chunks, few = (int)std::sqrt(40.0 * vt / chunks);
+  const int gx = std::max(1, std::min({vt, one * chunks >= 410 ? one : 1024 / chunks, few}));
   hipLaunchKernelGGL(conv3d_wgrad_tr_kernel, dim3(gx, chunks), dim3(256), 0, st, a, tiles_x, tiles_y, vt);
   FDK_HIP(hipGetLastError());
   return FDK_OK;

@@ -1,5 +1,5 @@
-"""3x3x3 convolution layers: the work split of the forward kernel, against the
-FP64 restatement."""
+"""3x3x3 convolution layers: the work split of the forward and weight-gradient
+kernels, against the FP64 restatement."""
 import numpy as np
 import pytest
 
@@ -15,6 +15,20 @@ def bf(torch, a):
 
 def rel(a, b):
     return float(np.linalg.norm(np.ravel(a - b)) / max(np.linalg.norm(np.ravel(b)), 1e-300))
+
+
+@pytest.mark.parametrize("cin,cout,n", [(32, 32, 3), (96, 32, 70), (288, 160, 13), (1216, 256, 3)])
+def test_weight_gradient_block_counts(torch_cuda, cin, cout, n):
+    """Weight gradients over 1, 3, 45 and 304 channel chunks, with 3, 30, 3 and 1
+    blocks a chunk: tiles that the blocks do not share evenly, one block for all."""
+    torch = torch_cuda
+    shape = (n, 2, 4, 32)
+    rng = np.random.default_rng(cin)
+    x = R.bf16_round(rng.standard_normal(shape + (cin,)))
+    dy = R.bf16_round(rng.standard_normal(shape + (cout,)))
+    dw = torch.zeros((27, cout, cin), device="cuda")
+    U.conv3d_wgrad(bf(torch, x), bf(torch, dy), dw, shape, cin, cout)
+    assert rel(dw.cpu().numpy(), R.conv3d_dw(x, dy)) < 1e-5
 
 
 @pytest.mark.parametrize("cout", [64, 96, 128, 224])
