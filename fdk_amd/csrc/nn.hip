@@ -1231,18 +1231,20 @@ __global__ void relu_bwd_kernel(const u16* dy, const u16* y, u16* dz, long long 
     dz[i] = relu_bwd1(dy[i], y[i], mode);
 }
 
+__device__ __forceinline__ uint4 relu_bwd8(uint4 g, uint4 v, int mode) {
+  const unsigned gw[4] = {g.x, g.y, g.z, g.w}, vw[4] = {v.x, v.y, v.z, v.w};
+  unsigned o[4];
+#pragma unroll
+  for (int e = 0; e < 4; ++e)
+    o[e] = (unsigned)relu_bwd1((u16)(gw[e] & 0xFFFF), (u16)(vw[e] & 0xFFFF), mode) |
+           ((unsigned)relu_bwd1((u16)(gw[e] >> 16), (u16)(vw[e] >> 16), mode) << 16);
+  return make_uint4(o[0], o[1], o[2], o[3]);
+}
+
 // The same, 8 values per 16-byte vector (n % 8 == 0, 16-byte aligned).
 __global__ void relu_bwd_v8_kernel(const uint4* dy, const uint4* y, uint4* dz, long long n8, int mode) {
-  for (long long i = (long long)blockIdx.x * 256 + threadIdx.x; i < n8; i += (long long)gridDim.x * 256) {
-    const uint4 g = dy[i], v = y[i];
-    const unsigned gw[4] = {g.x, g.y, g.z, g.w}, vw[4] = {v.x, v.y, v.z, v.w};
-    unsigned o[4];
-#pragma unroll
-    for (int e = 0; e < 4; ++e)
-      o[e] = (unsigned)relu_bwd1((u16)(gw[e] & 0xFFFF), (u16)(vw[e] & 0xFFFF), mode) |
-             ((unsigned)relu_bwd1((u16)(gw[e] >> 16), (u16)(vw[e] >> 16), mode) << 16);
-    dz[i] = make_uint4(o[0], o[1], o[2], o[3]);
-  }
+  for (long long i = (long long)blockIdx.x * 256 + threadIdx.x; i < n8; i += (long long)gridDim.x * 256)
+    dz[i] = relu_bwd8(dy[i], y[i], mode);
 }
 
 // 2x2x2 average pooling (and its adjoint) on [n][d][h][w][c].
@@ -1533,8 +1535,14 @@ __global__ __launch_bounds__(256) void head_bwd_v8_kernel(const float* dout, con
 // bias_grad_kernel for C % 8 == 0 channels with 16-byte loads: thread t sums
 // channels 8 (t % (C / 8)) .. + 7 over every (256 / (C / 8))-th voxel of the
 // block's share; partial sums meet in LDS, then one atomic per channel.
-template <int C>
-__global__ __launch_bounds__(256) void bias_grad_v8_kernel(const uint4* dy, float* db, long long nvox) {
+// With y (ACT) dy is the gradient behind the activation: the kernel writes the
+// adjoint dz as relu_bwd_v8_kernel does and sums that, so dz is not read again.
+// Bound by HBM: three tensors of 134 MB (2.1 M voxels x 32 channels) take 75 us,
+// 70 + 34 as two kernels.  The db atomics of all blocks meet in C addresses:
+// 512 blocks 75 us, 2048 82, 4096 100.
+template <int C, bool ACT>
+__global__ __launch_bounds__(256) void bias_grad_v8_kernel(const uint4* dy, const uint4* y, uint4* dz,
+                                                           float* db, long long nvox, int mode) {
   constexpr int G = C / 8, L = 256 / G;  // channel groups, voxel lanes
   __shared__ float red[C];
   for (int i = threadIdx.x; i < C; i += 256) red[i] = 0.f;
@@ -1542,7 +1550,11 @@ __global__ __launch_bounds__(256) void bias_grad_v8_kernel(const uint4* dy, floa
   const int g = threadIdx.x % G, l = threadIdx.x / G;
   float s[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
   for (long long v = (long long)blockIdx.x * L + l; v < nvox; v += (long long)gridDim.x * L) {
-    const uint4 q = dy[v * G + g];
+    uint4 q = dy[v * G + g];
+    if constexpr (ACT) {
+      q = relu_bwd8(q, y[v * G + g], mode);
+      dz[v * G + g] = q;
+    }
     const unsigned u[4] = {q.x, q.y, q.z, q.w};
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
@@ -2200,18 +2212,24 @@ extern "C" int fdk_nn_flip_weights(const void* w, void* wb, int cin, int cout, v
   return FDK_OK;
 }
 
+template <int C, bool ACT>
+static void launch_bias_v8(const uint4* dy, const uint4* y, uint4* dz, float* db, int64_t nvox, int mode,
+                           hipStream_t st) {
+  hipLaunchKernelGGL((bias_grad_v8_kernel<C, ACT>), dim3(ACT ? 512 : 1024), dim3(256), 0, st, dy, y, dz, db,
+                     (long long)nvox, mode);
+}
+
 extern "C" int fdk_nn_bias_grad(const void* dy, float* db, int64_t nvox, int c, void* stream) {
   FDK_REQUIRE(dy && db && c > 0 && c <= 256 && 256 % c == 0, "bias_grad needs c dividing 256");
   hipStream_t st = static_cast<hipStream_t>(stream);
-  const dim3 g(1024), b(256);
   const uint4* v = static_cast<const uint4*>(dy);
   if (!aligned16(dy)) c = -c;  // the scalar kernel below
   switch (c) {
-    case 32: hipLaunchKernelGGL(bias_grad_v8_kernel<32>, g, b, 0, st, v, db, (long long)nvox); break;
-    case 64: hipLaunchKernelGGL(bias_grad_v8_kernel<64>, g, b, 0, st, v, db, (long long)nvox); break;
-    case 128: hipLaunchKernelGGL(bias_grad_v8_kernel<128>, g, b, 0, st, v, db, (long long)nvox); break;
+    case 32: launch_bias_v8<32, false>(v, nullptr, nullptr, db, nvox, 0, st); break;
+    case 64: launch_bias_v8<64, false>(v, nullptr, nullptr, db, nvox, 0, st); break;
+    case 128: launch_bias_v8<128, false>(v, nullptr, nullptr, db, nvox, 0, st); break;
     default:
-      hipLaunchKernelGGL(bias_grad_kernel, g, b, 0, st, static_cast<const u16*>(dy), db, (long long)nvox,
+      hipLaunchKernelGGL(bias_grad_kernel, dim3(1024), dim3(256), 0, st, static_cast<const u16*>(dy), db, (long long)nvox,
                          c < 0 ? -c : c);
   }
   FDK_HIP(hipGetLastError());
@@ -2232,6 +2250,25 @@ extern "C" int fdk_nn_relu_bwd(const void* dy, const void* y, void* dz, int64_t 
                        (long long)n, mode);
   FDK_HIP(hipGetLastError());
   return FDK_OK;
+}
+
+extern "C" int fdk_nn_act_bias_bwd(const void* dy, const void* y, void* dz, float* db, int64_t nvox,
+                                   int c, int mode, void* stream) {
+  FDK_REQUIRE(dy && y && dz && db && c > 0, "NULL pointer or no channels");
+  FDK_REQUIRE(mode == 1 || mode == 2, "activation mode must be 1 (ReLU) or 2 (leaky ReLU)");
+  // one pass where bias_grad has a 16-byte form, else the two kernels
+  if ((c == 32 || c == 64 || c == 128) && aligned16(dy) && aligned16(y) && aligned16(dz)) {
+    hipStream_t st = static_cast<hipStream_t>(stream);
+    const uint4 *g = static_cast<const uint4*>(dy), *v = static_cast<const uint4*>(y);
+    uint4* o = static_cast<uint4*>(dz);
+    if (c == 32) launch_bias_v8<32, true>(g, v, o, db, nvox, mode, st);
+    else if (c == 64) launch_bias_v8<64, true>(g, v, o, db, nvox, mode, st);
+    else launch_bias_v8<128, true>(g, v, o, db, nvox, mode, st);
+    FDK_HIP(hipGetLastError());
+    return FDK_OK;
+  }
+  const int rc = fdk_nn_relu_bwd(dy, y, dz, nvox * c, mode, stream);
+  return rc != FDK_OK ? rc : fdk_nn_bias_grad(dz, db, nvox, c, stream);
 }
 
 extern "C" int fdk_nn_avgpool2(const void* x, void* y, int n, int d, int h, int w, int c, int adjoint,

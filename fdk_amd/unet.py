@@ -52,6 +52,7 @@ def _sig():
     L.fdk_nn_flip_weights.argtypes = [vp, vp, i, i, vp]
     L.fdk_nn_bias_grad.argtypes = [vp, vp, i64, i, vp]
     L.fdk_nn_relu_bwd.argtypes = [vp, vp, vp, i64, i, vp]
+    L.fdk_nn_act_bias_bwd.argtypes = [vp, vp, vp, vp, i64, i, i, vp]
     L.fdk_nn_avgpool2.argtypes = [vp, vp, i, i, i, i, i, i, vp]
     L.fdk_nn_upsample2.argtypes = [vp, vp, i, i, i, i, i, i, i, i, vp]
     L.fdk_nn_channel_copy.argtypes = [vp, i, i, vp, i, i, i, i64, vp]
@@ -127,6 +128,13 @@ def bias_grad(dy, db, nvox, c):
 
 def relu_bwd(dy, y, dz, mode=1):
     _check(L().fdk_nn_relu_bwd(_p(dy), _p(y), _p(dz), dy.numel(), int(mode), _st()), "relu_bwd")
+    return dz
+
+
+def act_bias_bwd(dy, y, dz, db, nvox, c, mode=1):
+    """relu_bwd into dz and bias_grad of dz into db, in one pass."""
+    _check(L().fdk_nn_act_bias_bwd(_p(dy), _p(y), _p(dz), _p(db), nvox, c, int(mode), _st()),
+           "act_bias_bwd")
     return dz
 
 
@@ -257,12 +265,16 @@ class Conv3:
         cat = (up, cup) the skip half of the input [upsample2(up), x] that
         forward_cat read."""
         torch = _torch()
-        dz = relu_bwd(dy, y, torch.empty_like(dy), self.relu) if self.relu else dy
+        nvox = int(np.prod(shape))
+        if self.relu:
+            dz = act_bias_bwd(dy, y, torch.empty_like(dy), self.gb, nvox, self.cout, self.relu)
+        else:
+            dz = dy
+            bias_grad(dz, self.gb, nvox, self.cout)
         if cat is None:
             conv3d_wgrad(x, dz, self.gw, shape, self.cin, self.cout)
         else:
             conv3d_wgrad_cat(cat[0], cat[1], x, dz, self.gw, shape, self.cin, self.cout)
-        bias_grad(dz, self.gb, int(np.prod(shape)), self.cout)
         if not need_dx:
             return None
         dx = torch.empty(shape + (self.cin,), dtype=I16, device=dy.device)

@@ -341,6 +341,10 @@ int fdk_nn_bias_grad(const void* dy, float* db, int64_t nvox, int c, void* strea
 /* Activation adjoint at output y: dz = dy where y > 0, else 0 (mode 1, ReLU) or
  * 0.01 dy (mode 2, leaky ReLU). */
 int fdk_nn_relu_bwd(const void* dy, const void* y, void* dz, int64_t n, int mode, void* stream);
+/* fdk_nn_relu_bwd of [nvox][c] followed by fdk_nn_bias_grad of dz, in one pass
+ * over the tensors for c 32, 64 or 128 (16-byte aligned). */
+int fdk_nn_act_bias_bwd(const void* dy, const void* y, void* dz, float* db, int64_t nvox, int c,
+                        int mode, void* stream);
 /* 2x2x2 average pooling of [n][d][h][w][c] (adjoint 1: [n][d/2][h/2][w/2][c] -> full). */
 int fdk_nn_avgpool2(const void* x, void* y, int n, int d, int h, int w, int c, int adjoint,
                     void* stream);

@@ -1,5 +1,6 @@
 """3x3x3 convolution layers: the work split of the forward and weight-gradient
-kernels, against the FP64 restatement."""
+kernels and the fused activation adjoint and bias gradient, against the FP64
+restatement."""
 import numpy as np
 import pytest
 
@@ -13,8 +14,37 @@ def bf(torch, a):
     return torch.as_tensor(R.to_bf16_bits(a).view(np.int16)).cuda()
 
 
+def from_bf(t):
+    return R.from_bf16_bits(t.cpu().numpy().view(np.uint16))
+
+
 def rel(a, b):
     return float(np.linalg.norm(np.ravel(a - b)) / max(np.linalg.norm(np.ravel(b)), 1e-300))
+
+
+@pytest.mark.parametrize("mode", [1, 2])
+@pytest.mark.parametrize("c,nvox,shift", [(16, 4099, 0), (32, 1, 0), (32, 70001, 0), (64, 3 * 4099, 0),
+                                          (128, 5003, 0), (128, 5003, 1)])
+def test_activation_and_bias(torch_cuda, c, nvox, shift, mode):
+    """dz bit for bit (dy where y > 0, else 0 or 0.01 dy rounded to BF16) and its
+    per-channel sums added to db: the one-pass form at 32, 64 and 128 channels,
+    the two kernels at 16 channels and for a tensor off 16-byte alignment."""
+    torch = torch_cuda
+    rng = np.random.default_rng(c + nvox + mode)
+    dy = R.bf16_round(rng.standard_normal((nvox, c)))
+    y = R.bf16_round(rng.standard_normal((nvox, c)))
+    y[::7] = 0.0
+    ref = np.where(y > 0, dy, 0.0 if mode == 1 else R.bf16_round(np.float32(0.01) * dy.astype(np.float32)))
+    buf = torch.empty(nvox * c + shift, dtype=torch.int16, device="cuda")
+    g = buf[shift:].view(nvox, c)
+    g.copy_(bf(torch, dy))
+    dz = torch.empty((nvox, c), dtype=torch.int16, device="cuda")
+    db = torch.ones(c, device="cuda")
+    U.act_bias_bwd(g, bf(torch, y), dz, db, nvox, c, mode)
+    assert np.array_equal(from_bf(dz), ref)
+    # FP32 sums: at most nvox roundings of 2^-24 of the sum of magnitudes, in practice their root
+    bound = (1.0 + np.abs(ref).sum(0)) * 2.0 ** -24 * (8.0 + nvox ** 0.5)
+    assert (np.abs(db.cpu().numpy() - (1.0 + ref.sum(0))) <= bound).all()
 
 
 @pytest.mark.parametrize("cin,cout,n", [(32, 32, 3), (96, 32, 70), (288, 160, 13), (1216, 256, 3)])
