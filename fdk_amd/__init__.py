@@ -120,6 +120,9 @@ _SIGS = {
                                       C.c_int, C.c_void_p]),
     "fdk_fp_project": (C.c_int, [C.c_void_p, C.c_void_p, C.c_int, C.c_int, C.c_double, C.c_int,
                                  C.c_void_p, C.c_void_p]),
+    "fdk_ratio_masked": (C.c_int, [C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p, C.c_int64,
+                                   C.c_int64, C.c_void_p]),
+    "fdk_ratio_update": (C.c_int, [C.c_void_p, C.c_void_p, C.c_void_p, C.c_int64, C.c_void_p]),
     "fdk_phantom_rasterize": (C.c_int, [C.c_void_p, C.c_int, C.c_void_p, C.c_void_p,
                                         C.c_void_p]),
     "fdk_phantom_project": (C.c_int, [C.c_void_p, C.c_int, C.c_void_p, C.c_int, C.c_int,

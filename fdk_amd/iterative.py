@@ -23,7 +23,7 @@ from __future__ import annotations
 
 import numpy as np
 
-from . import FP_ZERO, BackProjectionFDK, Parameter, forward_project
+from . import FP_ZERO, BackProjectionFDK, Parameter, _check, _dev_ptr, _stream, forward_project, lib
 
 
 class Projector:
@@ -88,6 +88,38 @@ def _safe_div(a, b):
     return torch.where(b != 0, a / torch.where(b != 0, b, torch.ones_like(b)), torch.zeros_like(a))
 
 
+def _fusable(*ts):
+    """Whether the fused quotient kernels take these arrays: plain FP32, dense, on the
+    current device, outside autograd; anything else keeps the element-wise form."""
+    import torch
+    return all(t.dtype == torch.float32 and t.is_cuda and t.is_contiguous() and not t.requires_grad
+               and t.device.index == torch.cuda.current_device() for t in ts)
+
+
+def _masked_ratio(a, b, mask):
+    """a / b * mask over views of the mask's shape, a zero divisor giving zero."""
+    import torch
+    if not (type(a) is torch.Tensor and a.shape == b.shape and a.shape[1:] == mask.shape
+            and _fusable(a, b, mask)):
+        return _safe_div(a, b) * mask
+    out = torch.empty_like(a)
+    _check(lib().fdk_ratio_masked(_dev_ptr(a), _dev_ptr(b), _dev_ptr(mask), _dev_ptr(out),
+                                  mask.numel(), a.shape[0], _stream(None)), "ratio_masked")
+    return out
+
+
+def _scale_by_ratio(x, a, b):
+    """x *= a / b in place, a zero divisor giving zero."""
+    import torch
+    if not (type(x) is torch.Tensor and x.shape == a.shape == b.shape and _fusable(x, a, b)):
+        x *= _safe_div(a, b)
+        return x
+    _check(lib().fdk_ratio_update(_dev_ptr(x), _dev_ptr(a), _dev_ptr(b), x.numel(), _stream(None)),
+           "ratio_update")
+    torch.autograd.graph.increment_version(x)  # written outside torch's sight
+    return x
+
+
 def ratio_reconstruct(para: Parameter, proj, iters: int, roi_border: int = 2, vol=None,
                       callback=None, projector: Projector | None = None):
     """proj: device (nproj, nv, nu) FP32 measured views.  Returns the volume
@@ -105,9 +137,8 @@ def ratio_reconstruct(para: Parameter, proj, iters: int, roi_border: int = 2, vo
     upd = torch.empty_like(norm)
     for it in range(iters):
         A.forward(x, views, fp)
-        ratio = _safe_div(p, fp) * mask
-        A.back(ratio, views, upd)
-        x *= _safe_div(upd, norm)
+        A.back(_masked_ratio(p, fp, mask), views, upd)
+        x = _scale_by_ratio(x, upd, norm)
         if callback:
             callback(it, x, fp)
     if projector is None:

@@ -291,6 +291,14 @@ int fdk_fp_project(const fdk_geometry* g, const float* dev_vol, int first, int c
 int fdk_fp_project_host(const fdk_geometry* g, const float* host_vol, int first, int count,
                         double step_mm, int mode, float* host_out);
 
+/* The quotients of the multiplicative update (Iterative3dReconstructionRatio,
+ * 3dct/3dct.cpp:1029-1205; a zero divisor gives zero, type.h:3908-3920):
+ * out[g][i] = a[g][i] / b[g][i] * mask[i] over `groups` arrays of `period` floats,
+ * and x[i] *= a[i] / b[i] over n floats, on device memory. */
+int fdk_ratio_masked(const float* a, const float* b, const float* mask, float* out, int64_t period,
+                     int64_t groups, void* stream);
+int fdk_ratio_update(float* x, const float* a, const float* b, int64_t n, void* stream);
+
 /* ------------------------------------------------------------ random phantoms */
 /* Voxel-centre rasterization into dev_vol (nz x ny x nx floats, overwritten). */
 int fdk_phantom_rasterize(const fdk_ellipsoid* host_ell, int n, const fdk_geometry* g,
