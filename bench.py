@@ -26,6 +26,7 @@ HBM_PEAK = 8.0e12               # MI355X HBM3E, B/s
 # MI355X vector issue: 256 CUs x 2.4 GHz x one wave64 VALU instruction per CU
 # per clock (four SIMD16 units, four clocks per wave64 instruction)
 VALU_PEAK = 256 * 2.4e9
+L1_PEAK = 256 * 2.4e9 * 64  # 64 B per CU per clock
 HERE = os.path.dirname(os.path.abspath(__file__))
 
 
@@ -659,7 +660,7 @@ def load_counters(kernel: str, dt: str, n: int):
 def roofline_of(kernel: str, dt: str, n: int, avg_ms: float, upd_per_launch: float,
                 b_upd: float):
     """Roofline of the dominant kernel.  The bound is the resource the committed
-    counters show closest to its peak (VALU issue for the LDS-staged kernel);
+    counters show closest to its peak (the L1 return path or VALU issue);
     `achieved` is that resource's per-update figure from the counter summary
     times this launch's updates over the live event-timed launch duration.  The
     algorithmic HBM figure (4 taps x sample bytes + 8 B / 32 views per update,
@@ -680,15 +681,18 @@ def roofline_of(kernel: str, dt: str, n: int, avg_ms: float, upd_per_launch: flo
     valu = c["valu_insts_per_update"] * upd_per_launch / (avg_ms * 1e-3)
     hbm = c["hbm_bytes_per_launch"] / (avg_ms * 1e-3)
     l2 = c.get("l2_bytes_per_launch")
+    busy = (f"VALU issue {c['valu_busy']:.0%} busy, LDS {c['lds_busy']:.0%}, HBM "
+            f"{c['hbm_bytes_per_launch'] / (c['gpu_cycles'] / 2.37e9) / HBM_PEAK:.0%}")
+    if c.get("l1_return_busy", 0.0) > c["valu_busy"]:
+        l1 = c["l1_bytes_per_launch"] / (avg_ms * 1e-3)
+        r.update({"bound": "l1", "achieved": round(l1 / 1e9, 1), "peak": round(L1_PEAK / 1e9, 1),
+                  "unit": "GB/s through the L1s", "frac": round(l1 / L1_PEAK, 4)})
+        busy = f"L1 return path {c['l1_return_busy']:.0%} busy, " + busy
+    else:
+        r.update({"bound": "valu", "achieved": round(valu / 1e9, 1), "peak": round(VALU_PEAK / 1e9, 1),
+                  "unit": "G VALU wave-instructions/s", "frac": round(valu / VALU_PEAK, 4)})
     r.update({
-        "bound": "valu",
-        "bound_note": ("the busiest resource in the counter summary (VALU issue "
-                       f"{c['valu_busy']:.0%} busy, LDS {c['lds_busy']:.0%}, HBM "
-                       f"{c['hbm_bytes_per_launch'] / (c['gpu_cycles'] / 2.37e9) / HBM_PEAK:.0%})"),
-        "achieved": round(valu / 1e9, 1),
-        "peak": round(VALU_PEAK / 1e9, 1),
-        "unit": "G VALU wave-instructions/s",
-        "frac": round(valu / VALU_PEAK, 4),
+        "bound_note": f"the busiest resource in the counter summary ({busy})",
         "traffic": c["hbm_bytes_per_launch"],
         "traffic_source": src,
         "valu_insts_per_update": c["valu_insts_per_update"],

@@ -7,7 +7,8 @@ Each ``<out_dir>/<pass_dir>`` holds one ``rocprofv3 --pmc ... -o pmc -f csv`` ru
 the rows of the named kernel and averaged over its dispatches.  HBM traffic
 scales FETCH_SIZE by 2.0 and WRITE_SIZE by 1.0 (KiB per dispatch; the factors a
 plain 1 GiB device copy reads on this part, ``bench.py --calibrate-copy``).
-Busy fractions divide by GRBM_GUI_ACTIVE / 8 (cycles per XCD).  The JSON goes
+Busy fractions divide by GRBM_GUI_ACTIVE / 8 (cycles per XCD); the L1 return
+path's are added where the passes hold TD_TD_BUSY_sum.  The JSON goes
 to stdout; ``bench.py`` reads ``profiles/<kernel>_<dtype>_<n>cube_counters.json``
 for its roofline object.
 """
@@ -39,7 +40,7 @@ def summarise(out_dir: str, kernel: str, workload: str, updates: float, passes: 
     fetch = avg["FETCH_SIZE"] * 1024 * FETCH_FACTOR
     write = avg["WRITE_SIZE"] * 1024 * WRITE_FACTOR
     cycles = avg["GRBM_GUI_ACTIVE"] / 8
-    return {
+    r = {
         "kernel": kernel, "workload": workload, "voxel_updates_per_launch": updates,
         "counters_avg_per_dispatch": {c: avg[c] for c in sorted(avg)},
         "dispatches": {c: len(v) for c, v in vals.items()},
@@ -56,6 +57,10 @@ def summarise(out_dir: str, kernel: str, workload: str, updates: float, passes: 
         "tcc_hit_rate": avg["TCC_HIT_sum"] / (avg["TCC_HIT_sum"] + avg["TCC_MISS_sum"]),
         "fetch_factor": FETCH_FACTOR, "write_factor": WRITE_FACTOR,
     }
+    if "TD_TD_BUSY_sum" in avg and "TCP_TOTAL_CACHE_ACCESSES_sum" in avg:
+        r["l1_return_busy"] = avg["TD_TD_BUSY_sum"] / 256 / cycles
+        r["l1_bytes_per_launch"] = avg["TCP_TOTAL_CACHE_ACCESSES_sum"] * 64
+    return r
 
 
 def main(argv=None) -> None:

@@ -1237,7 +1237,7 @@ __global__ __launch_bounds__(256) void volume_out_kernel(const float* __restrict
 
 // The same on 64 x 64 tiles with 16-byte loads and stores; nxs, nzz, z_begin
 // and nzc multiples of 4, `out` 16-byte aligned.  Bound by HBM (one read, one
-// write); a tile row is 256 bytes on both sides.  1024^3: 1.6 ms (5.4 TB/s), 2.63 (3.3
+// write); a tile row is 256 bytes on both sides.  1024^3: 1.73 ms (5.0 TB/s), 2.63 (3.3
 // TB/s) by 32 x 32 tiles of 4-byte accesses.  No bank conflicts: a wave's 4
 // rows x 16 groups of 4 fall in 64 different banks both ways.
 __global__ __launch_bounds__(256) void volume_out_v4_kernel(const float* __restrict__ vol,
