@@ -69,7 +69,8 @@ struct BpArgs {
   int tiles_x;           // tiles along x
   long long view_bytes;  // view_stride in bytes
   int view_bytes32;      // W * H * sample bytes (< 2^31), the range of a view's resource
-  int row_bytes;         // W * sample bytes
+  int pitch;             // samples between a view's rows: W, more in a re-pitched copy
+  int row_bytes;         // pitch * sample bytes
   int buf16;             // 16-bit samples with 4-byte aligned rows and views (buffer path)
   const unsigned* mm;    // per-view {min, max} words on the device (16-bit views), or null
 };
@@ -584,7 +585,7 @@ __device__ __forceinline__ void compute_direct(float (&acc)[ZPT], float (&accm)[
       __builtin_amdgcn_make_buffer_rsrc((void*)vbase, 0, a.view_bytes32, fdk::kRawRsrcWord3);
   const __amdgpu_buffer_rsrc_t g1 = __builtin_amdgcn_make_buffer_rsrc(
       (void*)(vbase + a.row_bytes), 0, a.view_bytes32 - a.row_bytes, fdk::kRawRsrcWord3);
-  const int rowbase = c.iu * a.W;
+  const int rowbase = c.iu * a.pitch;
   const float off = of * c.Z2;
 #pragma unroll
   for (int j = 0; j < ZPT; ++j) {
@@ -1063,7 +1064,7 @@ __global__ __launch_bounds__(256, (ws_waves<DT, SYM, ZPT>())) void bp_wave_kerne
     wv.quads = any ? (min(ihi + 1, a.W - 1) - wv.c0 + 4) >> 2 : 0;
     // With rows of a multiple of 4 samples the quads end with the row.  Else the
     // last one may reach up to 3 samples past it, which must not leave the view.
-    const int over = wv.c0 + 4 * wv.quads - a.W;
+    const int over = wv.c0 + 4 * wv.quads - a.pitch;
     const bool inside = over <= 0 || wv.iu + 3 <= a.H;
     fits = 4 * wv.quads <= CT - 2 && wv.quads <= kWave * NQ && inside;
   }
@@ -1329,6 +1330,7 @@ int fill_args(fdk_bp* h, int W, int H, long long view_stride, int esize, int npr
   a.tiles_x = ((a.nxs + 1) / 2 + kTile - 1) / kTile;
   a.view_bytes = view_stride * esize;
   a.view_bytes32 = (int)view_bytes;
+  a.pitch = W;
   a.row_bytes = W * esize;
   a.buf16 = esize == 2 && (W % 2 == 0) && (view_stride % 2 == 0) &&
             (reinterpret_cast<uintptr_t>(proj) % 4 == 0);
@@ -1547,6 +1549,65 @@ bool launch_wave_run(fdk_bp* h, const BpArgs& a, const BpMats& M, const BpScale&
   return false;
 }
 
+// 16-bit views [u][v] with rows of `pitch` samples, pitch % 4 == 0, zeros past the row.
+__global__ __launch_bounds__(256) void bp_pitch_kernel(const unsigned short* __restrict__ src,
+                                                       uint2* __restrict__ dst, long long view_stride, int W,
+                                                       int H, int pitch) {
+  const int quads = pitch / 4, n = H * quads;
+  const unsigned short* view = src + blockIdx.y * view_stride;
+  for (int i = blockIdx.x * 256 + threadIdx.x; i < n; i += gridDim.x * 256) {
+    const int row = i / quads, c = 4 * (i - row * quads);
+    unsigned q[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) q[e] = c + e < W ? view[(long long)row * W + c + e] : 0u;
+    dst[(long long)blockIdx.y * n + i] = make_uint2(q[0] | q[1] << 16, q[2] | q[3] << 16);
+  }
+}
+
+// bp_wave_kernel for 16-bit views whose rows no 4-byte load fits (odd rows or view
+// strides, odd addresses): on a copy with rows of a multiple of 4 samples, one run a
+// slab with the matrices' own positions.  The copy costs a launch, about 3 us, and 4
+// bytes a sample at about 1 TB/s; against the gather kernel an update saves 0.5 to 5 ps
+// (BF16 pair of 503 x 504 x 500 from 96 views of 513 x 517: 11.7 -> 6.0 ms; FP16 pair of
+// 254 x 243 x 242 from 29 of 300 x 279: 912 -> 345 us; 74 x 61 x 60 from 12 of 70 x 67:
+// 43 -> 39).  Not while a graph is captured or without memory for it.
+constexpr double kPitchSave = 1e-12;  // seconds an update
+
+template <int DT>
+bool launch_wave(fdk_bp* h, const BpArgs& a, const BpMats& M, const BpScale& S);
+
+template <int DT>
+bool launch_wave_pitched(fdk_bp* h, const BpArgs& a, const BpMats& M, const BpScale& S) {
+  if (DT == FDK_F32 || kernel_choice() < 5 || a.buf16) return false;
+  const int pitch = (a.W + 4) & ~3;  // never W: tells a copy from the caller's own views
+  const long long view = (long long)pitch * a.H;
+  if (view * 2 >= (1LL << 31)) return false;
+  const double updates = (double)a.nxs * a.nys * a.nzz * a.nproj;
+  if (updates * kPitchSave < 3e-6 + (double)view * a.nproj * 4 / 1e12) return false;
+  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(h->stream, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone) {
+    (void)hipGetLastError();
+    return false;
+  }
+  fdk::Scratch ws;
+  if (fdk::scratch_get(&ws, (size_t)view * 2 * a.nproj, h->stream) != FDK_OK) return false;
+  BpArgs b = a;
+  b.proj = ws.p;
+  b.pitch = pitch;
+  b.row_bytes = 2 * pitch;
+  b.view_stride = view;
+  b.view_bytes = 2 * view;
+  b.view_bytes32 = (int)(2 * view);
+  b.buf16 = 1;
+  const int blocks = (int)std::min<long long>(1024, (view / 4 + 255) / 256);
+  hipLaunchKernelGGL(bp_pitch_kernel, dim3(blocks, a.nproj), dim3(256), 0, h->stream,
+                     static_cast<const unsigned short*>(a.proj), static_cast<uint2*>(ws.p), a.view_stride, a.W,
+                     a.H, pitch);
+  const bool done = launch_wave<DT>(h, b, M, S);
+  fdk::scratch_put(&ws, h->stream);
+  return done;
+}
+
 template <int DT>
 bool launch_wave(fdk_bp* h, const BpArgs& a, const BpMats& M, const BpScale& S) {
   if (kernel_choice() < 5 || (DT != FDK_F32 && !a.buf16)) return false;
@@ -1556,7 +1617,7 @@ bool launch_wave(fdk_bp* h, const BpArgs& a, const BpMats& M, const BpScale& S) 
   // to rounding, but a voxel on the detector's edge can fall on the other side of it.
   // Rows of a multiple of 4 samples have always been read that way; others keep the
   // matrices' positions, one run a slab.
-  const bool quads = a.W % 4 == 0 && (DT == FDK_F32 || (reinterpret_cast<uintptr_t>(a.proj) % 8 == 0 &&
+  const bool quads = a.W % 4 == 0 && a.pitch == a.W && (DT == FDK_F32 || (reinterpret_cast<uintptr_t>(a.proj) % 8 == 0 &&
                                                         a.view_stride % 4 == 0));
   if (h->sym && quads && mirror_symmetric(a, M)) return launch_wave_run<DT, true>(h, a, M, S, dvz);
   if (!launch_wave_run<DT, false>(h, a, M, S, dvz)) return false;
@@ -1585,7 +1646,7 @@ int launch_bp_dt(fdk_bp* h, const BpArgs& a, const BpMats& M, const BpScale& S, 
     dim3 grid(nblk, (a.zext + kWave - 1) / kWave);
     if (h->sym) hipLaunchKernelGGL((bp_general_kernel<DT, true>), grid, dim3(256), 0, h->stream, a, M, S);
     else hipLaunchKernelGGL((bp_general_kernel<DT, false>), grid, dim3(256), 0, h->stream, a, M, S);
-  } else if (!launch_wave<DT>(h, a, M, S)) {
+  } else if (!launch_wave<DT>(h, a, M, S) && !launch_wave_pitched<DT>(h, a, M, S)) {
     switch (zpt_choice(a.zext)) {
       case 4: launch_column<DT, 4>(h, a, M, S, nblk); break;
       case 16: launch_column<DT, 16>(h, a, M, S, nblk); break;
