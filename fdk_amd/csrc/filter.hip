@@ -33,6 +33,7 @@
 #include <vector>
 
 #include "common.hpp"
+#include "launch_rules.hpp"
 
 namespace {
 
@@ -54,6 +55,7 @@ struct FilterArgs {
   // write (p - min) / (max - min) of view {min, max} words qmm as 16-bit.
   int qmode;
   const unsigned* qmm;
+  int far;                // kFilterWideFar: transposed FP32 stores check their points
 };
 
 constexpr int kStoreF32 = 0, kStoreNone = 1, kStoreF16 = 2, kStoreBF16 = 3;
@@ -682,13 +684,14 @@ __device__ __forceinline__ void wide_minmax(const FilterArgs& a, StoreCtx& c, in
 }
 
 // Stores the 16 points, cropped.  FP32 goes through a resource of the view (transposed)
-// or the row: points outside the row fall outside it and are dropped.
-template <int M, int Q, bool MM>
+// or the row: points outside the row fall outside it and are dropped.  Where their
+// offsets could wrap into the view (a.far) each point is checked instead.
+template <int M, int Q, bool MM, bool FAR = false>
 __device__ __forceinline__ void wide_store(const FilterArgs& a, int view, int ra, bool live, bool has_b,
                                            int t, int off, const float2 (&x)[16]) {
   constexpr int T = Wide<M>::T;
   StoreCtx c = store_ctx(a, view);
-  if constexpr (Q == kStoreF32 && T >= 64) {
+  if constexpr (Q == kStoreF32 && T >= 64 && !FAR) {
     float* d = a.dst + view * a.dst_view;
     if (a.transpose) {
       const __amdgpu_buffer_rsrc_t rd = __builtin_amdgcn_make_buffer_rsrc(
@@ -921,6 +924,9 @@ __global__ __launch_bounds__(Wide<M>::THREADS, (M == 14 ? 4 : 2)) void filter_wi
       wide_store<M, kStoreF16, false>(a, view, ra, live, has_b, t, off, x[0]);
     } else if (a.qmode == kStoreBF16) {
       wide_store<M, kStoreBF16, false>(a, view, ra, live, has_b, t, off, x[0]);
+    } else if (a.far) {
+      if (a.minmax) wide_store<M, kStoreF32, true, true>(a, view, ra, live, has_b, t, off, x[0]);
+      else wide_store<M, kStoreF32, false, true>(a, view, ra, live, has_b, t, off, x[0]);
     } else if (a.minmax) {
       wide_store<M, kStoreF32, true>(a, view, ra, live, has_b, t, off, x[0]);
     } else {
@@ -1070,14 +1076,8 @@ template <int M>
 int launch_wide(const FilterArgs& a, int nviews, hipStream_t st) {
   const long long waves = (long long)((a.nrows + 1) / 2) * nviews * Wide<M>::T / 64;
   if constexpr (M <= 13)
-    if (a.transpose && a.qmode == kStoreF32 && waves >= 4096) return launch_wide_sets<M, true>(a, nviews, st);
+    if (a.transpose && a.qmode == kStoreF32 && !a.far && waves >= 4096) return launch_wide_sets<M, true>(a, nviews, st);
   return launch_wide_sets<M, false>(a, nviews, st);
-}
-
-// 32-bit offsets in a row and a view, and pair counts that fit the kernel's ints.
-bool wide_ok(const FilterArgs& a, int nviews) {
-  return a.logN >= 7 && a.logN <= 14 && (long long)a.nu * a.nrows * 4 < (1LL << 31) &&
-         (long long)(a.nrows + 64) * nviews < (1LL << 29);
 }
 
 int launch_filter(FilterArgs& a, int nviews, hipStream_t st) {
@@ -1090,7 +1090,9 @@ int launch_filter(FilterArgs& a, int nviews, hipStream_t st) {
   a.logN = log2_exact(a.N);
   if (!a.tw)
     if (int r = twiddles(a.N, &a.tw)) return r;
-  if (fft_choice() && wide_ok(a, nviews)) {
+  const auto form = fdk::rules::filter_form(a.nu, a.nrows, nviews, a.logN, a.transpose && a.qmode == kStoreF32);
+  a.far = form == fdk::rules::kFilterWideFar;
+  if (fft_choice() && form != fdk::rules::kFilterInPlace) {
     switch (a.logN) {
       case 7: return launch_wide<7>(a, nviews, st);
       case 8: return launch_wide<8>(a, nviews, st);

@@ -1,0 +1,6 @@
+// The launch rules of csrc/launch_rules.hpp behind C entry points, for the tests.
+#include "launch_rules.hpp"
+
+extern "C" int check_filter_form(int nu, int nrows, int nviews, int log_n, int transposed_f32) {
+  return fdk::rules::filter_form(nu, nrows, nviews, log_n, transposed_f32 != 0);
+}
