@@ -321,7 +321,7 @@ __device__ __forceinline__ void store_pair(const FilterArgs& a, StoreCtx& c, int
     store_pair_q<kStoreF32, true>(a, c, view, u, ra, has_b, fa, fb);
 }
 
-// The other lengths (N < 128), views of 2 GiB and more, and FDK_FILTER_FFT=inplace: the
+// The other lengths (N < 128), 2^29 rows and more, and FDK_FILTER_FFT=inplace: the
 // in-place bit-reversed radix-2^2 FFT, a block per row pair.
 __global__ __launch_bounds__(256) void filter_rows_kernel(FilterArgs a) {
   extern __shared__ float2 buf[];

@@ -42,3 +42,16 @@ def test_ordinary_views_take_the_plain_form():
     for nu, nv, log_n in ((64, 64, 7), (2048, 2048, 12), (4096, 4096, 13), (8192, 8192, 14)):
         assert rules().check_filter_form(nu, nv, 32, log_n, 1) == WIDE
         assert rules().check_filter_form(nu, nv, 32, log_n, 0) == WIDE
+
+
+@pytest.mark.parametrize("log_n", range(7, 15))
+def test_no_view_size_leaves_the_wide_kernel(log_n):
+    """Views of 2 GiB and more too: the row-major and 16-bit stores address rows, and the
+    transposed FP32 store has its 64-bit form."""
+    nu = (1 << log_n) - 3
+    for nrows in (300, (1 << 29) // nu, (1 << 29) // nu + 1, 1 << 24):
+        assert rules().check_filter_form(nu, nrows, 1, log_n, 0) == WIDE
+        big = nu * nrows * 4 >= 2 ** 31
+        assert rules().check_filter_form(nu, nrows, 1, log_n, 1) == (FAR if big else WIDE)
+    for m in (4, 5, 6):
+        assert rules().check_filter_form(20, 30, 1, m, 1) == IN_PLACE

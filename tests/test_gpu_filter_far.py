@@ -24,3 +24,29 @@ def test_transposed_equals_row_major(torch_cuda, nu, nrows):
     F.filter_views(src, tr, None, H, F.PAD_MEAN4, True)
     torch.cuda.synchronize()
     assert torch.equal(tr[0].t(), row[0])
+
+
+@pytest.mark.parametrize("nu,parts", [(1000, 9), (300, 31)])
+def test_views_of_2_gib_equal_their_parts(torch_cuda, nu, parts):
+    """A view of 2 GiB and more against the same rows as several smaller views."""
+    import torch
+    nrows = ((1 << 29) // nu // parts + 3) // 2 * 2 * parts  # an even number of rows a part
+    assert nu * nrows * 4 >= 1 << 31
+    g = torch.Generator(device="cuda")
+    g.manual_seed(nu)
+    src = torch.randn((nrows, nu), device="cuda", generator=g)
+    N = 1 << nu.bit_length()
+    k = torch.arange(N, device="cuda")
+    H = torch.minimum(k, N - k) * (2.0 / N)
+    print(f"nu {nu} rows {nrows}", flush=True)
+    ref = torch.empty((parts, nrows // parts, nu), device="cuda")
+    F.filter_views(src.view(ref.shape), ref, None, H, F.PAD_MEAN3, False)
+    ref = ref.view(nrows, nu)
+    out = torch.full((1, nrows, nu), 7.0, device="cuda")
+    F.filter_views(src[None], out, None, H, F.PAD_MEAN3, False)
+    torch.cuda.synchronize()
+    assert torch.equal(out[0], ref)
+    out = out.view(1, nu, nrows).fill_(7.0)
+    F.filter_views(src[None], out, None, H, F.PAD_MEAN3, True)
+    torch.cuda.synchronize()
+    assert torch.equal(out[0].t(), ref)
