@@ -41,6 +41,7 @@
 #include <vector>
 
 #include "common.hpp"
+#include "launch_rules.hpp"
 
 namespace {
 
@@ -777,7 +778,8 @@ __global__ __launch_bounds__(256) void bp_lds_pf_kernel(BpArgs a, BpMats M, BpSc
 // kernels: 1024^3 pair, 64 FP16 views of 1024^2, with read-out 27.8 -> 22.3 ms;
 // 768 x 512 x 2048 pair, 32 FP32 views 12.5 -> 10.6 ms; 256^3 pair, 96 FP32 views
 // 1458 -> 784 us (the 128-deep slabs at ZPT 2 instead of half-empty ZPT 4 runs);
-// 256^3 box of a 1024^3 scan, 128 FP32 views 2096 -> 880 us; 101 x 92 x 83 volume,
+// 256^3 box of a 1024^3 scan, 128 FP32 views 2096 -> 834 us (878 with every second strip
+// 8 bytes off a 16-byte boundary); 101 x 92 x 83 volume,
 // detector 121 x 98, 2 x 40 views with the projector 632 -> 481 us (was the
 // direct-gather kernel: rows no multiple of 4).
 constexpr int kWsQuads = 3;  // strip quads per lane and run at ZPT 8
@@ -987,9 +989,9 @@ template <int DT, bool SYM, int ZPT, int VS>
 __global__ __launch_bounds__(256, (ws_waves<DT, SYM, ZPT>())) void bp_wave_kernel(
     BpArgs a, BpMats M, BpScale S, WsGrid G, int CT) {
   constexpr int NQ = ws_quads<ZPT>(), kSides = SYM ? 2 : 1;
-  // per wave: CT columns of kSides floats, the last two the zero slot; then, with
+  // per wave: CT columns of kSides floats (CT kSides % 4 == 0), the last two the zero slot; then, with
   // VS > 1, every wave's sums
-  extern __shared__ float wstrip[];
+  extern __shared__ __align__(16) float wstrip[];
   // Patches of 2x2 columns in kTile x kTile tiles, those at the right and lower edges
   // cut to the grid: runs of blocks stay in compact regions, and none is padding
   // (in whole tiles a grid of 101 x 92 columns would be a quarter padding, unevenly
@@ -1421,16 +1423,6 @@ bool mirror_symmetric(const BpArgs& a, const BpMats& M) {
   return true;
 }
 
-// Strip slot CT (columns, plus the two-column zero slot) of bp_wave_kernel: the
-// v extent of one wave's z-run (64 * zpt voxels) over the views and the
-// sub-volume's corners, with room for floor rounding and the 4-column alignment
-// of its start.  0 when a corner is behind the source.
-int wave_strip_ct(double dvz, int zpt) {
-  const double span = dvz * (kWave * zpt - 1);
-  const double quads = (std::ceil(span) + 9) / 4 + 1;
-  return quads < 1e6 ? 4 * (int)quads + 2 : 0;
-}
-
 // The largest |dv/dz| over the views and the sub-volume's corners; 0 when a
 // corner is behind the source.
 double max_dvz(const BpArgs& a, const BpMats& M) {
@@ -1522,7 +1514,7 @@ int wave_zpt(double dvz, int zext, int* CT) {
   int best = 0;
   long long cost = 0;
   for (int k = 0; k < 4; ++k) {
-    const int z = kZpt[k], ct = wave_strip_ct(dvz, z);
+    const int z = kZpt[k], ct = fdk::rules::wave_strip_columns(dvz, z, SYM ? 2 : 1);
     if (ct <= 0 || (ct - 2) / 4 > kWave * kSlots[k]) continue;
     if ((size_t)4 * ct * (SYM ? 2 : 1) * sizeof(float) > 60 * 1024) continue;
     const long long runs = (zext + kWave * z - 1) / (kWave * z);

@@ -1,6 +1,7 @@
 // Rules of the launches that need no device: which form of a kernel a call's sizes
 // take.  Host code without HIP, so that tests check them by themselves.
 #pragma once
+#include <cmath>
 #include <cstdint>
 
 namespace fdk {
@@ -23,6 +24,17 @@ inline FilterForm filter_form(int nu, int nrows, int nviews, int log_n, bool tra
                          (int64_t)(nu + (1 << log_n) / 16) * nrows * 4 > (int64_t)1 << 32))
     return kFilterWideFar;
   return kFilterWide;
+}
+
+// Columns of a wave's strip in bp_wave_kernel's LDS: the v extent of a run of 64 zpt
+// voxels at dvz pixels a voxel, with room for floor rounding and the 4-column alignment
+// of its start, then the two-column zero slot.  A column is `sides` floats; the strips of
+// a block's waves follow each other, so theirs are a multiple of 4 floats, which keeps
+// the 16-byte stores of every wave aligned.  0: no such strip.
+inline int wave_strip_columns(double dvz, int zpt, int sides) {
+  const double span = dvz * (64 * zpt - 1);
+  const double quads = (std::ceil(span) + 9) / 4 + 1;
+  return quads < 1e6 ? 4 * (int)quads + (sides == 2 ? 2 : 4) : 0;
 }
 
 }  // namespace rules
