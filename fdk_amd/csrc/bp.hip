@@ -647,12 +647,21 @@ template <bool SYM, int ZPT>
 __device__ __forceinline__ void column_write(const BpArgs& a, int xs, int ys, int zbase,
                                              const float (&acc)[ZPT], const float (&accm)[ZPT]) {
   float* col = a.vol + ((long long)xs * a.nys + ys) * (long long)a.nzz;
+  // every load before the first store: store by store they would wait for each other,
+  // up to 16 memory latencies a column (lanes past the slab load its last voxel)
+  float v[ZPT], m[ZPT];
+#pragma unroll
+  for (int j = 0; j < ZPT; ++j) {
+    const int zl = min(zbase + j * kWave, a.zext - 1);
+    v[j] = col[zl];
+    if (SYM) m[j] = col[a.nzz - 1 - zl];
+  }
 #pragma unroll
   for (int j = 0; j < ZPT; ++j) {
     const int zl = zbase + j * kWave;
     if (zl < a.zext) {
-      col[zl] += acc[j];
-      if (SYM) col[a.nzz - 1 - zl] += accm[j];
+      col[zl] = v[j] + acc[j];
+      if (SYM) col[a.nzz - 1 - zl] = m[j] + accm[j];
     }
   }
 }
@@ -753,8 +762,8 @@ __global__ __launch_bounds__(256) void bp_lds_pf_kernel(BpArgs a, BpMats M, BpSc
 //    columns W-1-c, stored reversed and interleaved with the top run's, so one
 //    16-byte LDS read brings r_top(iv), r_mir(iv), r_top(iv+1), r_mir(iv+1).  The
 //    mirror voxel has v' = W-1-v, so iv' = W-2-iv and t' = 1-t: it shares the top
-//    voxel's floor, fraction and validity (0 <= iv <= W-2).  Otherwise each slab
-//    is one run of its own, with one strip;
+//    voxel's floor, fraction and validity (0 <= iv <= W-2).  Otherwise each slab's
+//    runs are their own, with one strip;
 //  * the per-(column, view) values (u weights, v = Vb + z dV, strip bounds and
 //    flags) are computed once, lane s for view s, and broadcast with readlane;
 //  * the next view's strip loads are issued into registers before the current
@@ -973,8 +982,12 @@ constexpr int ws_waves() { return SYM && ZPT == 8 ? (DT == FDK_F32 ? 4 : 5) : SY
 
 // floor(2^32 / d) of the divisors of bp_wave_kernel's block numbering: a
 // division costs 20 vector instructions, the multiplication a few scalar ones.
+// A pair without SYM is one launch: the blocks from grid row `runs` on take the bottom
+// slab, which starts at plane zbot (a launch of its own costs small volumes 3.5 us,
+// 64^3 from one view 6.3 against 8.8).
 struct WsGrid {
   unsigned band, tile, cols;
+  int runs, zbot;
 };
 __host__ __device__ inline unsigned udiv_inv(unsigned d) {
   return d > 1 ? (unsigned)((1ull << 32) / d) : 0xffffffffu;
@@ -1017,7 +1030,13 @@ __global__ __launch_bounds__(256, (ws_waves<DT, SYM, ZPT>())) void bp_wave_kerne
   float* strip = wstrip + wave * CT * kSides;
   const int zslot = CT - 2;
   if (lane < 2 * kSides) strip[(CT - 2) * kSides + lane] = 0.f;
-  const int zb0 = blockIdx.y * (kWave * ZPT);
+  int run = blockIdx.y;
+  if (!SYM && run >= G.runs) {  // the bottom slab of a pair
+    run -= G.runs;
+    a.z0 = G.zbot;
+    a.vol += a.zext;
+  }
+  const int zb0 = run * (kWave * ZPT);
   const int zend = min(zb0 + kWave * ZPT, a.zext) - 1;  // the run's last voxel
   const int zbase = zb0 + lane;
   const float x = (float)(a.x0 + xs);
@@ -1481,9 +1500,10 @@ bool launch_wave_zpt(fdk_bp* h, const BpArgs& a, const BpMats& M, const BpScale&
   size_t lds = (size_t)4 * CT * kSides * sizeof(float);
   const unsigned npx = (unsigned)(a.nxs + 1) / 2, npy = (unsigned)(a.nys + 1) / 2;
   const unsigned patches = npx * npy;
+  const int runs = (a.zext + kWave * ZPT - 1) / (kWave * ZPT);
   const WsGrid G{udiv_inv(kTile * npx), udiv_inv(kTile * std::max(1u, npy % kTile)),
-                 udiv_inv(std::max(1u, npx % kTile))};
-  dim3 grid((patches + 7u) & ~7u, (a.zext + kWave * ZPT - 1) / (kWave * ZPT));
+                 udiv_inv(std::max(1u, npx % kTile)), runs, (int)h->bot.z};
+  dim3 grid((patches + 7u) & ~7u, !SYM && h->sym ? 2 * runs : runs);
   if constexpr (ZPT <= 2) {
     if ((long long)a.nxs * a.nys * grid.y < kSplitWaves && a.nproj >= 8) {
       grid.x *= 4;
@@ -1558,13 +1578,8 @@ __global__ __launch_bounds__(256) void bp_pitch_kernel(const unsigned short* __r
 
 // bp_wave_kernel for 16-bit views whose rows no 4-byte load fits (odd rows or view
 // strides, odd addresses): on a copy with rows of a multiple of 4 samples, one run a
-// slab with the matrices' own positions.  The copy costs a launch, about 3 us, and 4
-// bytes a sample at about 1 TB/s; against the gather kernel an update saves 0.5 to 5 ps
-// (BF16 pair of 503 x 504 x 500 from 96 views of 513 x 517: 11.7 -> 6.0 ms; FP16 pair of
-// 254 x 243 x 242 from 29 of 300 x 279: 912 -> 345 us; 74 x 61 x 60 from 12 of 70 x 67:
-// 43 -> 39).  Not while a graph is captured or without memory for it.
-constexpr double kPitchSave = 1e-12;  // seconds an update
-
+// slab with the matrices' own positions, where rules::pitched_copy_pays says so.  Not
+// while a graph is captured or without memory for it.
 template <int DT>
 bool launch_wave(fdk_bp* h, const BpArgs& a, const BpMats& M, const BpScale& S);
 
@@ -1574,8 +1589,8 @@ bool launch_wave_pitched(fdk_bp* h, const BpArgs& a, const BpMats& M, const BpSc
   const int pitch = (a.W + 4) & ~3;  // never W: tells a copy from the caller's own views
   const long long view = (long long)pitch * a.H;
   if (view * 2 >= (1LL << 31)) return false;
-  const double updates = (double)a.nxs * a.nys * a.nzz * a.nproj;
-  if (updates * kPitchSave < 3e-6 + (double)view * a.nproj * 4 / 1e12) return false;
+  if (!fdk::rules::pitched_copy_pays((double)a.nxs * a.nys, a.zext, h->sym ? 2 : 1, a.nproj, (double)view))
+    return false;
   hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
   if (hipStreamIsCapturing(h->stream, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone) {
     (void)hipGetLastError();
@@ -1612,14 +1627,11 @@ bool launch_wave(fdk_bp* h, const BpArgs& a, const BpMats& M, const BpScale& S) 
   const bool quads = a.W % 4 == 0 && a.pitch == a.W && (DT == FDK_F32 || (reinterpret_cast<uintptr_t>(a.proj) % 8 == 0 &&
                                                         a.view_stride % 4 == 0));
   if (h->sym && quads && mirror_symmetric(a, M)) return launch_wave_run<DT, true>(h, a, M, S, dvz);
-  if (!launch_wave_run<DT, false>(h, a, M, S, dvz)) return false;
-  if (h->sym) {  // the bottom slab as a run of its own
-    BpArgs b = a;
-    b.z0 = (int)h->bot.z;
-    b.vol = a.vol + a.zext;
-    return launch_wave_run<DT, false>(h, b, M, S, dvz);
-  }
-  return true;
+  // A strip staged for a single view is used once.  16-bit views: 512^3 from one of 512^2
+  // 266 us here, 215 by the block-strip kernel; FP32 rows off 4 samples: 256^3 pair 47.6,
+  // 41.8 by the gather kernel, but 512^3 pair 321 and 345, 300^3 54.5 and 64.5.
+  if (a.nproj == 1 && (DT != FDK_F32 || (a.W % 4 != 0 && (long long)a.nxs * a.nys < 80000))) return false;
+  return launch_wave_run<DT, false>(h, a, M, S, dvz);
 }
 
 template <int DT, int ZPT>

@@ -37,5 +37,19 @@ inline int wave_strip_columns(double dvz, int zpt, int sides) {
   return quads < 1e6 ? 4 * (int)quads + (sides == 2 ? 2 : 4) : 0;
 }
 
+// Whether 16-bit views with odd rows are worth copying to rows of a multiple of 4
+// samples, so that bp_wave_kernel takes them: columns of zext voxels in `slabs` slabs,
+// `nproj` views of `view` samples.  Per view and slab the gather kernel takes about
+// 0.5 us + 0.18 ns a wave more than nothing, the wave-strip kernel half of the latter;
+// the copy, its event and launch cost 14 us, and 4 bytes a sample at about 1 TB/s.  FP16
+// cubes of n^3 from views of (n + 1)^2, gather against copy, us: 48, pair, 32 views 68 / 28;
+// 96, pair, 4 views 20.3 / 22.4, 8 views 36.8 / 27.9; 160, one slab, 3 views 21.6 / 24.7;
+// 256, pair, 4 views 134 / 85; 512, 32 views 3950 / 1650.  One view never pays (256: 31 / 41).
+inline bool pitched_copy_pays(double columns, int zext, int slabs, int nproj, double view) {
+  const double waves = columns * ((zext + 511) / 512);
+  const double save = (double)nproj * slabs * (0.5e-6 + 0.09e-9 * waves);
+  return nproj > 1 && save > 14e-6 + view * nproj * 4 / 1e12;
+}
+
 }  // namespace rules
 }  // namespace fdk

@@ -8,3 +8,7 @@ extern "C" int check_filter_form(int nu, int nrows, int nviews, int log_n, int t
 extern "C" int check_wave_strip_columns(double dvz, int zpt, int sides) {
   return fdk::rules::wave_strip_columns(dvz, zpt, sides);
 }
+
+extern "C" int check_pitched_copy_pays(double columns, int zext, int slabs, int nproj, double view) {
+  return fdk::rules::pitched_copy_pays(columns, zext, slabs, nproj, view);
+}
