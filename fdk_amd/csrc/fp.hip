@@ -21,6 +21,7 @@
 #include <vector>
 
 #include "common.hpp"
+#include "launch_rules.hpp"
 
 namespace {
 
@@ -464,26 +465,16 @@ int upload_ell(const fdk_ellipsoid* host, int n, hipStream_t st, EllDev** out) {
   return FDK_OK;
 }
 
-// Seconds fp_kernel takes for a view's samples more than fp_zfast_kernel would.  Its
-// lanes step along u, so |sin a| of a voxel row apart: a gather costs it from one
-// line (rays along y) to a line a lane (rays along x).  Measured through 256^3: 2 ps a
-// sample at 0 degrees, 10 ps at 90, 7.4 ps averaged over a scan; fp_zfast_kernel
-// takes 1.2 ps at every angle.
-double zfast_saving(const RayGeom& r, int count, double step) {
-  const double diag = std::hypot(r.nx * r.vx, r.ny * r.vy);
-  const double samples = (double)r.nu * r.nv * 0.6 * diag / step;  // a view's, about
-  double ps = 0.0;
+bool zfast_pays(const RayGeom& r, int count, double step, double copy_bytes) {
+  fdk::rules::March m{r.nu, r.nv, r.cv, r.dv, r.sid / r.sod, r.nx, r.ny, r.nz, r.vx, r.vy, r.vz, step, count, 0.0, 0.0};
   for (int k = 0; k < count; ++k) {
     const double a = r.direction * ((r.first + k) * r.scan_deg / r.nproj) / 180.0 * kPi + r.vpa;
-    ps += 2.0 + 8.0 * std::fabs(std::sin(a)) - 1.2;
+    const double s = std::fabs(std::sin(a));
+    m.sum_sin += s;
+    m.max_sin = std::fmax(m.max_sin, s);
   }
-  return samples * ps * 1e-12;
+  return fdk::rules::zfast_pays(m, copy_bytes, (double)fdk::kScratchKeep);
 }
-
-// Seconds for the padded copy: 12 us for the second launch and the block's event, and
-// 12 bytes a voxel at 2.8 TB/s (75 us at 256^3).  One view at 0 degrees stays with
-// fp_kernel (256^3: 52 against 106 us), four round the scan do not (327 against 140).
-double zfast_cost(double voxels) { return 12e-6 + voxels * 12.0 / 2.8e12; }
 
 // Runs fp_zfast_kernel (and the padded copy it reads) where it pays; *done says
 // whether it did.  It does not while the stream is captured, where nothing is
@@ -492,14 +483,14 @@ int launch_zfast(const RayGeom& r, const float* vol, int count, float step, int 
                  hipStream_t st, bool* done) {
   *done = false;
   const long long mx = r.nx + 2 * kFpPad, my = r.ny + 2 * kFpPad, mz = r.nz + 2 * kFpPad;
-  if (zfast_saving(r, count, step) < 1.2 * zfast_cost((double)mx * my * mz)) return FDK_OK;
+  const size_t bytes = (size_t)(mx * my * mz) * sizeof(float2);
+  if (!zfast_pays(r, count, step, (double)bytes)) return FDK_OK;
   if (my > 65535) return FDK_OK;  // grid z of the copy
   hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
   if (hipStreamIsCapturing(st, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone) {
     (void)hipGetLastError();
     return FDK_OK;
   }
-  const size_t bytes = (size_t)(mx * my * mz) * sizeof(float2);
   const long long bv = (r.nv + 63) / 64, bu = (r.nu + 3) / 4, blocks = bv * bu * count;
   if (blocks > (1LL << 22)) return FDK_OK;  // 2^30 threads
   fdk::Scratch ws;

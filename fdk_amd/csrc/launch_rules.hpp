@@ -51,5 +51,43 @@ inline bool pitched_copy_pays(double columns, int zext, int slabs, int nproj, do
   return nproj > 1 && save > 14e-6 + view * nproj * 4 / 1e12;
 }
 
+// Which march of the forward projector is the faster: fp_kernel through the volume
+// itself or fp_zfast_kernel through its padded copy.
+struct March {
+  int nu, nv;               // detector, pitch dv, the volume's mid plane on row cv
+  double cv, dv, mag;       // magnification of the volume's centre
+  int nx, ny, nz;
+  double vx, vy, vz, step;  // mm
+  int views;
+  double sum_sin, max_sin;  // of |sin angle| over the views
+};
+
+// fp_zfast_kernel's waves are 64 rows of a column, and cost what 64 rays do however many
+// of them are on the detector and meet the volume: 0.95 ps a lane and sample, at least
+// 0.15 us a sample of a ray (its samples are a chain), plus 16 us and 12 bytes a voxel at
+// 2.8 TB/s for the copy.  A copy above what the scratch list keeps is mapped for the call:
+// 17 to 56 ms a GB where the caller waits between calls.  fp_kernel's waves are 64 columns
+// of a row: 0.7 ps a lane and sample where rays run along y to 7.4 where they run along x,
+// its chain 0.13 to 0.39 us a sample, more in rows over 256 voxels.  The constants give
+// fp_kernel where it measured faster, at 400 sizes, to 5 % or 2 us.  Measured, 256^3 at
+// half-voxel steps, fp_kernel / fp_zfast_kernel: 24 views of 256 x 64 round the scan 1216 /
+// 260 us, 60 of 256 x 16 686 / 524, 360 of 256 x 8 1902 / 2400, 360 of 256 x 1 268 / 2400,
+// 2 of 256 x 200 near 0 degrees 124 / 152; 80^3 at whole steps, 4 views 19.4 / 29.6.
+inline bool zfast_pays(const March& m, double copy_bytes, double kept_bytes) {
+  const double across = std::sqrt(m.nx * m.vx * m.nx * m.vx + m.ny * m.vy * m.ny * m.vy);
+  const double samples = 0.6 * across / m.step;  // a ray's, about
+  const double shadow = 0.6 * m.nz * m.vz * m.mag / m.dv + 1;  // half the volume's height in rows
+  const double r0 = std::fmax(0.0, m.cv + 0.5 - shadow), r1 = std::fmin((double)m.nv, m.cv + 0.5 + shadow);
+  if (!(r1 - r0 >= 16)) return false;
+  const double waves = (std::ceil(r1 / 64) - std::floor(r0 / 64)) * m.nu;
+  const double rays = (r1 - r0) * 64 * std::ceil(m.nu / 64.0);
+  const double direct = std::fmax(
+      samples * rays * (0.7e-12 * m.views + 6.7e-12 * m.sum_sin),
+      samples * (0.13e-6 + 0.26e-6 * std::fmax(1.0, m.nx / 256.0) * std::fmin(1.0, 1.3 * m.max_sin)));
+  const double copy = 16e-6 + copy_bytes * 1.5 / 2.8e12 + (copy_bytes > kept_bytes ? copy_bytes * 60e-12 : 0.0);
+  const double zfast = copy + samples * std::fmax(0.15e-6, 64 * 0.95e-12 * waves * m.views);
+  return direct > 1.05 * zfast;
+}
+
 }  // namespace rules
 }  // namespace fdk

@@ -12,3 +12,9 @@ extern "C" int check_wave_strip_columns(double dvz, int zpt, int sides) {
 extern "C" int check_pitched_copy_pays(double columns, int zext, int slabs, int nproj, double view) {
   return fdk::rules::pitched_copy_pays(columns, zext, slabs, nproj, view);
 }
+
+extern "C" int check_zfast_pays(int nu, int nv, double cv, double dv, int nx, int nz, double voxel, double step,
+                                int views, double sum_sin, double max_sin) {
+  const fdk::rules::March m{nu, nv, cv, dv, 1.5, nx, nx, nz, voxel, voxel, voxel, step, views, sum_sin, max_sin};
+  return fdk::rules::zfast_pays(m, 8.0 * (nx + 4) * (nx + 4) * (nz + 4), 512.0 * 1024 * 1024);
+}
