@@ -491,8 +491,9 @@ int launch_zfast(const RayGeom& r, const float* vol, int count, float step, int 
     (void)hipGetLastError();
     return FDK_OK;
   }
-  const long long bv = (r.nv + 63) / 64, bu = (r.nu + 3) / 4, blocks = bv * bu * count;
-  if (blocks > (1LL << 22)) return FDK_OK;  // 2^30 threads
+  // views a launch takes: 2^22 blocks, 2^30 threads
+  const long long bv = (r.nv + 63) / 64, bu = (r.nu + 3) / 4, most = (1LL << 22) / (bv * bu);
+  if (most == 0) return FDK_OK;
   fdk::Scratch ws;
   if (fdk::scratch_get(&ws, bytes, st) != FDK_OK) return FDK_OK;
   float2* pad = static_cast<float2*>(ws.p);
@@ -501,17 +502,17 @@ int launch_zfast(const RayGeom& r, const float* vol, int count, float step, int 
     hipLaunchKernelGGL((fp_pad_kernel<FDK_FP_CLAMP>), pg, dim3(32, 8), 0, st, vol, pad, r.nx, r.ny, r.nz);
   else
     hipLaunchKernelGGL((fp_pad_kernel<FDK_FP_ZERO>), pg, dim3(32, 8), 0, st, vol, pad, r.nx, r.ny, r.nz);
-  const dim3 grid((unsigned)((blocks + 7) / 8 * 8));
   const bool buf = bytes < (1ull << 31) && mx * my < (1LL << 23) && mz < (1LL << 23);
   const int nb = buf ? (int)bytes : 0, nbv = (int)bv, nbu = (int)bu;
-  if (mode == FDK_FP_CLAMP && buf)
-    hipLaunchKernelGGL((fp_zfast_kernel<FDK_FP_CLAMP, true>), grid, dim3(64, 4), 0, st, r, pad, nb, step, nbv, nbu, blocks, out);
-  else if (mode == FDK_FP_CLAMP)
-    hipLaunchKernelGGL((fp_zfast_kernel<FDK_FP_CLAMP, false>), grid, dim3(64, 4), 0, st, r, pad, nb, step, nbv, nbu, blocks, out);
-  else if (buf)
-    hipLaunchKernelGGL((fp_zfast_kernel<FDK_FP_ZERO, true>), grid, dim3(64, 4), 0, st, r, pad, nb, step, nbv, nbu, blocks, out);
-  else
-    hipLaunchKernelGGL((fp_zfast_kernel<FDK_FP_ZERO, false>), grid, dim3(64, 4), 0, st, r, pad, nb, step, nbv, nbu, blocks, out);
+  const auto march = mode == FDK_FP_CLAMP ? (buf ? fp_zfast_kernel<FDK_FP_CLAMP, true> : fp_zfast_kernel<FDK_FP_CLAMP, false>)
+                                          : (buf ? fp_zfast_kernel<FDK_FP_ZERO, true> : fp_zfast_kernel<FDK_FP_ZERO, false>);
+  RayGeom run = r;
+  for (long long v = 0; v < count; v += most) {
+    const long long blocks = bv * bu * std::min(most, count - v);
+    run.first = r.first + (int)v;
+    hipLaunchKernelGGL(march, dim3((unsigned)((blocks + 7) / 8 * 8)), dim3(64, 4), 0, st, run, pad, nb, step, nbv,
+                       nbu, blocks, out + v * r.nv * r.nu);
+  }
   const hipError_t e = hipGetLastError();
   fdk::scratch_put(&ws, st);
   if (e != hipSuccess) return fdk::fail(FDK_ERR_HIP, "forward projection: %s", hipGetErrorString(e));
