@@ -58,6 +58,16 @@ __device__ inline void pixel_ray(const RayGeom& g, int s, int i, int j, double o
   d[0] *= n; d[1] *= n; d[2] *= n;
 }
 
+// t<z><y><x>, blended along x, y, z.  Both marches form it, so that a ray's sum does not
+// depend on which one a call takes.
+__device__ __forceinline__ float trilinear(float t000, float t001, float t010, float t011, float t100,
+                                           float t101, float t110, float t111, float fx, float fy, float fz) {
+  const float gx = 1.f - fx, gy = 1.f - fy;
+  const float v0 = (t000 * gx + t001 * fx) * gy + (t010 * gx + t011 * fx) * fy;
+  const float v1 = (t100 * gx + t101 * fx) * gy + (t110 * gx + t111 * fx) * fy;
+  return v0 * (1.f - fz) + v1 * fz;
+}
+
 template <int MODE>
 __device__ inline float tap_sample(const float* __restrict__ vol, int nx, int ny, int nz, float px,
                                    float py, float pz) {
@@ -85,10 +95,7 @@ __device__ inline float tap_sample(const float* __restrict__ vol, int nx, int ny
   const float t010 = vol[r01 + x0] * (mx0 * my1 * mz0), t011 = vol[r01 + x1] * (mx1 * my1 * mz0);
   const float t100 = vol[r10 + x0] * (mx0 * my0 * mz1), t101 = vol[r10 + x1] * (mx1 * my0 * mz1);
   const float t110 = vol[r11 + x0] * (mx0 * my1 * mz1), t111 = vol[r11 + x1] * (mx1 * my1 * mz1);
-  const float gx = 1.f - fx, gy = 1.f - fy;
-  const float v0 = (t000 * gx + t001 * fx) * gy + (t010 * gx + t011 * fx) * fy;
-  const float v1 = (t100 * gx + t101 * fx) * gy + (t110 * gx + t111 * fx) * fy;
-  return v0 * (1.f - fz) + v1 * fz;
+  return trilinear(t000, t001, t010, t011, t100, t101, t110, t111, fx, fy, fz);
 }
 
 // tap_sample through a buffer resource over the volume (32-bit offsets, for
@@ -144,10 +151,7 @@ __device__ inline float tap_blend(const TapBuf& b) {
   const float t101 = (b.s1 ? b.q[2].y : b.q[2].x) * (b.mx1 * b.my0 * b.mz1);
   const float t110 = (b.s0 ? b.q[3].y : b.q[3].x) * (b.mx0 * b.my1 * b.mz1);
   const float t111 = (b.s1 ? b.q[3].y : b.q[3].x) * (b.mx1 * b.my1 * b.mz1);
-  const float gx = 1.f - b.fx, gy = 1.f - b.fy;
-  const float v0 = (t000 * gx + t001 * b.fx) * gy + (t010 * gx + t011 * b.fx) * b.fy;
-  const float v1 = (t100 * gx + t101 * b.fx) * gy + (t110 * gx + t111 * b.fx) * b.fy;
-  return v0 * (1.f - b.fz) + v1 * b.fz;
+  return trilinear(t000, t001, t010, t011, t100, t101, t110, t111, b.fx, b.fy, b.fz);
 }
 
 // The ray of a pixel in voxel coordinates, o + t s with t in mm, and the part of it
@@ -230,8 +234,9 @@ __global__ __launch_bounds__(256) void fp_kernel(RayGeom g, const float* __restr
 // every step, whatever the view angle, and 64 neighbouring z of them, so a tap load
 // reads one run of about 70 voxels.  (Lanes along u, as in fp_kernel, step across the
 // volume's rows: one cache line a lane where the rays run along x.)  The pads hold
-// what the edge mode asks for -- the edge voxel, or zero -- so no tap is clamped,
-// selected or masked; indices past the pads are clamped into them.
+// what the edge mode asks for -- the edge voxel, or the edge voxel times zero, as the
+// masked taps of fp_kernel -- so no tap is clamped, selected or masked; indices past the
+// pads are clamped into them.  The sums equal fp_kernel's to the bit.
 //
 // What bounds it: the texture-address unit, which takes 16 clocks for a wave's
 // gather whether a lane asks for 4, 8 or (nearly) 16 bytes (busy 91 % of the time
@@ -239,7 +244,7 @@ __global__ __launch_bounds__(256) void fp_kernel(RayGeom g, const float* __restr
 // voxel beside its y neighbour and one 16-byte gather brings four of the eight taps:
 // two gathers a sample.
 // Measured, 24 views of 256^2 through 256^3 at half-voxel steps: 5.10 ms (fp_kernel)
-// -> 1.38 (8-byte gathers) -> 0.78 ms, 830 Gsamples/s, copy included.  Splitting the rays over
+// -> 1.38 (8-byte gathers) -> 0.79 ms, 820 Gsamples/s, copy included.  Splitting the rays over
 // 4 or 16 waves for launches with few of them gained nothing (8 views: 313 against
 // 230 us).
 constexpr int kFpPad = 2;
@@ -260,7 +265,7 @@ __global__ __launch_bounds__(256) void fp_pad_kernel(const float* __restrict__ v
       const int x = x0 + (int)threadIdx.x - kFpPad, z = z0 + k - kFpPad;
       const int cx = min(max(x, 0), nx - 1), cz = min(max(z, 0), nz - 1);
       const float v = vol[((long long)cz * ny + cy) * nx + cx];
-      t[h][k][threadIdx.x] = MODE == FDK_FP_CLAMP || (cx == x && cy == y && cz == z) ? v : 0.f;
+      t[h][k][threadIdx.x] = MODE == FDK_FP_CLAMP || (cx == x && cy == y && cz == z) ? v : v * 0.f;
     }
   }
   __syncthreads();
@@ -308,13 +313,9 @@ __device__ __forceinline__ TapZ tap_fetch_z(__amdgpu_buffer_rsrc_t rv, const flo
   return b;
 }
 
-__device__ __forceinline__ float lerp(float a, float b, float t) { return fmaf(t, b - a, a); }
-
 __device__ __forceinline__ float tap_blend_z(const TapZ& b) {
   const float4 a = b.q[0], c = b.q[1];
-  const float v0 = lerp(lerp(a.x, c.x, b.fx), lerp(a.y, c.y, b.fx), b.fy);
-  const float v1 = lerp(lerp(a.z, c.z, b.fx), lerp(a.w, c.w, b.fx), b.fy);
-  return lerp(v0, v1, b.fz);
+  return trilinear(a.x, c.x, a.y, c.y, a.z, c.z, a.w, c.w, b.fx, b.fy, b.fz);
 }
 
 // Grid: x = blocks in the order v, u, view, rounded up to a multiple of 8 and
