@@ -4,8 +4,9 @@
 #include <cstring>
 #include <map>
 #include <mutex>
+#include <new>
 #include <string>
-#include <vector>
+#include <utility>
 
 #include "common.hpp"
 
@@ -66,97 +67,137 @@ struct Relaxed {
   ~Relaxed() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
 };
 
+// A device's blocks: those not in use, and the bytes of all of them.
+struct ScratchList {
+  ScratchBlock* idle = nullptr;
+  size_t total = 0;
+};
+constexpr int kScratchDevices = 64;
 std::mutex g_scratch_mutex;
-std::map<int, std::vector<Scratch>> g_scratch;  // kept blocks, by device
+ScratchList g_scratch[kScratchDevices];
 
-void scratch_free(Scratch& s) {
+// Frees blocks no longer on a list, waiting for the work behind them.
+void scratch_free(ScratchBlock* b) {
   Relaxed relaxed;
-  (void)hipEventSynchronize(s.done);
-  (void)hipFree(s.p);
-  (void)hipEventDestroy(s.done);
+  while (b) {
+    ScratchBlock* next = b->next;
+    (void)hipEventSynchronize(b->done);
+    (void)hipFree(b->p);
+    (void)hipEventDestroy(b->done);
+    delete b;
+    b = next;
+  }
   (void)hipGetLastError();
-  s = Scratch{};
 }
 
-// The current device's kept blocks, taken off the list.
-std::vector<Scratch> scratch_take_all() {
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess) return {};
-  std::lock_guard<std::mutex> lock(g_scratch_mutex);
-  std::vector<Scratch> v;
-  v.swap(g_scratch[dev]);
-  return v;
+// Takes off the list what is needed of the idle blocks whose work is done, smallest
+// first, so that `bytes` more fit the limit; nothing if they would not make room.
+ScratchBlock* scratch_make_room(ScratchList& l, size_t bytes) {
+  size_t done = 0;
+  for (ScratchBlock* b = l.idle; b; b = b->next) {
+    b->ready = hipEventQuery(b->done) == hipSuccess;
+    if (b->ready) done += b->bytes;
+  }
+  (void)hipGetLastError();
+  ScratchBlock* out = nullptr;
+  if (l.total - done + bytes > kScratchKeep) return out;
+  while (l.total + bytes > kScratchKeep) {
+    ScratchBlock** least = nullptr;
+    for (ScratchBlock** q = &l.idle; *q; q = &(*q)->next)
+      if ((*q)->ready && (!least || (*q)->bytes < (*least)->bytes)) least = q;
+    ScratchBlock* b = *least;
+    *least = b->next;
+    l.total -= b->bytes;
+    b->next = out;
+    out = b;
+  }
+  return out;
 }
 
 }  // namespace
 
 void scratch_trim() {
-  for (Scratch& s : scratch_take_all()) scratch_free(s);
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev >= kScratchDevices) return;
+  ScratchBlock* b = nullptr;
+  {
+    std::lock_guard<std::mutex> lock(g_scratch_mutex);
+    std::swap(b, g_scratch[dev].idle);
+    for (ScratchBlock* q = b; q; q = q->next) g_scratch[dev].total -= q->bytes;
+  }
+  scratch_free(b);
 }
 
 int scratch_get(Scratch* s, size_t bytes, hipStream_t st) {
   *s = Scratch{};
   int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess) return FDK_ERR_HIP;
-  if (bytes > kScratchKeep) {
-    s->bytes = bytes;
-    if (hipMallocAsync(&s->p, bytes, st) == hipSuccess) return FDK_OK;
-    (void)hipGetLastError();
-    *s = Scratch{};
-    return FDK_ERR_OOM;
-  }
-  {
+  if (hipGetDevice(&dev) != hipSuccess || dev >= kScratchDevices) return FDK_ERR_HIP;
+  const size_t size = (bytes + (2u << 20) - 1) >> 21 << 21;
+  ScratchBlock *b = nullptr, *old = nullptr;
+  bool make = false;
+  if (size <= kScratchKeep) {
     std::lock_guard<std::mutex> lock(g_scratch_mutex);
-    std::vector<Scratch>& v = g_scratch[dev];
-    size_t best = v.size();
-    for (size_t k = 0; k < v.size(); ++k)
-      if (v[k].bytes >= bytes && (best == v.size() || v[k].bytes < v[best].bytes)) best = k;
-    if (best < v.size()) {
-      *s = v[best];
-      v.erase(v.begin() + (long)best);
+    ScratchList& l = g_scratch[dev];
+    ScratchBlock** best = nullptr;
+    for (ScratchBlock** q = &l.idle; *q; q = &(*q)->next)
+      if ((*q)->bytes >= bytes && (!best || (*q)->bytes < (*best)->bytes)) best = q;
+    if (best) {
+      b = *best;
+      *best = b->next;
+    } else {
+      if (l.total + size > kScratchKeep) old = scratch_make_room(l, size);
+      make = l.total + size <= kScratchKeep;
+      if (make) l.total += size;
     }
   }
-  if (s->p) {
-    if (hipStreamWaitEvent(st, s->done, 0) == hipSuccess) return FDK_OK;
-    scratch_free(*s);  // waits for the block's last work instead
+  if (b) {
+    if (hipStreamWaitEvent(st, b->done, 0) == hipSuccess) {
+      s->p = b->p;
+      s->block = b;
+      return FDK_OK;
+    }
+    (void)hipGetLastError();
+    std::lock_guard<std::mutex> lock(g_scratch_mutex);
+    b->next = g_scratch[dev].idle;
+    g_scratch[dev].idle = b;
+    return FDK_ERR_OOM;
   }
-  scratch_trim();  // a larger block replaces the kept ones
-  Relaxed relaxed;
-  s->bytes = (bytes + (2u << 20) - 1) >> 21 << 21;
-  if (hipEventCreateWithFlags(&s->done, hipEventDisableTiming) == hipSuccess) {
-    if (hipMalloc(&s->p, s->bytes) == hipSuccess) return FDK_OK;
-    (void)hipEventDestroy(s->done);
+  scratch_free(old);
+  if (make) {
+    Relaxed relaxed;
+    b = new (std::nothrow) ScratchBlock;
+    if (b && hipEventCreateWithFlags(&b->done, hipEventDisableTiming) == hipSuccess) {
+      if (hipMalloc(&b->p, size) == hipSuccess) {
+        b->bytes = size;
+        b->device = dev;
+        s->p = b->p;
+        s->block = b;
+        return FDK_OK;
+      }
+      (void)hipEventDestroy(b->done);
+    }
+    (void)hipGetLastError();
+    delete b;
+    std::lock_guard<std::mutex> lock(g_scratch_mutex);
+    g_scratch[dev].total -= size;
+    return FDK_ERR_OOM;
   }
+  if (hipMallocAsync(&s->p, bytes, st) == hipSuccess) return FDK_OK;
   (void)hipGetLastError();
   *s = Scratch{};
   return FDK_ERR_OOM;
 }
 
 void scratch_put(Scratch* s, hipStream_t st) {
-  if (!s->p) return;
-  if (!s->done) {
-    (void)hipFreeAsync(s->p, st);
-    *s = Scratch{};
-    return;
-  }
-  int dev = 0;
-  if (hipEventRecord(s->done, st) != hipSuccess || hipGetDevice(&dev) != hipSuccess) {
-    (void)hipStreamSynchronize(st);
-    scratch_free(*s);
-    return;
-  }
-  {
-    std::lock_guard<std::mutex> lock(g_scratch_mutex);
-    std::vector<Scratch>& v = g_scratch[dev];
-    size_t kept = s->bytes;
-    for (const Scratch& q : v) kept += q.bytes;
-    if (kept <= kScratchKeep) {
-      v.push_back(*s);
-      *s = Scratch{};
-      return;
-    }
-  }
-  scratch_free(*s);
+  ScratchBlock* b = s->block;
+  if (s->p && !b) (void)hipFreeAsync(s->p, st);
+  *s = Scratch{};
+  if (!b) return;
+  const bool behind = hipEventRecord(b->done, st) == hipSuccess;
+  if (!behind) (void)hipStreamSynchronize(st);
+  std::lock_guard<std::mutex> lock(g_scratch_mutex);
+  b->next = g_scratch[b->device].idle;
+  g_scratch[b->device].idle = b;
 }
 
 }  // namespace fdk

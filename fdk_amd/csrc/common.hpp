@@ -27,17 +27,26 @@ int fail(int code, const char* fmt, ...) __attribute__((format(printf, 2, 3)));
 // not on every call.
 int stage_alloc(void** p, size_t bytes, hipStream_t st);
 
-// Device memory a call needs only while its kernels run.  scratch_get takes it from a
-// list of blocks kept per device (at most kScratchKeep bytes of them; larger requests
-// are stream-ordered allocations, gone when the call's work is) and scratch_put gives
-// it back behind the work queued on `st`: the next user's stream waits for that work,
-// so blocks pass between streams and threads.  Not for streams being captured.
-// scratch_get returns FDK_ERR_OOM without a last-error message: the caller does
-// without.  scratch_trim frees the kept blocks of the current device.
-struct Scratch {
+// Device memory a call needs only while its kernels run.  scratch_get takes it from
+// blocks kept per device, at most kScratchKeep bytes of them in use and idle, and
+// scratch_put gives it back behind the work queued on `st`: the next user's stream waits
+// for that work, so blocks pass between streams and threads.  Neither waits on the host;
+// but a request larger than every idle block frees those whose work is done where that
+// makes room, and hipFree waits for the device: once as sizes grow.  Requests past the
+// limit are stream-ordered allocations, gone when the call's work is.  Not for streams
+// being captured.  scratch_get returns FDK_ERR_OOM without a last-error message: the
+// caller does without.  scratch_trim frees the idle blocks of the current device.
+struct ScratchBlock {
   void* p = nullptr;
   size_t bytes = 0;
-  hipEvent_t done = nullptr;  // null: a stream-ordered allocation
+  hipEvent_t done = nullptr;  // behind the last user's work
+  ScratchBlock* next = nullptr;
+  int device = 0;
+  bool ready = false;
+};
+struct Scratch {
+  void* p = nullptr;
+  ScratchBlock* block = nullptr;  // null: a stream-ordered allocation
 };
 constexpr size_t kScratchKeep = 512u << 20;
 int scratch_get(Scratch* s, size_t bytes, hipStream_t st);
