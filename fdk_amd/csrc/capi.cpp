@@ -67,6 +67,18 @@ struct Relaxed {
   ~Relaxed() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
 };
 
+// The device that memory and events are made on, the caller's afterwards.
+struct OnDevice {
+  int before = -1;
+  explicit OnDevice(int dev) {
+    int now = dev;
+    if (hipGetDevice(&now) == hipSuccess && now != dev && hipSetDevice(dev) == hipSuccess) before = now;
+  }
+  ~OnDevice() {
+    if (before >= 0) (void)hipSetDevice(before);
+  }
+};
+
 // A device's blocks: those not in use, and the bytes of all of them.
 struct ScratchList {
   ScratchBlock* idle = nullptr;
@@ -131,7 +143,11 @@ void scratch_trim() {
 int scratch_get(Scratch* s, size_t bytes, hipStream_t st) {
   *s = Scratch{};
   int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev >= kScratchDevices) return FDK_ERR_HIP;
+  if (hipStreamGetDevice(st, &dev) != hipSuccess || dev >= kScratchDevices) {
+    (void)hipGetLastError();
+    return FDK_ERR_OOM;
+  }
+  OnDevice here(dev);
   const size_t size = (bytes + (2u << 20) - 1) >> 21 << 21;
   ScratchBlock *b = nullptr, *old = nullptr;
   bool make = false;

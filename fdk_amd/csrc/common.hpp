@@ -27,15 +27,15 @@ int fail(int code, const char* fmt, ...) __attribute__((format(printf, 2, 3)));
 // not on every call.
 int stage_alloc(void** p, size_t bytes, hipStream_t st);
 
-// Device memory a call needs only while its kernels run.  scratch_get takes it from
-// blocks kept per device, at most kScratchKeep bytes of them in use and idle, and
-// scratch_put gives it back behind the work queued on `st`: the next user's stream waits
-// for that work, so blocks pass between streams and threads.  Neither waits on the host;
-// but a request larger than every idle block frees those whose work is done where that
-// makes room, and hipFree waits for the device: once as sizes grow.  Requests past the
-// limit are stream-ordered allocations, gone when the call's work is.  Not for streams
-// being captured.  scratch_get returns FDK_ERR_OOM without a last-error message: the
-// caller does without.  scratch_trim frees the idle blocks of the current device.
+// Device memory a call needs only while its kernels run, on the stream's device.
+// scratch_get takes it from blocks kept per device, at most kScratchKeep bytes of them in
+// use and idle, and scratch_put gives it back behind the work queued on `st`: the next
+// user's stream waits for that work, so blocks pass between streams and threads.  Neither
+// waits on the host; but a request larger than every idle block frees those whose work is
+// done where that makes room, and hipFree waits for the device: once as sizes grow.
+// Requests past the limit are stream-ordered allocations, gone when the call's work is.
+// Not for streams being captured.  scratch_get returns FDK_ERR_OOM without a last-error
+// message: the caller does without.  scratch_trim frees the current device's idle blocks.
 struct ScratchBlock {
   void* p = nullptr;
   size_t bytes = 0;
