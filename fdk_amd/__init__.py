@@ -62,6 +62,7 @@ _lib = None
 _SIGS = {
     "fdk_last_error": (C.c_int, [C.c_char_p, C.c_size_t]),
     "fdk_version": (C.c_int, []),
+    "fdk_release_scratch": (C.c_int, []),
     "fdk_device_count": (C.c_int, []),
     "fdk_geom_angular_ramp_factor": (C.c_int, [C.c_void_p, C.c_void_p]),
     "fdk_geom_cos_table": (C.c_int, [C.c_void_p, C.c_void_p]),
@@ -169,6 +170,12 @@ def _check(rc: int, what: str) -> int:
     if rc < 0:
         raise FdkError(f"{what}: {last_error()} (status {rc})")
     return rc
+
+
+def release_scratch() -> None:
+    """Frees the device memory the library keeps between calls on the current device (at
+    most 512 MiB), for a program whose own allocations fail."""
+    _check(lib().fdk_release_scratch(), "release_scratch")
 
 
 def _np_ptr(a: np.ndarray):

@@ -1733,15 +1733,10 @@ extern "C" int fdk_bp_create(int proj_width, int proj_height, int proj_count, in
   h->nzz = (int)(h->top.d + (h->sym ? h->bot.d : 0));
   (void)hipGetDevice(&h->device);
   const size_t nvox = (size_t)h->top.w * h->top.h * h->nzz;
-  hipError_t e = hipMalloc(&h->vol, nvox * sizeof(float));
-  if (e == hipErrorOutOfMemory) {  // once more with the library's scratch given back
-    (void)hipGetLastError();
-    fdk::scratch_trim();
-    e = hipMalloc(&h->vol, nvox * sizeof(float));
-  }
+  hipError_t e = fdk::dev_malloc((void**)&h->vol, nvox * sizeof(float));
   if (e == hipSuccess) e = hipMemset(h->vol, 0, nvox * sizeof(float));
   h->staging_elems = (size_t)proj_width * proj_height * proj_count;
-  if (e == hipSuccess) e = hipMalloc(&h->staging, h->staging_elems * sizeof(float));
+  if (e == hipSuccess) e = fdk::dev_malloc((void**)&h->staging, h->staging_elems * sizeof(float));
   if (e == hipSuccess) e = hipStreamCreateWithFlags(&h->stream, hipStreamNonBlocking);
   if (e == hipSuccess) h->own_stream = true;
   if (e == hipSuccess) e = hipEventCreate(&h->ev0);
@@ -1797,7 +1792,7 @@ extern "C" int fdk_bp_batch(fdk_bp_t h, int transpose, const float* host_proj, i
     FDK_HIP(hipMemcpyAsync(h->staging, host_proj, view * nproj * sizeof(float),
                            hipMemcpyHostToDevice, h->stream));
   } else {
-    if (!h->staging_t) FDK_HIP(hipMalloc(&h->staging_t, h->staging_elems * sizeof(float)));
+    if (!h->staging_t) FDK_HIP(fdk::dev_malloc((void**)&h->staging_t, h->staging_elems * sizeof(float)));
     FDK_HIP(hipMemcpyAsync(h->staging_t, host_proj, view * nproj * sizeof(float),
                            hipMemcpyHostToDevice, h->stream));
     if (int r = launch_transpose(h->staging_t, h->staging, height, width, nproj, view, view, h->stream))
@@ -1888,7 +1883,7 @@ int volume_out(fdk_bp* h, float* dst, size_t count, bool device_dst) {
   int chunk = (int)std::max<size_t>(1, std::min<size_t>(h->nzz, (256u << 20) / (plane * 4)));
   if (chunk >= 4 && chunk < h->nzz) chunk -= chunk % 4;  // whole 16-byte groups of planes
   float* tmp = nullptr;
-  FDK_HIP(hipMalloc(&tmp, plane * chunk * sizeof(float)));
+  FDK_HIP(fdk::dev_malloc((void**)&tmp, plane * chunk * sizeof(float)));
   int rc = FDK_OK;
   for (int z = 0; z < h->nzz && rc == FDK_OK; z += chunk) {
     const int nzc = std::min(chunk, h->nzz - z);
@@ -2129,11 +2124,11 @@ extern "C" int fdk_rtk_create(int proj_width, int proj_height, int proj_count, i
   FDK_REQUIRE(nx > 0 && ny > 0 && nz > 0, "bad volume size");
   fdk_rtk* h = new fdk_rtk{proj_width, proj_height, proj_count, nx, ny, nz};
   const size_t nvox = (size_t)nx * ny * nz;
-  hipError_t e = hipMalloc(&h->vin, nvox * 4);
-  if (e == hipSuccess) e = hipMalloc(&h->vout, nvox * 4);
+  hipError_t e = fdk::dev_malloc((void**)&h->vin, nvox * 4);
+  if (e == hipSuccess) e = fdk::dev_malloc((void**)&h->vout, nvox * 4);
   if (e == hipSuccess) e = hipMemset(h->vin, 0, nvox * 4);
   if (e == hipSuccess) e = hipMemset(h->vout, 0, nvox * 4);
-  if (e == hipSuccess) e = hipMalloc(&h->staging, (size_t)proj_width * proj_height * proj_count * 4);
+  if (e == hipSuccess) e = fdk::dev_malloc((void**)&h->staging, (size_t)proj_width * proj_height * proj_count * 4);
   if (e == hipSuccess) e = hipStreamCreateWithFlags(&h->stream, hipStreamNonBlocking);
   if (e == hipSuccess) e = hipEventCreate(&h->ev0);
   if (e == hipSuccess) e = hipEventCreate(&h->ev1);
@@ -2201,7 +2196,7 @@ extern "C" int fdk_reconstruct_conebeam(const int proj_size[3], const int vol_si
   if (proj_on_device) return launch_rtk(proj_size, vol_size, mats, dev_vol_in, dev_vol_out, proj, st);
   const size_t bytes = (size_t)proj_size[0] * proj_size[1] * std::max(proj_size[2], 0) * 4;
   float* tmp = nullptr;
-  FDK_HIP(hipMalloc(&tmp, std::max<size_t>(bytes, 4)));
+  FDK_HIP(fdk::dev_malloc((void**)&tmp, std::max<size_t>(bytes, 4)));
   hipError_t e = hipMemcpyAsync(tmp, proj, bytes, hipMemcpyHostToDevice, st);
   int r = e == hipSuccess ? launch_rtk(proj_size, vol_size, mats, dev_vol_in, dev_vol_out, tmp, st)
                           : fdk::fail(FDK_ERR_HIP, "upload: %s", hipGetErrorString(e));

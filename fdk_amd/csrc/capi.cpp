@@ -53,7 +53,13 @@ int stage_alloc(void** p, size_t bytes, hipStream_t st) {
       pools[dev] = pool;
     }
   }
-  FDK_HIP(hipMallocFromPoolAsync(p, bytes, pool, st));
+  hipError_t e = hipMallocFromPoolAsync(p, bytes, pool, st);
+  if (e == hipErrorOutOfMemory) {
+    (void)hipGetLastError();
+    scratch_trim();
+    e = hipMallocFromPoolAsync(p, bytes, pool, st);
+  }
+  FDK_HIP(e);
   return FDK_OK;
 }
 
@@ -138,6 +144,14 @@ void scratch_trim() {
     for (ScratchBlock* q = b; q; q = q->next) g_scratch[dev].total -= q->bytes;
   }
   scratch_free(b);
+}
+
+hipError_t dev_malloc(void** p, size_t bytes) {
+  hipError_t e = hipMalloc(p, bytes);
+  if (e != hipErrorOutOfMemory) return e;
+  (void)hipGetLastError();
+  scratch_trim();
+  return hipMalloc(p, bytes);
 }
 
 int scratch_get(Scratch* s, size_t bytes, hipStream_t st) {
@@ -226,6 +240,11 @@ extern "C" int fdk_last_error(char* buf, size_t len) {
   return (int)g_last_error.size();
 }
 
+extern "C" int fdk_release_scratch(void) {
+  fdk::scratch_trim();
+  return FDK_OK;
+}
+
 extern "C" int fdk_version(void) { return 100; }
 
 extern "C" int fdk_device_count(void) {
@@ -240,7 +259,7 @@ extern "C" int fdk_dev_malloc(void** out, size_t bytes) {
   FDK_REQUIRE(out, "null output pointer");
   *out = nullptr;
   if (bytes == 0) return FDK_OK;
-  FDK_HIP(hipMalloc(out, bytes));
+  FDK_HIP(fdk::dev_malloc(out, bytes));
   return FDK_OK;
 }
 

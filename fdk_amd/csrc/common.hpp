@@ -53,6 +53,9 @@ int scratch_get(Scratch* s, size_t bytes, hipStream_t st);
 void scratch_put(Scratch* s, hipStream_t st);
 void scratch_trim();
 
+// hipMalloc, once more with the idle scratch blocks freed where memory is short.
+hipError_t dev_malloc(void** p, size_t bytes);
+
 }  // namespace fdk
 
 #define FDK_HIP(call)                                                                  \

@@ -1010,7 +1010,7 @@ int twiddles(int N, const float2** out) {
     return FDK_OK;
   }
   float2* d = nullptr;
-  FDK_HIP(hipMalloc(&d, sizeof(float2) * N));
+  FDK_HIP(fdk::dev_malloc((void**)&d, sizeof(float2) * N));
   hipStream_t st = nullptr;
   FDK_HIP(hipStreamCreateWithFlags(&st, hipStreamNonBlocking));
   launch_twiddles(d, N, st);
@@ -1290,10 +1290,10 @@ extern "C" int fdk_filter_proj_image(float* host_proj, int nu, int nv, int nview
   int r = FDK_OK;
   hipError_t e = hipEventCreate(&ev0);
   if (e == hipSuccess) e = hipEventCreate(&ev1);
-  if (e == hipSuccess) e = hipMalloc(&d, view * depth * sizeof(float));
-  if (e == hipSuccess) e = hipMalloc(&dH, sizeof(float) * N);
+  if (e == hipSuccess) e = fdk::dev_malloc((void**)&d, view * depth * sizeof(float));
+  if (e == hipSuccess) e = fdk::dev_malloc((void**)&dH, sizeof(float) * N);
   if (e == hipSuccess) e = hipMemcpy(dH, host_filter, sizeof(float) * N, hipMemcpyHostToDevice);
-  if (e == hipSuccess && host_cos) e = hipMalloc(&dcos, view * sizeof(float));
+  if (e == hipSuccess && host_cos) e = fdk::dev_malloc((void**)&dcos, view * sizeof(float));
   if (e == hipSuccess && host_cos) e = hipMemcpy(dcos, host_cos, view * sizeof(float), hipMemcpyHostToDevice);
   if (e != hipSuccess) r = fdk::fail(e == hipErrorOutOfMemory ? FDK_ERR_OOM : FDK_ERR_HIP, "FilterProjImage setup: %s", hipGetErrorString(e));
   // Each batch -- upload, cos weighting + filter, download -- is timed between
@@ -1333,10 +1333,10 @@ extern "C" int fdk_filter_frame_host(float* host_src, float* host_dst, int nu, i
   FDK_REQUIRE(nu > 0 && nv > 0, "bad image size");
   const size_t view = (size_t)nu * nv;
   float *s = nullptr, *d = nullptr, *c = nullptr, *h = nullptr;
-  hipError_t e = hipMalloc(&s, view * 4);
-  if (e == hipSuccess) e = hipMalloc(&d, view * 4);
-  if (e == hipSuccess) e = hipMalloc(&c, view * 4);
-  if (e == hipSuccess) e = hipMalloc(&h, sizeof(float) * std::max(N, 1));
+  hipError_t e = fdk::dev_malloc((void**)&s, view * 4);
+  if (e == hipSuccess) e = fdk::dev_malloc((void**)&d, view * 4);
+  if (e == hipSuccess) e = fdk::dev_malloc((void**)&c, view * 4);
+  if (e == hipSuccess) e = fdk::dev_malloc((void**)&h, sizeof(float) * std::max(N, 1));
   if (e == hipSuccess) e = hipMemcpy(s, host_src, view * 4, hipMemcpyHostToDevice);
   if (e == hipSuccess) e = hipMemcpy(c, host_cos, view * 4, hipMemcpyHostToDevice);
   if (e == hipSuccess) e = hipMemcpy(h, host_filter, sizeof(float) * N, hipMemcpyHostToDevice);

@@ -613,8 +613,8 @@ extern "C" int fdk_fp_project_host(const fdk_geometry* g, const float* host_vol,
   const size_t nvox = (size_t)g->nx * g->ny * g->nz;
   const size_t nout = (size_t)g->nu * g->nv * count;
   float *v = nullptr, *o = nullptr;
-  hipError_t e = hipMalloc(&v, std::max<size_t>(nvox, 1) * 4);
-  if (e == hipSuccess) e = hipMalloc(&o, std::max<size_t>(nout, 1) * 4);
+  hipError_t e = fdk::dev_malloc((void**)&v, std::max<size_t>(nvox, 1) * 4);
+  if (e == hipSuccess) e = fdk::dev_malloc((void**)&o, std::max<size_t>(nout, 1) * 4);
   if (e == hipSuccess) e = hipMemcpy(v, host_vol, nvox * 4, hipMemcpyHostToDevice);
   int r = e == hipSuccess ? FDK_OK : fdk::fail(FDK_ERR_HIP, "forward projection upload: %s", hipGetErrorString(e));
   if (r == FDK_OK) r = fdk_fp_project(g, v, first, count, step_mm, mode, o, nullptr);

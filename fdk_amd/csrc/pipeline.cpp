@@ -113,16 +113,16 @@ int setup(fdk_pipe* p, const fdk_geometry* g, const int64_t top[6], const int64_
   FDK_HIP(hipStreamCreateWithFlags(&p->compute, hipStreamNonBlocking));
   rc = fdk_bp_set_stream(p->bp, p->compute);
   if (rc < 0) return rc;
-  FDK_HIP(hipMalloc(&p->d_cos, cos.size() * sizeof(float)));
-  FDK_HIP(hipMalloc(&p->d_filter, hf.size() * sizeof(float)));
+  FDK_HIP(fdk::dev_malloc((void**)&p->d_cos, cos.size() * sizeof(float)));
+  FDK_HIP(fdk::dev_malloc((void**)&p->d_filter, hf.size() * sizeof(float)));
   FDK_HIP(hipMemcpy(p->d_cos, cos.data(), cos.size() * sizeof(float), hipMemcpyHostToDevice));
   FDK_HIP(hipMemcpy(p->d_filter, hf.data(), hf.size() * sizeof(float), hipMemcpyHostToDevice));
   p->slots.resize(nslots);
   const size_t store_bytes = FDK_BP_MAX_PROJ * p->view_elems * esize(p->store_dtype);
   for (auto& s : p->slots) {
-    FDK_HIP(hipMalloc(&s.store, store_bytes));
+    FDK_HIP(fdk::dev_malloc((void**)&s.store, store_bytes));
     if (p->store_dtype != FDK_F32)
-      FDK_HIP(hipMalloc((void**)&s.mm, 2 * FDK_BP_MAX_PROJ * sizeof(unsigned)));
+      FDK_HIP(fdk::dev_malloc((void**)&s.mm, 2 * FDK_BP_MAX_PROJ * sizeof(unsigned)));
     for (hipEvent_t* e : {&s.copied, &s.flt_start, &s.flt_end, &s.bp_start, &s.bp_end})
       FDK_HIP(hipEventCreate(e));
   }
@@ -164,9 +164,9 @@ int push(fdk_pipe* p, const void* host, int count, int first, int step, bool raw
   rc = collect(p, s);
   if (rc < 0) return rc;
   if (raw && !s.raw)
-    FDK_HIP(hipMalloc(&s.raw, FDK_BP_MAX_PROJ * p->view_elems * sizeof(float)));
+    FDK_HIP(fdk::dev_malloc((void**)&s.raw, FDK_BP_MAX_PROJ * p->view_elems * sizeof(float)));
   if (raw && p->store_dtype != FDK_F32 && !p->d_stage)
-    FDK_HIP(hipMalloc((void**)&p->d_stage, FDK_BP_MAX_PROJ * p->view_elems * sizeof(float)));
+    FDK_HIP(fdk::dev_malloc((void**)&p->d_stage, FDK_BP_MAX_PROJ * p->view_elems * sizeof(float)));
 
   const size_t bytes = count * p->view_elems * (raw ? sizeof(float) : esize(p->store_dtype));
   FDK_HIP(hipMemcpyAsync(raw ? s.raw : s.store, host, bytes, hipMemcpyHostToDevice, p->copy));

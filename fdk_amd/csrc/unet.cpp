@@ -191,7 +191,7 @@ void release(fdk_unet* u) {
 
 int upload_f32(const NpyArray& a, const std::vector<int64_t>& shape, const char* name, float** dev) {
   if (a.descr != "<f4" || a.shape != shape) return fdk::fail(FDK_ERR_INVALID, "%s: unexpected dtype or shape", name);
-  FDK_HIP(hipMalloc(dev, a.data.size()));
+  FDK_HIP(fdk::dev_malloc((void**)dev, a.data.size()));
   FDK_HIP(hipMemcpy(*dev, a.data.data(), a.data.size(), hipMemcpyHostToDevice));
   return FDK_OK;
 }
@@ -342,7 +342,7 @@ extern "C" int fdk_unet_load(const char* path, fdk_unet** out) {
     r = upload_f32(wi->second, ws, wn.c_str(), &tmp);
     if (r == FDK_OK) {
       const int64_t nw = wi->second.count();
-      hipError_t e = hipMalloc(&l.w, nw * 2);
+      hipError_t e = fdk::dev_malloc((void**)&l.w, nw * 2);
       if (e == hipSuccess) {
         r = fdk_nn_convert(tmp, l.w, nw, 1, nullptr);  // round to nearest even, as the trainer
         if (r == FDK_OK) e = hipDeviceSynchronize();

@@ -91,6 +91,11 @@ int fdk_last_error(char* buf, size_t len);
 int fdk_version(void);
 /* Number of HIP devices visible (0 when none); never fails. */
 int fdk_device_count(void);
+/* Frees the device memory the library keeps between calls for the scratch needs of its
+ * kernels, on the current device (at most 512 MiB; waits for the work that uses it).
+ * The library does so by itself before an allocation of its own fails; a program whose
+ * own allocator runs short calls it.  Safe at any time, from any thread. */
+int fdk_release_scratch(void);
 
 /* Device memory for the C++ layer's DevData / DevArray3D (cudaBP/cudaLib.cuh:298-420,
  * 552-640): linear allocations on the current device; copies use unified

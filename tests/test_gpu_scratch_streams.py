@@ -87,3 +87,24 @@ def test_results_are_those_of_calls_made_alone(torch_cuda, threads):
     assert not failed, failed
     for i, o in enumerate(out):
         assert torch.equal(o, ref[i // 2]), jobs[i // 2].kind
+
+
+def test_release_gives_the_memory_back(torch_cuda):
+    """A projection's copy stays with the library until it is released."""
+    torch = torch_cuda
+    n = 200
+    p = F.Parameter(nx=n, ny=n, nz=n, nu=n, nv=n, du=2.0, dv=2.0, nproj=24)
+    assert takes_the_copy(p, 0, 24, 0.5)
+    vol, out = torch.rand((n, n, n), device="cuda"), torch.empty((24, n, n), device="cuda")
+    F.release_scratch()
+    before = torch.cuda.mem_get_info()[0]
+    F.forward_project(p, vol, 0, 24, out, 0.5)
+    torch.cuda.synchronize()
+    kept = before - torch.cuda.mem_get_info()[0]
+    assert 8 * n ** 3 <= kept <= 1 << 29
+    F.release_scratch()
+    assert torch.cuda.mem_get_info()[0] >= before
+    again = torch.empty_like(out)
+    F.forward_project(p, vol, 0, 24, again, 0.5)
+    torch.cuda.synchronize()
+    assert torch.equal(out, again)

@@ -30,7 +30,8 @@ def program():
 
 
 @pytest.mark.parametrize("check", ["hand-over", "two streams past the limit", "larger while busy",
-                                   "larger beside a smaller", "other device", "threads"])
+                                   "larger beside a smaller", "other device", "out of memory",
+                                   "threads"])
 def test_scratch_list(check):
     r = subprocess.run([program()[0], check], capture_output=True, text=True, timeout=60)
     assert r.returncode == 0, r.stdout + r.stderr
