@@ -2043,30 +2043,33 @@ __global__ __launch_bounds__(256) void rtk_column_kernel(RtkArgs a, BpMats M,
   }
 }
 
-template <int K>
-void launch_rtk_column(const RtkArgs& a, const BpMats& M, const float2* pairs, hipStream_t st) {
-  const dim3 grid((a.nx + 63) / 64, (a.ny + 3) / 4, (a.nz + K - 1) / K);
-  if (pairs) hipLaunchKernelGGL((rtk_column_kernel<true, K>), grid, dim3(64, 4), 0, st, a, M, pairs);
-  else hipLaunchKernelGGL((rtk_column_kernel<false, K>), grid, dim3(64, 4), 0, st, a, M, pairs);
+// Detector samples a voxel step covers along u and v, at most, at the volume's centre.
+void rtk_steps(const RtkArgs& a, const BpMats& M, double* pu, double* pv) {
+  const double x = 0.5 * (a.nx - 1), y = 0.5 * (a.ny - 1);
+  *pu = *pv = 0.0;
+  for (int s = 0; s < a.nproj; ++s) {
+    const float* m = M.m[s];
+    const double Z = 1.0 / ((double)m[8] * x + (double)m[9] * y + m[11]);
+    const double U = ((double)m[0] * x + (double)m[1] * y + m[3]) * Z;
+    const double u = std::hypot((m[0] - U * m[8]) * Z, (m[1] - U * m[9]) * Z), v = std::fabs(m[6] * Z);
+    if (!(u <= *pu)) *pu = u;  // NaN stays, and selects rtk_kernel
+    if (!(v <= *pv)) *pv = v;
+    if (std::isnan(u) || std::isnan(v)) return;
+  }
 }
 
-// rtk_column_kernel where its matrices and sizes allow; false: rtk_kernel runs, also
-// for volumes of too few voxels to fill the chip with two or more a lane (64^3: 16.2
-// against 17.4 us; 96^3 46 against 43).
-constexpr double kRtkPairSave = 0.4e-12;  // seconds an update
-
+// rtk_column_kernel where its matrices and sizes allow; false: rtk_kernel runs.
 bool launch_rtk_columns(const RtkArgs& a, const BpMats& M, hipStream_t st) {
   for (int s = 0; s < a.nproj; ++s)
     if (M.m[s][2] != 0.0f || M.m[s][10] != 0.0f) return false;
   // 32-bit offsets in a view, 24-bit row counts and row bytes
   if ((long long)a.W * a.H * 8 >= (1LL << 31) || a.W >= (1 << 20) || a.H >= (1 << 23)) return false;
-  if ((long long)((a.nx + 63) / 64) * a.ny * a.nz < 8192) return false;
-  const double updates = (double)a.nx * a.ny * a.nz * a.nproj;
-  const double samples = (double)a.W * a.H * a.nproj;
+  double pu, pv;
+  rtk_steps(a, M, &pu, &pv);
+  fdk::rules::RtkForm f = fdk::rules::rtk_form(a.nx, a.ny, a.nz, a.nproj, a.W, a.H, pu, pv);
+  if (!f.per_lane) return false;
   fdk::Scratch ws;
-  // The pairs cost 12 us and 12 bytes a sample at 2.8 TB/s (128^3: 49 against 66 us
-  // without them, 96^3 42 against 43).
-  if (updates * kRtkPairSave > 12e-6 + samples * 12.0 / 2.8e12 && a.H <= 65536) {
+  if (f.pairs && a.H <= 65536) {
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(st, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone)
       (void)hipGetLastError();
@@ -2077,9 +2080,12 @@ bool launch_rtk_columns(const RtkArgs& a, const BpMats& M, hipStream_t st) {
   if (pairs)
     hipLaunchKernelGGL(rtk_pair_kernel, dim3((a.W + 255) / 256, a.H - 1, a.nproj), dim3(256), 0, st,
                        a.proj, pairs, a.W, a.H);
-  const long long waves = (long long)((a.nx + 63) / 64) * a.ny * ((a.nz + 7) / 8);
-  if (waves >= 4096) launch_rtk_column<8>(a, M, pairs, st);
-  else launch_rtk_column<2>(a, M, pairs, st);
+  else if (f.pairs)
+    f.per_lane = 2;  // no memory for them
+  const dim3 grid((a.nx + 63) / 64, (a.ny + 3) / 4, (a.nz + f.per_lane - 1) / f.per_lane);
+  const auto kernel = f.per_lane == 8 ? (pairs ? rtk_column_kernel<true, 8> : rtk_column_kernel<false, 8>)
+                                      : (pairs ? rtk_column_kernel<true, 2> : rtk_column_kernel<false, 2>);
+  hipLaunchKernelGGL(kernel, grid, dim3(64, 4), 0, st, a, M, pairs);
   fdk::scratch_put(&ws, st);
   return true;
 }

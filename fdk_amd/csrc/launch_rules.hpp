@@ -89,5 +89,35 @@ inline bool zfast_pays(const March& m, double copy_bytes, double kept_bytes) {
   return direct > 1.05 * zfast;
 }
 
+// How the RTK-form backprojector runs matrices without a z term: voxels of a column a lane
+// takes (0: rtk_kernel, a voxel a lane), and whether the views' rows are paired first.
+struct RtkForm {
+  int per_lane;
+  bool pairs;
+};
+
+// pu, pv: detector samples a voxel step covers along u and v, at most, at the volume's
+// centre.  Microseconds a voxel a lane / two / two or eight with pairs, 32 views unless said:
+//  * below 8192 waves of single voxels the chip is not filled: 64^3 16.4 / 17.3 / 27;
+//  * dense views leave neighbouring lanes nothing to share: 160^3, pu = pv 5.6, 254 / 292 /
+//    607, 320^3 with 3.7 1668 / 1738 / 2540, with 2.8 1346 / 1231 / 1520; with 8 views the
+//    line lies higher (3.7: 54 / 43 / 60, 5.6: 56.5 / 58.6 / 107);
+//  * pairs lose first, along u: 256^3 with pu 3.7, pv 0.9 606 / 491 / 510, the other way
+//    round 613 / 549 / 345.  They cost 9 us and 12 bytes a sample at 2.8 TB/s, and save 0.4
+//    ps an update: 96^3 45.1 / 47.4 / 43.9, 128^3 76 / 65 / 48, 512 x 512 x 2 24 / 18 / 29;
+//  * eight a lane where that leaves 4096 waves: 128^3 paired two 55, eight 48; 96^3 44, 40.
+//    Without pairs only for a view or two, where the volume's own traffic is all: 256^3
+//    from one view 42 / 32, eight 27; from 32 of 480^2 160^3 two 151, eight 165.
+inline RtkForm rtk_form(int nx, int ny, int nz, int nproj, int W, int H, double pu, double pv) {
+  const double rows = (double)((nx + 63) / 64) * ny;
+  const bool fill = rows * ((nz + 7) / 8) >= 4096;
+  if (rows * nz < 8192 || !(pu * pv >= 0)) return {0, false};
+  if (nproj <= 2 && fill && nz >= 8) return {8, false};
+  if (pu * pv >= (nproj >= 16 ? 12.0 : 20.0)) return {0, false};
+  const double updates = (double)nx * ny * nz * nproj, samples = (double)W * H * nproj;
+  if (pu >= 2.4 || updates * 0.4e-12 < 9e-6 + samples * 12.0 / 2.8e12) return {2, false};
+  return {fill ? 8 : 2, true};
+}
+
 }  // namespace rules
 }  // namespace fdk

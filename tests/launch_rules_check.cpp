@@ -18,3 +18,9 @@ extern "C" int check_zfast_pays(int nu, int nv, double cv, double dv, int nx, in
   const fdk::rules::March m{nu, nv, cv, dv, 1.5, nx, nx, nz, voxel, voxel, voxel, step, views, sum_sin, max_sin};
   return fdk::rules::zfast_pays(m, 8.0 * (nx + 4) * (nx + 4) * (nz + 4), 512.0 * 1024 * 1024);
 }
+
+// voxels a lane, negative with pairs
+extern "C" int check_rtk_form(int nx, int ny, int nz, int nproj, int W, int H, double pu, double pv) {
+  const fdk::rules::RtkForm f = fdk::rules::rtk_form(nx, ny, nz, nproj, W, H, pu, pv);
+  return f.pairs ? -f.per_lane : f.per_lane;
+}
