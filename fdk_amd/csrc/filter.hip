@@ -429,25 +429,28 @@ __global__ __launch_bounds__(256) void filter_rows_kernel(FilterArgs a) {
 // busy 90 % of the time: 60 strided twiddle loads, 64 row and cos loads of which half are
 // pads, 32 loads of edge samples and 8 scattered stores a thread.  Measured, 32 views of
 // 2048^2 transposed: 916 -> 598 us (row-major 765 -> 540); 32 of 1000^2 241 -> 90; 8 of
-// 4096^2 into FP16 1900 -> 1025; 4 of 300^2 11.0 -> 12.5 (the only loss seen:
-// too few rows to fill the chip at 16 points a thread); one of 9000^2 (was in place)
-// 2425 -> 782.
-typedef unsigned u32x2_t __attribute__((ext_vector_type(2)));
-typedef unsigned u32x4_t __attribute__((ext_vector_type(4)));
+// 4096^2 into FP16 1900 -> 1025; 32 of 500 x 300 row-major 26 -> 19; one of 9000^2 (was in
+// place) 2425 -> 782, although the 1024 threads of N = 16384 have 128 registers each and
+// spill 114 (460 bytes a thread).
+// Small calls: a launch costs 10.5 us whatever it does, and a wave's chain of loads and
+// passes has to fit in that.  So rows that lie side by side in a wave (N < 1024) are
+// loaded without branches, all 8 slices in flight (4 views of 500 x 300, N = 512, 14.3 us
+// with a branch a point, 10.9), and few pairs get blocks of one or two (one view of 2000
+// x 128 12.3 -> 10.5, two of 768^2 13.8 -> 12.1).
 typedef unsigned u32x2_t __attribute__((ext_vector_type(2)));
 typedef unsigned u32x4_t __attribute__((ext_vector_type(4)));
 
 template <int M>
 struct Wide {
   static constexpr int N = 1 << M, T = N / 16;
-  static constexpr int THREADS = T > 256 ? T : 256, PB = THREADS / T;  // row pairs per block
+  static constexpr int THREADS = T > 256 ? T : 256, SMALL = T > 64 ? T : 64;  // of a block
   static constexpr int R2 = M == 7 ? 8 : 16;
   static constexpr int R3 = M <= 8 ? 1 : M >= 12 ? 16 : N / 256;
   static constexpr int R4 = M >= 13 ? N / 4096 : 1;
   static constexpr int SLOTS = N + N / 16;  // LDS points of a pair, one spare per 16
   static constexpr int TW2 = (R2 - 1) * 16;
-  static constexpr size_t lds(bool quad) {
-    return sizeof(float2) * ((quad ? 2 : 1) * PB * SLOTS + TW2);
+  static constexpr size_t lds(bool quad, int pairs) {
+    return sizeof(float2) * ((quad ? 2 : 1) * pairs * SLOTS + TW2);
   }
 };
 
@@ -567,105 +570,85 @@ __device__ __forceinline__ float wide_lane(float v, int k) {
 // 0, so no address is clamped; slices that hold no sample are not loaded.
 template <int M>
 __device__ __forceinline__ void wide_load(const FilterArgs& a, const float* sa, const float* sb,
-                                          const float* ca, bool live, bool has_b, int t, int off,
-                                          float2 (&x)[16]) {
+                                          const float* ca, const float* cb, bool live, bool has_b,
+                                          int t, int off, float2 (&x)[16]) {
   constexpr int T = Wide<M>::T;
-  const int nu = a.nu, row_bytes = nu * 4;
-  float la = 0.f, lb = 0.f, ra = 0.f, rb = 0.f;
-  const int kpad = a.pad;
-  if constexpr (T >= 64) {
-    const int na = live ? row_bytes : 0, nb = has_b ? row_bytes : 0;
-    const __amdgpu_buffer_rsrc_t rxa = __builtin_amdgcn_make_buffer_rsrc((void*)sa, 0, na, fdk::kRawRsrcWord3);
-    const __amdgpu_buffer_rsrc_t rxb = __builtin_amdgcn_make_buffer_rsrc((void*)sb, 0, nb, fdk::kRawRsrcWord3);
-    const __amdgpu_buffer_rsrc_t rca = __builtin_amdgcn_make_buffer_rsrc((void*)ca, 0, ca ? na : 0, fdk::kRawRsrcWord3);
-    const __amdgpu_buffer_rsrc_t rcb =
-        __builtin_amdgcn_make_buffer_rsrc((void*)(ca + nu), 0, ca ? nb : 0, fdk::kRawRsrcWord3);
-    const auto ld = [](__amdgpu_buffer_rsrc_t r, int o) {
-      return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, o, 0, 0));
-    };
-    float ea = 0.f, eb = 0.f;  // lanes 0..3: samples 0..3, lanes 4..7: nu-1 .. nu-4
-    if (kpad) {
-      const int l = threadIdx.x & 7, e = (l < 4 ? l : nu + 3 - l) * 4;
-      ea = ld(rxa, e);
-      eb = ld(rxb, e);
-      if (ca) {
-        ea *= ld(rca, e);
-        eb *= ld(rcb, e);
-      }
+  const int nu = a.nu, row_bytes = nu * 4, kpad = a.pad;
+  // Row a and b and their cos rows: resources of the rows where a wave has one pair,
+  // clamped addresses where it has several (the rows differ between lanes; sa and sb are
+  // rows of the view also where there is no pair, and what is read there is not used).
+  const int na = live ? row_bytes : 0, nb = has_b ? row_bytes : 0;
+  const __amdgpu_buffer_rsrc_t rxa = __builtin_amdgcn_make_buffer_rsrc((void*)sa, 0, na, fdk::kRawRsrcWord3);
+  const __amdgpu_buffer_rsrc_t rxb = __builtin_amdgcn_make_buffer_rsrc((void*)sb, 0, nb, fdk::kRawRsrcWord3);
+  const __amdgpu_buffer_rsrc_t rca = __builtin_amdgcn_make_buffer_rsrc((void*)ca, 0, ca ? na : 0, fdk::kRawRsrcWord3);
+  const __amdgpu_buffer_rsrc_t rcb = __builtin_amdgcn_make_buffer_rsrc((void*)cb, 0, cb ? nb : 0, fdk::kRawRsrcWord3);
+  const auto ld = [&](__amdgpu_buffer_rsrc_t r, const float* row, int p) {
+    if constexpr (T >= 64) return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, p * 4, 0, 0));
+    else return row[p];
+  };
+  float ea = 0.f, eb = 0.f;  // lanes 0..3: samples 0..3, lanes 4..7: nu-1 .. nu-4
+  if (kpad) {
+    const int l = threadIdx.x & 7, e = l < 4 ? l : nu + 3 - l;
+    ea = ld(rxa, sa, e);
+    eb = ld(rxb, sb, e);
+    if (ca) {
+      ea *= ld(rca, ca, e);
+      eb *= ld(rcb, cb, e);
     }
+  }
 #pragma unroll
-    for (int c = 0; c < 16; c += 8) {  // 8 slices in flight
-      float xa[8], xb[8], wa[8], wb[8];
+  for (int c = 0; c < 16; c += 8) {  // 8 slices in flight
+    float xa[8], xb[8], wa[8], wb[8];
 #pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        const int lo = T * (c + i) - off;
-        xa[i] = xb[i] = 0.f;
-        wa[i] = wb[i] = 1.f;
-        if (lo + T > 0 && lo < nu) {
-          xa[i] = ld(rxa, (t + lo) * 4);
-          xb[i] = ld(rxb, (t + lo) * 4);
-          if (ca) {
-            wa[i] = ld(rca, (t + lo) * 4);
-            wb[i] = ld(rcb, (t + lo) * 4);
-          }
+    for (int i = 0; i < 8; ++i) {
+      const int lo = T * (c + i) - off;
+      xa[i] = xb[i] = 0.f;
+      wa[i] = wb[i] = 1.f;
+      if (lo + T > 0 && lo < nu) {
+        const int p = T >= 64 ? t + lo : min(max(t + lo, 0), nu - 1);
+        xa[i] = ld(rxa, sa, p);
+        xb[i] = ld(rxb, sb, p);
+        if (ca) {
+          wa[i] = ld(rca, ca, p);
+          wb[i] = ld(rcb, cb, p);
         }
       }
-#pragma unroll
-      for (int i = 0; i < 8; ++i) x[c + i] = make_float2(xa[i] * wa[i], xb[i] * wb[i]);
-    }
-    if (kpad == 0) return;
-    const auto la_of = [&](float v, int k) { return wide_lane<64>(v, k); };
-    if (kpad == 4) {
-      la = (la_of(ea, 0) + la_of(ea, 1) + la_of(ea, 2) + la_of(ea, 3)) / 4;
-      ra = (la_of(ea, 4) + la_of(ea, 5) + la_of(ea, 6) + la_of(ea, 7)) / 4;
-      lb = (la_of(eb, 0) + la_of(eb, 1) + la_of(eb, 2) + la_of(eb, 3)) / 4;
-      rb = (la_of(eb, 4) + la_of(eb, 5) + la_of(eb, 6) + la_of(eb, 7)) / 4;
-    } else {
-      la = (float)(((double)la_of(ea, 0) + la_of(ea, 1) + la_of(ea, 2)) / 3);
-      ra = (float)(((double)la_of(ea, 4) + la_of(ea, 5) + la_of(ea, 6)) / 3);
-      lb = (float)(((double)la_of(eb, 0) + la_of(eb, 1) + la_of(eb, 2)) / 3);
-      rb = (float)(((double)la_of(eb, 4) + la_of(eb, 5) + la_of(eb, 6)) / 3);
     }
 #pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      const int lo = T * i - off;
-      if (lo < 0 || lo + T > nu) {
-        if (t + lo < 0) x[i] = make_float2(la, lb);
-        else if (t + lo >= nu) x[i] = make_float2(ra, rb);
+    for (int i = 0; i < 8; ++i) {
+      x[c + i] = make_float2(xa[i] * wa[i], xb[i] * wb[i]);
+      if constexpr (T < 64) {  // nothing outside the row or in a row that does not exist
+        const int p = t + T * (c + i) - off;
+        const bool in = p >= 0 && p < nu;
+        x[c + i].x = live && in ? x[c + i].x : 0.f;
+        x[c + i].y = has_b && in ? x[c + i].y : 0.f;
       }
     }
+  }
+  if (kpad == 0) return;
+  if constexpr (T < 64) {
+    ea = live ? ea : 0.f;
+    eb = has_b ? eb : 0.f;
+  }
+  const auto at = [&](float v, int k) { return wide_lane<T>(v, k); };
+  float la, lb, ra, rb;
+  if (kpad == 4) {
+    la = (at(ea, 0) + at(ea, 1) + at(ea, 2) + at(ea, 3)) / 4;
+    ra = (at(ea, 4) + at(ea, 5) + at(ea, 6) + at(ea, 7)) / 4;
+    lb = (at(eb, 0) + at(eb, 1) + at(eb, 2) + at(eb, 3)) / 4;
+    rb = (at(eb, 4) + at(eb, 5) + at(eb, 6) + at(eb, 7)) / 4;
   } else {
-    // several pairs in a wave
-    const auto at = [&](const float* s, const float* c, bool ok, int p) {
-      return ok ? s[p] * (c ? c[p] : 1.f) : 0.f;
-    };
-    const float* cb = ca ? ca + nu : nullptr;
-    float ea[8], eb[8];
-    if (kpad) {
+    la = (float)(((double)at(ea, 0) + at(ea, 1) + at(ea, 2)) / 3);
+    ra = (float)(((double)at(ea, 4) + at(ea, 5) + at(ea, 6)) / 3);
+    lb = (float)(((double)at(eb, 0) + at(eb, 1) + at(eb, 2)) / 3);
+    rb = (float)(((double)at(eb, 4) + at(eb, 5) + at(eb, 6)) / 3);
+  }
 #pragma unroll
-      for (int l = 0; l < 8; ++l) {
-        const int e = l < 4 ? l : nu + 3 - l;
-        ea[l] = at(sa, ca, live, e);
-        eb[l] = at(sb, cb, has_b, e);
-      }
-      if (kpad == 4) {
-        la = (ea[0] + ea[1] + ea[2] + ea[3]) / 4;
-        ra = (ea[4] + ea[5] + ea[6] + ea[7]) / 4;
-        lb = (eb[0] + eb[1] + eb[2] + eb[3]) / 4;
-        rb = (eb[4] + eb[5] + eb[6] + eb[7]) / 4;
-      } else {
-        la = (float)(((double)ea[0] + ea[1] + ea[2]) / 3);
-        ra = (float)(((double)ea[4] + ea[5] + ea[6]) / 3);
-        lb = (float)(((double)eb[0] + eb[1] + eb[2]) / 3);
-        rb = (float)(((double)eb[4] + eb[5] + eb[6]) / 3);
-      }
-    }
-#pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      const int p = t + T * i - off;
-      x[i] = p < 0 ? make_float2(la, lb)
-             : p >= nu ? make_float2(ra, rb)
-                       : make_float2(at(sa, ca, live, p), at(sb, cb, has_b, p));
+  for (int i = 0; i < 16; ++i) {
+    const int lo = T * i - off;
+    if (lo < 0 || lo + T > nu) {
+      if (t + lo < 0) x[i] = make_float2(la, lb);
+      else if (t + lo >= nu) x[i] = make_float2(ra, rb);
     }
   }
 }
@@ -804,9 +787,10 @@ struct WideGrid {
   int nviews, group;
 };
 
-template <int M, bool QUAD>
-__global__ __launch_bounds__(Wide<M>::THREADS, (M == 14 ? 4 : 2)) void filter_wide_kernel(FilterArgs a, WideGrid g) {
+template <int M, bool QUAD, int THREADS>
+__global__ __launch_bounds__(THREADS, (M == 14 ? 4 : 2)) void filter_wide_kernel(FilterArgs a, WideGrid g) {
   using W = Wide<M>;
+  constexpr int PB = THREADS / W::T;  // row pairs (or quads) per block
   constexpr int N = W::N, T = W::T, R2 = W::R2, R3 = W::R3, R4 = W::R4;
   constexpr int P = QUAD ? 2 : 1, ROWS = 2 * P;  // row pairs and rows of an item
   extern __shared__ float2 wide_lds[];
@@ -816,7 +800,7 @@ __global__ __launch_bounds__(Wide<M>::THREADS, (M == 14 ? 4 : 2)) void filter_wi
   float2* buf[P];
 #pragma unroll
   for (int p = 0; p < P; ++p) buf[p] = wide_lds + W::TW2 + (sub * P + p) * W::SLOTS;
-  for (int k = threadIdx.x; k < W::TW2; k += W::THREADS)
+  for (int k = threadIdx.x; k < W::TW2; k += THREADS)
     tw2[k] = a.tw[(k & 15) * (k / 16 + 1) * (N / (16 * R2))];
   WideTw<M, R3, 256> tw3;
   tw3.load(a.tw, t);
@@ -830,9 +814,9 @@ __global__ __launch_bounds__(Wide<M>::THREADS, (M == 14 ? 4 : 2)) void filter_wi
   // (the first barrier below also covers tw2)
 
   // XCD x (block % 8) walks items [x chunk, (x + 1) chunk)
-  const int xcd = blockIdx.x % 8u, stride = (int)(gridDim.x / 8u) * W::PB;
+  const int xcd = blockIdx.x % 8u, stride = (int)(gridDim.x / 8u) * PB;
   const int end = min(g.items, (xcd + 1) * g.chunk);
-  for (int it0 = xcd * g.chunk + (int)(blockIdx.x / 8u) * W::PB; it0 < end; it0 += stride) {
+  for (int it0 = xcd * g.chunk + (int)(blockIdx.x / 8u) * PB; it0 < end; it0 += stride) {
     const int it = it0 + sub;
     const int grp = it / per_group, in = it - grp * per_group;
     const int set = grp * g.group + in % g.group;
@@ -843,9 +827,10 @@ __global__ __launch_bounds__(Wide<M>::THREADS, (M == 14 ? 4 : 2)) void filter_wi
     WIDE_EACH {
       const int r = ra + 2 * p;
       const bool has_a = live && r < a.nrows, has_b = live && r + 1 < a.nrows;
-      const float* sa = a.src + view * a.src_view + (long long)r * a.src_pitch;
-      wide_load<M>(a, sa, sa + a.src_pitch, a.cos_table ? a.cos_table + (long long)r * a.nu : nullptr,
-                   has_a, has_b, t, off, x[p]);
+      const float* sa = a.src + view * a.src_view + (long long)(has_a ? r : 0) * a.src_pitch;
+      const float* ca = a.cos_table ? a.cos_table + (long long)(has_a ? r : 0) * a.nu : nullptr;
+      wide_load<M>(a, sa, has_b ? sa + a.src_pitch : sa, ca, ca && has_b ? ca + a.nu : ca, has_a, has_b, t, off,
+                   x[p]);
     }
     WIDE_EACH {
       wide_dft<16, false>(x[p]);
@@ -1051,33 +1036,39 @@ int fft_choice() {
 
 // Blocks per CU that the LDS and the registers (2 waves per SIMD; 4 at M = 14, whose
 // block has 16 waves) allow.
-template <int M>
-constexpr int wide_resident() { return M <= 12 ? 2 : 1; }
+template <int M, int THREADS>
+constexpr int wide_resident() { return M <= 12 ? 512 / THREADS : 1; }
 
-template <int M, bool QUAD>
+template <int M, bool QUAD, int THREADS>
 int launch_wide_sets(const FilterArgs& a, int nviews, hipStream_t st) {
   using W = Wide<M>;
-  constexpr int ROWS = QUAD ? 4 : 2;
+  constexpr int ROWS = QUAD ? 4 : 2, PB = THREADS / W::T;
   const int nsets = (a.nrows + ROWS - 1) / ROWS;
   const int group = std::max(32 / ROWS, (nsets + 7) / 8);  // 32 rows fill a 128-byte line
   const long long items = (long long)((nsets + group - 1) / group) * group * nviews;
-  const long long chunk = ((items + 7) / 8 + W::PB - 1) / W::PB * W::PB;
-  const long long per_xcd = std::min<long long>(chunk / W::PB, 32 * wide_resident<M>());
+  const long long chunk = ((items + 7) / 8 + PB - 1) / PB * PB;
+  const long long per_xcd = std::min<long long>(chunk / PB, 32 * wide_resident<M, THREADS>());
   const WideGrid g{(int)items, (int)chunk, nviews, group};
-  const void* fn = reinterpret_cast<const void*>(&filter_wide_kernel<M, QUAD>);
-  const size_t lds = W::lds(QUAD);
+  const void* fn = reinterpret_cast<const void*>(&filter_wide_kernel<M, QUAD, THREADS>);
+  const size_t lds = W::lds(QUAD, PB);
   if (lds > 64 * 1024) FDK_HIP(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-  hipLaunchKernelGGL((filter_wide_kernel<M, QUAD>), dim3((unsigned)(8 * per_xcd)), dim3(W::THREADS), lds, st, a, g);
+  hipLaunchKernelGGL((filter_wide_kernel<M, QUAD, THREADS>), dim3((unsigned)(8 * per_xcd)), dim3(THREADS), lds, st, a, g);
   FDK_HIP(hipGetLastError());
   return FDK_OK;
 }
 
 template <int M>
 int launch_wide(const FilterArgs& a, int nviews, hipStream_t st) {
-  const long long waves = (long long)((a.nrows + 1) / 2) * nviews * Wide<M>::T / 64;
+  using W = Wide<M>;
+  const long long pairs = (long long)((a.nrows + 1) / 2) * nviews, waves = pairs * W::T / 64;
   if constexpr (M <= 13)
-    if (a.transpose && a.qmode == kStoreF32 && !a.far && waves >= 4096) return launch_wide_sets<M, true>(a, nviews, st);
-  return launch_wide_sets<M, false>(a, nviews, st);
+    if (a.transpose && a.qmode == kStoreF32 && !a.far && waves >= 4096)
+      return launch_wide_sets<M, true, W::THREADS>(a, nviews, st);
+  // Below two blocks a CU the pairs of a block of 256 threads would share a CU and leave
+  // others idle.
+  if constexpr (W::SMALL < W::THREADS)
+    if (pairs * W::T / W::THREADS < 512) return launch_wide_sets<M, false, W::SMALL>(a, nviews, st);
+  return launch_wide_sets<M, false, W::THREADS>(a, nviews, st);
 }
 
 int launch_filter(FilterArgs& a, int nviews, hipStream_t st) {
