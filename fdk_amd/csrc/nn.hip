@@ -2009,7 +2009,12 @@ static int launch_fwd5_pass(const Conv& a, int passes, hipStream_t st) {
   // 16 x 64 x 96 21.5 -> 12.1).  Two on the 4-plane tiles from 16 rounds on,
   // where the second tile's loads run under the first (96 -> 32 on 128 x 256 x
   // 256 1198 -> 1170 us; 3, 4 and 8 no faster).
-  const int tpb = TP == 4 && ntiles >= 8192 ? 2 : 1;
+  // With 32 input channels a tile's own loads have little to run under: two also where
+  // that leaves no round of the 512 blocks less than three quarters full (896 tiles
+  // 34.8 -> 31.2, 1024 36.8 -> 33.5, 2048 67.5 -> 64.2, but 1280 46 -> 48.5; 96 input
+  // channels 2048 169 -> 178).
+  const bool full = a.cin == 32 && (ntiles - 1) % 1024 >= 768;
+  const int tpb = TP == 4 && (ntiles >= 8192 || full) ? 2 : 1;
   hipLaunchKernelGGL((conv3d_fwd5_kernel<2, 4, TP>), dim3((ntiles + tpb - 1) / tpb, passes), dim3(256), lds,
                      st, a, tiles_x, tiles_y, ntiles, tpb);
   FDK_HIP(hipGetLastError());
