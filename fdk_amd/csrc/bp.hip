@@ -791,7 +791,7 @@ __global__ __launch_bounds__(256) void bp_lds_pf_kernel(BpArgs a, BpMats M, BpSc
 // 8 bytes off a 16-byte boundary); 101 x 92 x 83 volume,
 // detector 121 x 98, 2 x 40 views with the projector 632 -> 481 us (was the
 // direct-gather kernel: rows no multiple of 4).
-constexpr int kWsQuads = 3;  // strip quads per lane and run at ZPT 8
+constexpr int kWsQuads = 3;  // strip quads per lane and run at ZPT 8 (rules::wave_run checks strips against it)
 // Quad slots a lane stages: a 64 ZPT-voxel run's strip of the usual 1.3 columns
 // a voxel fits 64 slots of 4 columns each up to ZPT 2, 128 at ZPT 4 and 192 at 8;
 // a slot that is always empty would still issue its loads every view.
@@ -1516,49 +1516,35 @@ bool launch_wave_zpt(fdk_bp* h, const BpArgs& a, const BpMats& M, const BpScale&
   return true;
 }
 
-// Voxels per lane of bp_wave_kernel: of the values whose strips fit, the one with
-// the least vector instructions per view for a column of zext voxels.  A run of
-// 64 ZPT voxels costs about fixed + NQ staged quad slots + ZPT taps.  Forced values
-// (ZPT 1 / 2 / 4 / 8) agree: 512-deep slabs 34.5 / 19.7 / 15.1 / 14.4 ms, 256-deep
-// 8.1 / 4.5 / 3.2 / 4.1 ms, 128-deep 1.48 / 0.79 / 0.88 / 1.37 ms, a 256-deep single
-// slab 2.21 / 1.22 / 0.86 / 1.17 ms.
-template <bool SYM>
-int wave_zpt(double dvz, int zext, int* CT) {
-  constexpr int kZpt[4] = {8, 4, 2, 1}, kSlots[4] = {kWsQuads, 2, 1, 1};
-  constexpr int kFixed = 25, kSlot = SYM ? 20 : 10, kTap = SYM ? 9 : 7;
+// FDK_BP_ZPT: voxels per lane for bp_wave_kernel whatever its rule says (16 meaning 8).
+int wave_zpt_forced() {
   static const int forced = [] {
     const char* e = std::getenv("FDK_BP_ZPT");
     const int v = e ? std::atoi(e) : 0;
     return v >= 8 ? 8 : (v == 4 || v == 2 || v == 1) ? v : 0;
   }();
-  int best = 0;
-  long long cost = 0;
-  for (int k = 0; k < 4; ++k) {
-    const int z = kZpt[k], ct = fdk::rules::wave_strip_columns(dvz, z, SYM ? 2 : 1);
-    if (ct <= 0 || (ct - 2) / 4 > kWave * kSlots[k]) continue;
-    if ((size_t)4 * ct * (SYM ? 2 : 1) * sizeof(float) > 60 * 1024) continue;
-    const long long runs = (zext + kWave * z - 1) / (kWave * z);
-    const long long c = runs * (kFixed + kSlots[k] * kSlot + z * kTap);
-    if (forced ? z == forced : (!best || c < cost)) {
-      best = z;
-      cost = c;
-      *CT = ct;
-    }
-  }
-  return best;
+  return forced;
 }
 
 template <int DT, bool SYM>
 bool launch_wave_run(fdk_bp* h, const BpArgs& a, const BpMats& M, const BpScale& S,
                      double dvz) {
-  int CT = 0;
-  switch (wave_zpt<SYM>(dvz, a.zext, &CT)) {
-    case 8: return launch_wave_zpt<DT, SYM, 8>(h, a, M, S, CT);
-    case 4: return launch_wave_zpt<DT, SYM, 4>(h, a, M, S, CT);
-    case 2: return launch_wave_zpt<DT, SYM, 2>(h, a, M, S, CT);
-    case 1: return launch_wave_zpt<DT, SYM, 1>(h, a, M, S, CT);
+  const fdk::rules::WaveRun r = fdk::rules::wave_run(dvz, a.zext, SYM ? 2 : 1, a.nproj, wave_zpt_forced());
+  switch (r.zpt) {
+    case 8: return launch_wave_zpt<DT, SYM, 8>(h, a, M, S, r.columns);
+    case 4: return launch_wave_zpt<DT, SYM, 4>(h, a, M, S, r.columns);
+    case 2: return launch_wave_zpt<DT, SYM, 2>(h, a, M, S, r.columns);
+    case 1: return launch_wave_zpt<DT, SYM, 1>(h, a, M, S, r.columns);
   }
   return false;
+}
+
+// Whether single-slab runs are the faster (see rules::wave_run_pays); a forced value
+// always is.
+bool wave_single_pays(const BpArgs& a, double dvz, double least = 1.0) {
+  const int forced = wave_zpt_forced();
+  const fdk::rules::WaveRun r = fdk::rules::wave_run(dvz, a.zext, 1, a.nproj, forced);
+  return forced ? r.zpt != 0 : fdk::rules::wave_run_pays(r, a.zext, a.nproj, least);
 }
 
 // 16-bit views [u][v] with rows of `pitch` samples, pitch % 4 == 0, zeros past the row.
@@ -1589,7 +1575,9 @@ bool launch_wave_pitched(fdk_bp* h, const BpArgs& a, const BpMats& M, const BpSc
   const int pitch = (a.W + 4) & ~3;  // never W: tells a copy from the caller's own views
   const long long view = (long long)pitch * a.H;
   if (view * 2 >= (1LL << 31)) return false;
-  if (!fdk::rules::pitched_copy_pays((double)a.nxs * a.nys, a.zext, h->sym ? 2 : 1, a.nproj, (double)view))
+  const double dvz = max_dvz(a, M);
+  if (!(dvz > 0.0) || !wave_single_pays(a, dvz, 4.0 / 3) ||
+      !fdk::rules::pitched_copy_pays((double)a.nxs * a.nys, a.zext, h->sym ? 2 : 1, a.nproj, (double)view))
     return false;
   hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
   if (hipStreamIsCapturing(h->stream, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone) {
@@ -1627,10 +1615,9 @@ bool launch_wave(fdk_bp* h, const BpArgs& a, const BpMats& M, const BpScale& S) 
   const bool quads = a.W % 4 == 0 && a.pitch == a.W && (DT == FDK_F32 || (reinterpret_cast<uintptr_t>(a.proj) % 8 == 0 &&
                                                         a.view_stride % 4 == 0));
   if (h->sym && quads && mirror_symmetric(a, M)) return launch_wave_run<DT, true>(h, a, M, S, dvz);
-  // A strip staged for a single view is used once.  16-bit views: 512^3 from one of 512^2
-  // 266 us here, 215 by the block-strip kernel; FP32 rows off 4 samples: 256^3 pair 47.6,
-  // 41.8 by the gather kernel, but 512^3 pair 321 and 345, 300^3 54.5 and 64.5.
-  if (a.nproj == 1 && (DT != FDK_F32 || (a.W % 4 != 0 && (long long)a.nxs * a.nys < 80000))) return false;
+  // A strip staged for a single 16-bit view is used once: 512^3 from one of 512^2 266 us
+  // here, 215 by the block-strip kernel.
+  if ((DT != FDK_F32 && a.nproj == 1) || !wave_single_pays(a, dvz)) return false;
   return launch_wave_run<DT, false>(h, a, M, S, dvz);
 }
 

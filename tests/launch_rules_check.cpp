@@ -24,3 +24,9 @@ extern "C" int check_rtk_form(int nx, int ny, int nz, int nproj, int W, int H, d
   const fdk::rules::RtkForm f = fdk::rules::rtk_form(nx, ny, nz, nproj, W, H, pu, pv);
   return f.pairs ? -f.per_lane : f.per_lane;
 }
+
+extern "C" int check_wave_run(double dvz, int zext, int sides, int nproj, int* columns) {
+  const fdk::rules::WaveRun r = fdk::rules::wave_run(dvz, zext, sides, nproj, 0);
+  *columns = r.columns;
+  return fdk::rules::wave_run_pays(r, zext, nproj) ? r.zpt : -r.zpt;
+}
