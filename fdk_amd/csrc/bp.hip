@@ -784,12 +784,12 @@ __global__ __launch_bounds__(256) void bp_lds_pf_kernel(BpArgs a, BpMats M, BpSc
 // 16-byte loads) and the strip's round trip through LDS.  Measured against the form
 // that formed 64-bit addresses per slot, kept three tap forms in one loop (16 to 32
 // register moves a view where they joined) and ran single slabs on the block-strip
-// kernels: 1024^3 pair, 64 FP16 views of 1024^2, with read-out 27.8 -> 22.3 ms;
-// 768 x 512 x 2048 pair, 32 FP32 views 12.5 -> 10.6 ms; 256^3 pair, 96 FP32 views
-// 1458 -> 784 us (the 128-deep slabs at ZPT 2 instead of half-empty ZPT 4 runs);
-// 256^3 box of a 1024^3 scan, 128 FP32 views 2096 -> 834 us (878 with every second strip
+// kernels: 1024^3 pair, 64 FP16 views of 1024^2, with read-out 27.8 -> 20.9 ms;
+// 768 x 512 x 2048 pair, a pass of 32 FP32 views 10.1 -> 7.2 ms; 256^3 pair, 96 FP32 views
+// 1454 -> 777 us (the 128-deep slabs at ZPT 2 instead of half-empty ZPT 4 runs);
+// 256^3 box of a 1024^3 scan, 128 FP32 views 2100 -> 825 us (878 with every second strip
 // 8 bytes off a 16-byte boundary); 101 x 92 x 83 volume,
-// detector 121 x 98, 2 x 40 views with the projector 632 -> 481 us (was the
+// detector 121 x 98, 2 x 40 views with the projector 632 -> 343 us (was the
 // direct-gather kernel: rows no multiple of 4).
 constexpr int kWsQuads = 3;  // strip quads per lane and run at ZPT 8 (rules::wave_run checks strips against it)
 // Quad slots a lane stages: a 64 ZPT-voxel run's strip of the usual 1.3 columns

@@ -244,11 +244,12 @@ __global__ __launch_bounds__(256) void fp_kernel(RayGeom g, const float* __restr
 // voxel beside its y neighbour and one 16-byte gather brings four of the eight taps:
 // two gathers a sample.
 // Measured, 24 views of 256^2 through 256^3 at half-voxel steps: 5.10 ms (fp_kernel)
-// -> 1.38 (8-byte gathers) -> 0.79 ms, 820 Gsamples/s, copy included.  Splitting the rays over
+// -> 1.38 (8-byte gathers) -> 0.81 ms, 800 Gsamples/s, copy included (0.80 with a
+// blend one operation an axis shorter, which did not give fp_kernel's bits).  Splitting the rays over
 // 4 or 16 waves for launches with few of them gained nothing (8 views: 313 against
 // 230 us).
 constexpr int kFpPad = 2;
-constexpr int kFpTurn = 3;  // samples in flight a ray: 3 and 4 alike (783 us), 2 slower (807 us)
+constexpr int kFpTurn = 3;  // samples in flight a ray: 3 takes 812 us, 4 823, 2 830
 
 // dst[x][y][z] = {v(x, y, z), v(x, y + 1, z)} over the padded volume.
 template <int MODE>

@@ -46,9 +46,10 @@ struct WaveRun {
 
 // Voxels per lane: of the values whose strips fit, the one with the least vector
 // instructions per view for a column of zext voxels.  A run of 64 zpt voxels costs about
-// fixed + staged quad slots + taps, and 95 once a launch.  Forced values (1 / 2 / 4 / 8) agree: pairs of 512-deep
-// slabs 34.5 / 19.7 / 15.1 / 14.4 ms, 256-deep 8.1 / 4.5 / 3.2 / 4.1 ms, 128-deep 1.48 /
-// 0.79 / 0.88 / 1.37 ms, a 256-deep single slab 2.21 / 1.22 / 0.86 / 1.17 ms.
+// fixed + staged quad slots + taps, and 95 once a launch.  Forced values (1 / 2 / 4 / 8)
+// agree, a pass of 32 FP32 views of n^2 into n^3: 1024, pair 30.7 / 15.9 / 10.9 / 9.9 ms;
+// 512, pair 3.84 / 2.00 / 1.26 / 1.77 ms; 256, pair 470 / 243 / 268 / 431 us; 256, one slab
+// 536 / 286 / 181 / 281 us.
 inline WaveRun wave_run(double dvz, int zext, int sides, int nproj, int forced) {
   constexpr int kZpt[4] = {8, 4, 2, 1}, kSlots[4] = {3, 2, 1, 1};
   WaveRun best{0, 0, 0.0};
@@ -63,12 +64,13 @@ inline WaveRun wave_run(double dvz, int zext, int sides, int nproj, int forced) 
 }
 
 // Whether runs of single slabs beat the block-strip and gather kernels.  Those take
-// about 35 instructions a view and 64 voxels, in groups of 256.  Where a voxel step covers two samples and more, only strips of one voxel a lane
-// fit: 256^3 from 4 FP32 views of 513^2 67.5 us by the gather kernel, 126 by runs, from 32
-// 459 and 545, 512^3 from 32 of 1025^2 3.80 and 4.59 ms.  Single views: 256^3 pair from one
-// of 257^2 41.8 and 47.6 us, 512^3 pair 345 and 321, 300^3 64.5 and 54.5, 128^3 pair 11.1
-// and 13.1.  `least`: by how much, where the runs need their views copied first (160^3 pair
-// from 4 views of 321^2 48 us, 59 with a copy).
+// about 35 instructions a view and 64 voxels, in groups of 256.  Where a voxel step covers
+// two samples and more, only strips of one voxel a lane fit: 256^3 from 4 FP32 views of
+// 513^2 67.5 us by the gather kernel, 126 by runs, from 32 459 and 545, 512^3 from 32 of
+// 1025^2 3.80 and 4.59 ms.  Single views: 256^3 pair from one of 257^2 41.8 and 47.6 us,
+// 512^3 pair 345 and 321, 300^3 64.5 and 54.5, 128^3 pair 11.1 and 13.1.  `least`: by how
+// much, where the runs need their views copied first (160^3 pair from 4 views of 321^2
+// 48 us, 59 with a copy).
 inline bool wave_run_pays(const WaveRun& r, int zext, int nproj, double least = 1.0) {
   if (!r.zpt || (nproj == 1 && zext <= 64)) return false;
   return r.cost * least <= 35.0 * 4 * ((zext + 255) / 256);
